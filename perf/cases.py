@@ -49,11 +49,11 @@ def listed():
         # a half channel with a free-slip top, every length odd
         named("step_135x75x99_o4_open", "step", 135, 75, 99, order=4, wall="open"),
         # the production grid, triquintic interpolation
-        named("step_256x256x256_o6", "step", 256, 256, 256, cfl=1.6),
+        named("step_256x256x256_o6", "step", 256, 256, 256, cfl=1.0),
         # tricubic with the fields stored in single precision for the gathers
-        named("step_256x192x160_o4_fp32", "step", 256, 192, 160, order=4, storage=32),
-        # a large box at a high trajectory CFL
-        named("step_512x512x256_o6", "step", 512, 512, 256, cfl=4.0),
+        named("step_256x192x160_o4_fp32", "step", 256, 192, 160, order=4, storage=32, cfl=1.2),
+        # a large box
+        named("step_512x512x256_o6", "step", 512, 512, 256, cfl=1.5),
         # the Eulerian scheme on a production grid, at its own small CFL
         named("imex_256x192x192", "imex", 256, 192, 192, cfl=0.25),
         # the reference's advection benchmark grid, tricubic
@@ -79,15 +79,17 @@ def draw(rng):
 
     kind = rng.choice(("step", "step", "step", "imex", "advect", "plugin", "stats", "ensemble"))
     order = rng.choice((4, 6))
-    wall = rng.choice(("channel", "channel", "open"))
+    # the free-slip top is run with tricubic interpolation (triquintic is unstable there)
+    wall = rng.choice(("channel", "open")) if order == 4 else "channel"
     if kind == "ensemble":
         return _case(kind, size(24, 64), size(16, 48), size(24, 64), order=order, cfl=2.0,
                      members=rng.randint(4, 15), steps=rng.choice((4, 8)))
-    cfl = 0.25 if kind == "imex" else round(rng.uniform(1.0, 4.0), 2)
     storage = 32 if kind in ("step", "advect") and rng.random() < 0.25 else 64
     most = _cost(_case("step", 512, 512, 256))
     while True:
         nx = size(24, 768)
+        # a fine grid's time step is held by accuracy, not by the CFL number
+        cfl = 0.25 if kind == "imex" else round(rng.uniform(1.0, min(3.0, max(1.2, 600.0 / nx))), 2)
         # the box is twice as long as wide: cells at most a few times longer than wide
         c = _case(kind, nx, size(max(16, int(0.4 * nx)), int(1.1 * nx)), size(24, 256),
                   order=order, wall=wall, cfl=cfl, storage=storage)
