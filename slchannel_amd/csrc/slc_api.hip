@@ -97,6 +97,13 @@ std::vector<double> modified_k2(int n, double delta, bool half) {
     return out;
 }
 
+// 1/d as h + l: h the rounded reciprocal, l the exact residual of h times h
+// (the next 53 bits).
+void recip_pair(double d, double& h, double& l) {
+    h = 1.0 / d;
+    l = std::fma(-d, h, 1.0) * h;
+}
+
 int check_plan(slc_plan* p) {
     if (!p) return fail(SLC_EINVAL, "null plan");
     return SLC_OK;
@@ -197,6 +204,8 @@ int slc::plan_create(const slc_grid_desc* d, int device, bool spectral, slc_plan
     g.xy_lagged = 0;
     g.dx = dx;
     g.dy = dy;
+    recip_pair(dx, g.rdx_h, g.rdx_l);
+    recip_pair(dy, g.rdy_h, g.rdy_l);
     g.Lz = d->Lz;
     g.gamma = d->gamma;
     g.tanh_g = d->tanh_g;

@@ -32,6 +32,7 @@ struct Grid {
     int top_neumann;  // top wall: 0 no-slip (odd ghost), 1 free-slip (even ghost)
     int xy_lagged;    // BDF2 predictor xy RHS: 0 2R^n - R^{n-1} ('extrap'), 1 R^n ('lagged')
     double dx, dy, Lz, gamma, tanh_g, z_lo, z_hi, nu;
+    double rdx_h, rdx_l, rdy_h, rdy_l;  // 1/dx and 1/dy as pairs h + l (quotient)
     float rLz_f, rgamma_f, tanh_g_f;  // 1/Lz, 1/gamma, tanh(gamma) in float (z estimates)
     float split_f;  // slope of the centre-split estimate: -gamma/(2 nz) symmetric, gamma/(4 nz) bottom
     const double* z_c;      // nz+2 centres incl. ghost centres
@@ -110,6 +111,27 @@ __device__ inline int wrap_idx(int i, int n) {
     r = r >= n ? r - n : r;
     if (__builtin_expect((unsigned)r >= (unsigned)n, 0)) r = wrap_far(i, n);
     return r;
+}
+
+// x / d, correctly rounded, for a d whose reciprocal is held as a pair:
+// h = RN(1/d) and h + l = 1/d to twice the precision (recip_pair).  The first
+// two operations give x (h + l) to just over half an ulp; with its exact
+// residual the last fused operation rounds to RN(x / d) (the correction step
+// of a division whose reciprocal is correctly rounded).  Four FP64
+// instructions where the general division's scaling, quarter-rate
+// reciprocal, refinement and fix-up take eleven; a tile lane divides eight
+// times.
+__device__ inline double quotient(double x, double d, double h, double l) {
+    const double q = fma(x, h, x * l);
+    return fma(fma(-d, q, x), h, q);
+}
+
+__device__ inline double over_dx(const Grid& g, double x) {
+    return quotient(x, g.dx, g.rdx_h, g.rdx_l);
+}
+
+__device__ inline double over_dy(const Grid& g, double y) {
+    return quotient(y, g.dy, g.rdy_h, g.rdy_l);
 }
 
 // An integral-valued double (a floor) as an int.  The conversion instruction
@@ -530,8 +552,8 @@ __device__ inline void foot(const Grid& g, const TV& V, double xa, double ya, do
     double xm = xa, ym = ya, zm = za;
     for (int it = 0; it < g.n_iters; ++it) {
         double zc = clampd(zm, g.z_lo, g.z_hi);
-        double xdx = xm / g.dx;
-        double ydy = ym / g.dy;
+        double xdx = over_dx(g, xm);
+        double ydy = over_dy(g, ym);
         int cell = face_cell_fast(g, zc);
         double us, vs, ws;
         if constexpr (T == 4) {
@@ -564,10 +586,10 @@ template <int C, int P>
 __device__ inline void build_stencil(const Grid& g, double x, double y, double z,
                                      Stencil<C, P>& s) {
     constexpr int h = P / 2 - 1;
-    double sx = x / g.dx + Comp<C>::shift_x;
+    double sx = over_dx(g, x) + Comp<C>::shift_x;
     double ix0 = floor(sx);
     double tx = sx - ix0;
-    double sy = y / g.dy + Comp<C>::shift_y;
+    double sy = over_dy(g, y) + Comp<C>::shift_y;
     double iy0 = floor(sy);
     double ty = sy - iy0;
     int x0 = wrap_idx(floor_int(ix0) - h, g.nx), y0 = wrap_idx(floor_int(iy0) - h, g.ny);
@@ -619,10 +641,10 @@ template <int C, int P>
 __device__ inline void stencil_base(const Grid& g, double x, double y, double z, int& bx,
                                     int& by, int& k0, double& tx, double& ty) {
     constexpr int h = P / 2 - 1;
-    double sx = x / g.dx + Comp<C>::shift_x;
+    double sx = over_dx(g, x) + Comp<C>::shift_x;
     double ix0 = floor(sx);
     tx = sx - ix0;
-    double sy = y / g.dy + Comp<C>::shift_y;
+    double sy = over_dy(g, y) + Comp<C>::shift_y;
     double iy0 = floor(sy);
     ty = sy - iy0;
     bx = floor_int(ix0) - h;

@@ -105,6 +105,7 @@ struct EnsLaunch {
     int nmem;
     unsigned total;
     const int* umap;        // member of every unit (SL tile kinds only)
+    bool big;               // a member needs 64-bit addressing (big_index)
 };
 
 // SL tile shapes the ensemble kernels are compiled for (autotuned):

@@ -115,6 +115,7 @@ struct slc_ens {
     std::vector<unsigned> h_start;
     unsigned totals[EK_COUNT] = {};
     size_t zs_lds[3] = {0, 0, 0};
+    bool big = false;  // a member needs the tile kernels' 64-bit addressing (tile shape 0 only)
     bool zs_short[3] = {false, false, false};  // every member: <= 2 unknowns per lane
     // rocFFT
     rocfft_execution_info info = nullptr;
@@ -312,6 +313,8 @@ int rebuild(slc_ens* e) {
         e->zs_lds[k] = 0;
         e->zs_short[k] = true;
     }
+    e->big = false;
+    for (const Member* m : e->members) e->big = e->big || big_index(m->plan->g);
     for (int i = 0; i < n; ++i) {
         Member* m = e->members[i];
         slc_plan* pl = m->plan;
@@ -363,7 +366,7 @@ int rebuild(slc_ens* e) {
         for (int k = 0; k < 3; ++k) nmax = std::max(nmax, field_elems(k, m->nx, m->ny, m->nz));
         units[EK_ELEM] = ublocks(nmax);
         for (int k = 0; k < 3; ++k) {
-            units[EK_TILE0 + k] = tiles_of(m, k, e->tile_shape);
+            units[EK_TILE0 + k] = tiles_of(m, k, e->big ? 0 : e->tile_shape);
             const long ncols = (long)m->nx * m->ny;
             units[EK_ZS0 + k] = (unsigned)((ncols + M.zcols[k] - 1) / M.zcols[k]);
             if (M.zch[k] == 0)
@@ -431,6 +434,7 @@ EnsLaunch launch(const slc_ens* e, int kind, int comp = -1) {
     L.nmem = n;
     L.total = e->totals[kind];
     L.umap = comp >= 0 ? e->d_umap[comp] : nullptr;
+    L.big = e->big;
     return L;
 }
 

@@ -13,15 +13,18 @@ namespace slc {
 // One workgroup per tile: unit = xcd-ordered block index, its member from the
 // per-unit member map (the persistent chunk walk of the other batched kernels
 // keeps ~25 more registers live here and halves the occupancy).
-template <typename T, int C, int P, int PASS, int TI, int TJ, int TK, int kEnsLds, int WAVES>
+template <typename T, int C, int P, int PASS, int TI, int TJ, int TK, int kEnsLds, int WAVES,
+          bool BIG>
 __global__ __launch_bounds__(kSB) __attribute__((amdgpu_waves_per_eu(WAVES))) void
 ens_tile_kernel(const EnsMember* __restrict__ mem,
                                                        const unsigned* __restrict__ start,
                                                        const int* __restrict__ umap) {
-    __shared__ __align__(16) T lds[kEnsLds / sizeof(T)];  // 16-byte pairs land here (stage_box)
-    __shared__ int sh[PASS == 2 ? 12 : 6];
-    __shared__ int s_cnt;
-    __shared__ FootSt nst[PASS == 2 ? TI * TJ * TK : 1];
+    // one of the two tile bodies runs: the bootstrap's LDS is the fused pass's
+    constexpr int NPT = TI * TJ * TK;
+    constexpr int M0 = PASS == 0 ? MODE_FAR : PASS == 1 ? MODE_NEAR : MODE_BDF2;
+    __shared__ TileLds<T, M0, NPT, kEnsLds> L;
+    TileLds<T, MODE_BDF1, NPT, kEnsLds>& L1 =
+        reinterpret_cast<TileLds<T, MODE_BDF1, NPT, kEnsLds>&>(L);
     const unsigned uu = (unsigned)xcd_block(gridDim.x);
     // member and state are the same for the whole workgroup: broadcast them
     // so the member table is read with scalar loads and its pointers stay in
@@ -46,37 +49,40 @@ ens_tile_kernel(const EnsMember* __restrict__ mem,
     }
     if (ens_bdf2(st)) {
         const TrajVel V{{M.us[0], M.us[1], M.us[2]}, {nullptr, nullptr, nullptr}};
-        if (PASS == 0)
-            sl_tile_body<T, C, P, MODE_FAR, TI, TJ, TK, kEnsLds>(
-                M.g, M.at[C], V, Fa, Fb, Sa, Sb, M.dt, M.fld[c][C], ft, M.ncl, u, lds, sh, &s_cnt);
-        else if (PASS == 2)
-            sl_tile_body<T, C, P, MODE_BDF2, TI, TJ, TK, kEnsLds>(
-                M.g, M.at[C], V, Fa, Fb, Sa, Sb, M.dt, M.fld[c][C], ft, M.ncl, u, lds, sh, &s_cnt,
-                nst);
+        if constexpr (PASS == 0)
+            sl_tile_body<T, C, P, MODE_FAR, TI, TJ, TK, kEnsLds, BIG>(
+                M.g, M.at[C], V, Fa, Fb, Sa, Sb, M.dt, M.fld[c][C], ft, M.ncl, u, L);
+        else if constexpr (PASS == 2)
+            sl_tile_body<T, C, P, MODE_BDF2, TI, TJ, TK, kEnsLds, BIG>(
+                M.g, M.at[C], V, Fa, Fb, Sa, Sb, M.dt, M.fld[c][C], ft, M.ncl, u, L);
         else
-            sl_tile_body<T, C, P, MODE_NEAR, TI, TJ, TK, kEnsLds>(
-                M.g, M.at[C], V, Fa, Fb, Sa, Sb, M.dt, M.fld[c][C], ft, M.ncl, u, lds, sh, &s_cnt);
-    } else if (PASS >= 1) {
+            sl_tile_body<T, C, P, MODE_NEAR, TI, TJ, TK, kEnsLds, BIG>(
+                M.g, M.at[C], V, Fa, Fb, Sa, Sb, M.dt, M.fld[c][C], ft, M.ncl, u, L);
+    } else if constexpr (PASS >= 1) {
         const TrajVel V{{M.fld[a][0], M.fld[a][1], M.fld[a][2]}, {nullptr, nullptr, nullptr}};
-        sl_tile_body<T, C, P, MODE_BDF1, TI, TJ, TK, kEnsLds>(
-            M.g, M.at[C], V, Fa, nullptr, Sa, nullptr, M.dt, M.fld[c][C], ft, M.ncl, u, lds, sh,
-            &s_cnt);
+        sl_tile_body<T, C, P, MODE_BDF1, TI, TJ, TK, kEnsLds, BIG>(
+            M.g, M.at[C], V, Fa, nullptr, Sa, nullptr, M.dt, M.fld[c][C], ft, M.ncl, u, L1);
     }
 }
 
 template <typename T, int C, int P, int PASS>
 inline void launch_tile_shape(const EnsLaunch& L, int shape, unsigned grid, hipStream_t s) {
+    if (L.big) {  // a member past the 32-bit offsets: one shape
+        hipLaunchKernelGGL((ens_tile_kernel<T, C, P, PASS, 4, 4, 16, 31104, 4, true>), dim3(grid),
+                           dim3(kSB), 0, s, L.mem, L.start, L.umap);
+        return;
+    }
     switch (shape) {
         case 1:
-            hipLaunchKernelGGL((ens_tile_kernel<T, C, P, PASS, 4, 4, 32, 40960, 1>), dim3(grid),
+            hipLaunchKernelGGL((ens_tile_kernel<T, C, P, PASS, 4, 4, 32, 40960, 1, false>), dim3(grid),
                                dim3(kSB), 0, s, L.mem, L.start, L.umap);
             break;
         case 2:
-            hipLaunchKernelGGL((ens_tile_kernel<T, C, P, PASS, 2, 8, 16, 24576, 4>), dim3(grid),
+            hipLaunchKernelGGL((ens_tile_kernel<T, C, P, PASS, 2, 8, 16, 31104, 4, false>), dim3(grid),
                                dim3(kSB), 0, s, L.mem, L.start, L.umap);
             break;
         default:
-            hipLaunchKernelGGL((ens_tile_kernel<T, C, P, PASS, 4, 4, 16, 24576, 4>), dim3(grid),
+            hipLaunchKernelGGL((ens_tile_kernel<T, C, P, PASS, 4, 4, 16, 31104, 4, false>), dim3(grid),
                                dim3(kSB), 0, s, L.mem, L.start, L.umap);
     }
 }

@@ -50,6 +50,14 @@ struct ArrivalTabs {
     const int* csel;
 };
 
+// Whether the tile kernels address this grid's fields in 64 bits with 32-bit
+// index products (BIG): a field of 4 GiB or more, or a row, plane or index of
+// 2^24 or more.  All other grids take 32-bit byte offsets and 24-bit products.
+inline bool big_index(const Grid& g) {
+    const double pl = (double)(g.ny + 2) * (g.nz + 2);
+    return pl * (g.nx + 2) >= 536870912.0 || pl >= 16777216.0 || g.nx + 2 >= (1 << 24);
+}
+
 // LDS-tiled step kernels (slc_step.hip); mode: 0 advect, 1 bdf1, 2 far,
 // 3 near, 4 gather (feet given), 5 far + near in one pass (no feet arrays)
 // Fn32 / Fm32: float copies of F / Fm to gather from (FP32 storage), or null.

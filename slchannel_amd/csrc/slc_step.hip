@@ -6,61 +6,36 @@
 
 namespace slc {
 
-// tile shape of the step kernels: 4 x 4 x 16 arrival points (one per
-// thread), 24 KB of LDS, at least 4 waves per SIMD (measured at 256^3 order 6
-// against 4x4x32 / 2x8x16 / 8x4x8 / 4x8x8 tiles and 20-40 KB budgets).
-// Compile-time overridable with -DSLC_TILE_TI=... for tile-shape sweeps.
+// Tile of the step kernels: 4 x 4 x 16 arrival points, one per thread (measured
+// at 256^3 order 6 against 4x4x32, 2x8x16, 8x4x8 and 4x8x8 tiles).  Compile-time
+// overridable with -DSLC_TILE_TI=... for tile-shape sweeps.  The box budgets
+// fill a CU's 160 KB of LDS at the occupancy the registers allow: four
+// workgroups per CU (four waves per SIMD), less the workgroup's other LDS.
 #ifndef SLC_TILE_TI
 #define SLC_TILE_TI 4
 #define SLC_TILE_TJ 4
 #define SLC_TILE_TK 16
-#define SLC_TILE_LDS 24576
-#define SLC_TILE_WAVES 4
 #endif
+constexpr int kTI = SLC_TILE_TI, kTJ = SLC_TILE_TJ, kTK = SLC_TILE_TK;
+constexpr int kTileLds = 40576;
+constexpr int kTileLdsBdf2 = 31104;  // beside the near stencils' 9 KB
+constexpr int kTileWavesPerSimd = 4;
+// The gather at given feet and the near pass at order 4 fit seven waves per
+// SIMD (72 VGPRs) with a 21 KB budget (an order-4 box of a 4x4x16 tile at the
+// usual CFL takes 16-20 KB); at order 6 five or more spill.
+constexpr int kGatherWaves4 = 7;
+constexpr int kGatherLds4 = 21504;
 
-#ifndef SLC_TILE_WAVES
-#define SLC_TILE_WAVES 4
-#endif
-// waves per SIMD the near pass and the gather at given feet are built for
-// (order 6).  At order 4 they are built for seven, with a 21 KB box budget so
-// that seven workgroups fit a CU's 160 KB of LDS (72 VGPRs, 16 B spilled per
-// lane; measured at 256^3: six waves 0.446 ms, seven 0.415 ms, eight with a
-// 19 KB budget spill 40 B per lane and take 0.445 ms).  The order-4 box of a
-// 4x4x16 tile at the usual CFL is about 10 KB.
-#ifndef SLC_TILE_WAVES_GATHER
-#define SLC_TILE_WAVES_GATHER SLC_TILE_WAVES
-#endif
-#ifndef SLC_TILE_WAVES_GATHER4
-#define SLC_TILE_WAVES_GATHER4 7
-#endif
-#ifndef SLC_GTILE_LDS4
-#define SLC_GTILE_LDS4 21504
-#endif
-// waves per SIMD the fused far + near pass is built for
-#ifndef SLC_TILE_WAVES_BDF2
-#define SLC_TILE_WAVES_BDF2 SLC_TILE_WAVES
-#endif
-// tile of the near pass and the gather at given feet (default: the same)
-#ifndef SLC_GTILE_TI
-#define SLC_GTILE_TI SLC_TILE_TI
-#define SLC_GTILE_TJ SLC_TILE_TJ
-#define SLC_GTILE_TK SLC_TILE_TK
-#define SLC_GTILE_LDS SLC_TILE_LDS
-#endif
-
-template <typename T, int C, int P, int MODE, int TI, int TJ, int TK, int LDS_BYTES, int WAVES>
+template <typename T, int C, int P, int MODE, int TI, int TJ, int TK, int LDS_BYTES, int WAVES,
+          bool BIG>
 __global__ __launch_bounds__(kSB) __attribute__((amdgpu_waves_per_eu(WAVES))) void sl_tile_kernel(
     Grid g, ArrivalTabs A, TrajVel V, const double* __restrict__ F,
     const double* __restrict__ Fm, const T* __restrict__ Sn, const T* __restrict__ Sm,
     double dt, double* __restrict__ out, Feet ft, unsigned long long* nclamp,
     unsigned* defer) {
-    __shared__ __align__(16) T lds[LDS_BYTES / sizeof(T)];  // 16-byte pairs land here (stage_box)
-    __shared__ int sh[MODE == MODE_BDF2 ? 12 : 6];
-    __shared__ int s_cnt;
-    __shared__ FootSt nst[MODE == MODE_BDF2 ? TI * TJ * TK : 1];  // near stencils (MODE_BDF2)
-    sl_tile_body<T, C, P, MODE, TI, TJ, TK, LDS_BYTES>(g, A, V, F, Fm, Sn, Sm, dt, out, ft,
-                                                       nclamp, xcd_block(gridDim.x), lds, sh,
-                                                       &s_cnt, nst, defer);
+    __shared__ TileLds<T, MODE, TI * TJ * TK, LDS_BYTES> L;
+    sl_tile_body<T, C, P, MODE, TI, TJ, TK, LDS_BYTES, BIG>(
+        g, A, V, F, Fm, Sn, Sm, dt, out, ft, nclamp, (unsigned)xcd_block(gridDim.x), L, defer);
 }
 
 // The gather at given feet for the tiles a first pass deferred (their boxes
@@ -77,18 +52,15 @@ __global__ __launch_bounds__(kSB) __attribute__((amdgpu_waves_per_eu(WAVES))) vo
 // 11.7 ms with one workgroup per tile and 12.6 ms persistent (below); every
 // tile 8 x 8 x 4 in the first pass 10.3 ms, but the normal gather 16% slower.
 constexpr int kWideTI = 8, kWideTJ = 8, kWideTK = 4;
-constexpr int kWideLds = 40832;  // 160 KB / 4, less the block's other LDS
-#ifndef SLC_WIDE_WAVES
-#define SLC_WIDE_WAVES 4
-#endif
-constexpr int kWideBlocksPerCU = SLC_WIDE_WAVES;
+constexpr int kWideLds = 40576;  // 160 KB / 4, less the block's other LDS
+constexpr int kWideWaves = 4;
 
 // Whether wide tile wt overlaps a flagged first-pass tile (FI x FJ x FK
 // tiles, numbered like the wide ones, z fastest).  Independent loads; indices
 // past the domain's last tile repeat that tile.
 template <int C>
 __device__ inline bool wide_wanted(const Grid& g, const unsigned* __restrict__ flags, long wt) {
-    constexpr int FI = SLC_GTILE_TI, FJ = SLC_GTILE_TJ, FK = SLC_GTILE_TK;
+    constexpr int FI = kTI, FJ = kTJ, FK = kTK;
     static_assert(kWideTI % FI == 0 && kWideTJ % FJ == 0 && FK % kWideTK == 0,
                   "a wide tile covers whole first-pass tiles in x, y and lies in one in z");
     constexpr int NI = kWideTI / FI, NJ = kWideTJ / FJ;
@@ -121,20 +93,18 @@ __device__ inline bool wide_wanted(const Grid& g, const unsigned* __restrict__ f
 // order 6 the SGPRs overflow into VGPR lanes and 96 B per lane spill (+-5
 // cells at 512^3: 12.6 ms against 11.7 ms one workgroup per tile; three
 // workgroups per CU, without the spill, 14.2 ms).
-template <int C, int P>
-__global__ __launch_bounds__(kSB) __attribute__((amdgpu_waves_per_eu(SLC_WIDE_WAVES))) void gather_wide_kernel(
+template <int C, int P, bool BIG>
+__global__ __launch_bounds__(kSB) __attribute__((amdgpu_waves_per_eu(kWideWaves))) void gather_wide_kernel(
     Grid g, ArrivalTabs A, const double* __restrict__ F, Feet ft, double* __restrict__ out,
     unsigned long long* nclamp, const unsigned* __restrict__ flags, long wtiles) {
-    __shared__ __align__(16) double lds[kWideLds / sizeof(double)];
-    __shared__ int sh[6];
-    __shared__ int s_cnt;
+    __shared__ TileLds<double, MODE_GATHER, kWideTI * kWideTJ * kWideTK, kWideLds> L;
     __shared__ unsigned long long s_want[kSB / 64];
     const TrajVel V{{nullptr, nullptr, nullptr}, {nullptr, nullptr, nullptr}};
     Redo redo;
     redo.flags = flags;
-    redo.ti = SLC_GTILE_TI;
-    redo.tj = SLC_GTILE_TJ;
-    redo.tk = SLC_GTILE_TK;
+    redo.ti = kTI;
+    redo.tj = kTJ;
+    redo.tk = kTK;
     const long nchunks = (wtiles + kSB - 1) / kSB;
     for (long ch = xcd_block(gridDim.x); ch < nchunks; ch += gridDim.x) {
         const long wt = ch * kSB + threadIdx.x;
@@ -157,9 +127,10 @@ __global__ __launch_bounds__(kSB) __attribute__((amdgpu_waves_per_eu(SLC_WIDE_WA
                     bit = 32 + __builtin_ctz(hi);
                     hi &= hi - 1;
                 }
-                sl_tile_body<double, C, P, MODE_GATHER, kWideTI, kWideTJ, kWideTK, kWideLds>(
-                    g, A, V, F, F, F, F, 0.0, out, ft, nclamp, ch * kSB + w * 64 + bit, lds, sh,
-                    &s_cnt, nullptr, nullptr, redo);
+                sl_tile_body<double, C, P, MODE_GATHER, kWideTI, kWideTJ, kWideTK, kWideLds, BIG>(
+                    g, A, V, F, F, F, F, 0.0, out, ft, nclamp,
+                    (unsigned)(ch * kSB + w * 64 + bit), L, nullptr, redo);
+                __syncthreads();  // the next tile reuses L
             }
         }
         __syncthreads();  // s_want is rewritten by the next chunk
@@ -293,8 +264,6 @@ hipError_t run_to_f32(const Grid& g, float* const o[3], const double* const a[3]
     return hipGetLastError();
 }
 
-constexpr int kTI = SLC_TILE_TI, kTJ = SLC_TILE_TJ, kTK = SLC_TILE_TK, kLDS = SLC_TILE_LDS;
-
 struct StepArgs {
     const double* F;
     const double* Fm;
@@ -307,21 +276,19 @@ struct StepArgs {
     unsigned* defer;  // MODE_GATHER: per-tile flags of the wide second pass, or null
 };
 
-template <typename T, int C, int P, int MODE>
-static void launch_mode(const Grid& g, const ArrivalTabs& A, const TrajVel& V,
+template <typename T, int C, int P, int MODE, bool BIG>
+static void launch_mode_t(const Grid& g, const ArrivalTabs& A, const TrajVel& V,
                         const StepArgs& a, hipStream_t s) {
-    constexpr bool G = MODE == MODE_NEAR || MODE == MODE_GATHER;
-    constexpr int TI = G ? SLC_GTILE_TI : kTI, TJ = G ? SLC_GTILE_TJ : kTJ;
-    constexpr int TK = G ? SLC_GTILE_TK : kTK;
-    constexpr int LDS = G ? (P == 4 ? SLC_GTILE_LDS4 : SLC_GTILE_LDS) : kLDS;
-    constexpr int W = G ? (P == 4 ? SLC_TILE_WAVES_GATHER4 : SLC_TILE_WAVES_GATHER)
-                        : (MODE == MODE_BDF2 ? SLC_TILE_WAVES_BDF2 : SLC_TILE_WAVES);
+    constexpr bool G4 = (MODE == MODE_NEAR || MODE == MODE_GATHER) && P == 4;
+    constexpr int TI = kTI, TJ = kTJ, TK = kTK;
+    constexpr int LDS = G4 ? kGatherLds4 : MODE == MODE_BDF2 ? kTileLdsBdf2 : kTileLds;
+    constexpr int W = G4 ? kGatherWaves4 : kTileWavesPerSimd;
     const long nzi = (C == 2) ? g.nz - 1 : g.nz;
     const unsigned tiles = (unsigned)(((long)(g.nx + TI - 1) / TI) *
                                       ((g.ny + TJ - 1) / TJ) * ((nzi + TK - 1) / TK));
     if (tiles == 0) return;
     unsigned* defer = (MODE == MODE_GATHER) ? a.defer : nullptr;
-    hipLaunchKernelGGL((sl_tile_kernel<T, C, P, MODE, TI, TJ, TK, LDS, W>), dim3(tiles),
+    hipLaunchKernelGGL((sl_tile_kernel<T, C, P, MODE, TI, TJ, TK, LDS, W, BIG>), dim3(tiles),
                        dim3(kSB), 0, s, g, A, V, a.F, a.Fm, (const T*)a.Sn, (const T*)a.Sm, a.dt,
                        a.out, a.ft, a.ncl, defer);
     if constexpr (MODE == MODE_GATHER && sizeof(T) == 8) {
@@ -330,12 +297,19 @@ static void launch_mode(const Grid& g, const ArrivalTabs& A, const TrajVel& V,
                                 ((g.ny + kWideTJ - 1) / kWideTJ) *
                                 ((nzi + kWideTK - 1) / kWideTK);
             const long nchunks = (wtiles + kSB - 1) / kSB;
-            const long cap = (long)device_cus() * kWideBlocksPerCU;
-            hipLaunchKernelGGL((gather_wide_kernel<C, P>),
+            const long cap = (long)device_cus() * kWideWaves;
+            hipLaunchKernelGGL((gather_wide_kernel<C, P, BIG>),
                                dim3((unsigned)(nchunks < cap ? nchunks : cap)), dim3(kSB), 0, s,
                                g, A, (const double*)a.Sn, a.ft, a.out, a.ncl, defer, wtiles);
         }
     }
+}
+
+template <typename T, int C, int P, int MODE>
+static void launch_mode(const Grid& g, const ArrivalTabs& A, const TrajVel& V, const StepArgs& a,
+                        hipStream_t s) {
+    if (big_index(g)) launch_mode_t<T, C, P, MODE, true>(g, A, V, a, s);
+    else launch_mode_t<T, C, P, MODE, false>(g, A, V, a, s);
 }
 
 template <typename T, int C, int MODE>
@@ -385,8 +359,8 @@ hipError_t run_tile_step(const Grid& g, int comp, int mode, const ArrivalTabs& A
 
 long gather_tiles(const Grid& g, int comp) {
     const long nzi = (comp == 2) ? g.nz - 1 : g.nz;
-    return ((long)(g.nx + SLC_GTILE_TI - 1) / SLC_GTILE_TI) *
-           ((g.ny + SLC_GTILE_TJ - 1) / SLC_GTILE_TJ) * ((nzi + SLC_GTILE_TK - 1) / SLC_GTILE_TK);
+    return ((long)(g.nx + kTI - 1) / kTI) *
+           ((g.ny + kTJ - 1) / kTJ) * ((nzi + kTK - 1) / kTK);
 }
 
 }  // namespace slc

@@ -24,10 +24,20 @@
 // A workgroup owns a TI x TJ x TK tile of arrival points (z fastest).  Phase 1
 // traces the tile's feet and keeps each foot's stencil (base indices,
 // fractional offsets, clamped z) in registers; the tile's stencil bounding
-// box (its trajectory-CFL halo, measured) is reduced and staged in LDS with
-// coalesced z-contiguous loads; phase 2 contracts every P^3 stencil from LDS
-// (z, then y, then x, with FMAs -- the same order as the direct gather).  A
-// box larger than the LDS budget falls back to global loads for that tile.
+// box (its trajectory-CFL halo, measured) is reduced and staged in LDS; phase 2
+// contracts every P^3 stencil from LDS (z, then y, then x, with FMAs -- the
+// same order as the direct gather).
+//
+// What bounds it (fused BDF2 pass of u, 256^3, order 6; counters per
+// wavefront): 2200 VALU instructions (64% of the launch; half of them FP64),
+// 216 stencil values per foot from LDS (68%), the trajectory corners and z
+// tables through the vector cache (70%): no unit is full, four waves per SIMD
+// (128 VGPRs) do not hide the rest.  Measured with the index arithmetic in 32
+// bits and scalar registers, the row stride on the LDS banks and the boxes in
+// direct-to-LDS pieces: 1.61 -> 1.40 ms (w, whose odd rows went through
+// registers, 1.70 -> 1.48), order 4 with FP32 storage at 256x192x160
+// 0.63 -> 0.55 ms, advection of a component at 768x768x180, order 4,
+// 4.36 -> 3.74 ms.
 #pragma once
 
 #include <climits>
@@ -42,6 +52,14 @@ namespace slc {
 #define SLC_TILE_NT 256
 #endif
 constexpr int kSB = SLC_TILE_NT;
+
+// threadIdx.x, opaque to the optimiser: what a phase derives from it is
+// formed there, not formed once at entry and spilled in between.
+__device__ inline int phase_tid() {
+    int t = (int)threadIdx.x;
+    asm volatile("" : "+v"(t));
+    return t;
+}
 
 enum { MODE_ADVECT = 0, MODE_BDF1 = 1, MODE_FAR = 2, MODE_NEAR = 3, MODE_GATHER = 4,
        MODE_BDF2 = 5 };
@@ -81,107 +99,175 @@ __device__ inline int s_wave_min(int v) { return s_wave_reduce<true>(v); }
 
 __device__ inline int s_wave_max(int v) { return s_wave_reduce<false>(v); }
 
-// The workgroup unions of two boxes at once (one pair of barriers): b's left
-// in sh[0..5] and returned (wave-uniform), bn's left in sh[6..11].
-__device__ inline SBox s_block_box2(SBox l, SBox ln, int* sh) {
-    if (threadIdx.x == 0) {
-#pragma unroll
-        for (int q = 0; q < 12; q += 2) {
-            sh[q] = INT_MAX;
-            sh[q + 1] = INT_MIN;
-        }
-    }
-    __syncthreads();
-    int v[12] = {s_wave_min(l.xmin), s_wave_max(l.xmax), s_wave_min(l.ymin),
-                 s_wave_max(l.ymax), s_wave_min(l.kmin), s_wave_max(l.kmax),
-                 s_wave_min(ln.xmin), s_wave_max(ln.xmax), s_wave_min(ln.ymin),
-                 s_wave_max(ln.ymax), s_wave_min(ln.kmin), s_wave_max(ln.kmax)};
+constexpr int kTileWaves = kSB / 64;
+
+// The workgroup unions of the lanes' boxes, without atomics: every wavefront
+// reduces its lanes' boxes in registers and leaves them in red; after one
+// barrier (the caller's) box_union reads them back as wave-uniform values.
+struct BoxRed {
+    int v[2][kTileWaves][8];
+};
+
+__device__ inline void box_reduce(const SBox& l, int (&dst)[kTileWaves][8]) {
+    const int v0 = s_wave_min(l.xmin), v1 = s_wave_max(l.xmax), v2 = s_wave_min(l.ymin),
+              v3 = s_wave_max(l.ymax), v4 = s_wave_min(l.kmin), v5 = s_wave_max(l.kmax);
     if ((threadIdx.x & 63) == 0) {
+        int* d = dst[threadIdx.x >> 6];
+        *reinterpret_cast<int4*>(d) = make_int4(v0, v1, v2, v3);
+        *reinterpret_cast<int2*>(d + 4) = make_int2(v4, v5);
+    }
+}
+
+__device__ inline SBox box_union(const int (&src)[kTileWaves][8]) {
+    int r[6];
 #pragma unroll
-        for (int q = 0; q < 12; q += 2) {
-            atomicMin(&sh[q], v[q]);
-            atomicMax(&sh[q + 1], v[q + 1]);
-        }
+    for (int w = 0; w < kTileWaves; ++w) {
+        const int4 a = *reinterpret_cast<const int4*>(src[w]);
+        const int2 c = *reinterpret_cast<const int2*>(src[w] + 4);
+        r[0] = w ? min(r[0], a.x) : a.x;
+        r[1] = w ? max(r[1], a.y) : a.y;
+        r[2] = w ? min(r[2], a.z) : a.z;
+        r[3] = w ? max(r[3], a.w) : a.w;
+        r[4] = w ? min(r[4], c.x) : c.x;
+        r[5] = w ? max(r[5], c.y) : c.y;
     }
-    __syncthreads();
-    return SBox{sh[0], sh[1], sh[2], sh[3], sh[4], sh[5]};
+#pragma unroll
+    for (int q = 0; q < 6; ++q) r[q] = __builtin_amdgcn_readfirstlane(r[q]);
+    return SBox{r[0], r[1], r[2], r[3], r[4], r[5]};
 }
 
-__device__ inline SBox s_block_box(SBox l, int* sh) {
-    if (threadIdx.x == 0) {
-        sh[0] = INT_MAX; sh[1] = INT_MIN;
-        sh[2] = INT_MAX; sh[3] = INT_MIN;
-        sh[4] = INT_MAX; sh[5] = INT_MIN;
-    }
-    __syncthreads();
-    int a = s_wave_min(l.xmin), b = s_wave_max(l.xmax);
-    int c = s_wave_min(l.ymin), d = s_wave_max(l.ymax);
-    int e = s_wave_min(l.kmin), f = s_wave_max(l.kmax);
-    if ((threadIdx.x & 63) == 0) {
-        atomicMin(&sh[0], a); atomicMax(&sh[1], b);
-        atomicMin(&sh[2], c); atomicMax(&sh[3], d);
-        atomicMin(&sh[4], e); atomicMax(&sh[5], f);
-    }
-    __syncthreads();
-    SBox r{sh[0], sh[1], sh[2], sh[3], sh[4], sh[5]};
-    __syncthreads();
-    return r;
+// Element i of p, addressed by a byte offset in 32 bits (one scalar base and
+// one lane offset per load, no 64-bit lane arithmetic) when every field of the
+// grid is below 4 GiB; BIG: in 64 bits.
+template <bool BIG, typename T>
+__device__ inline T* elem(T* p, unsigned i) {
+    if (BIG) return p + (size_t)i;
+    return reinterpret_cast<T*>(
+        const_cast<char*>(reinterpret_cast<const char*>(p)) + (size_t)(i * (unsigned)sizeof(T)));
 }
 
-// Trajectory samples of the three U* components at one point (they share
-// x/dx, y/dy and the face cell of z; semilag.py:512-528 recomputes them with
-// identical results).  Two rounds of loads: the faces of the estimated
-// interval, then the corners.
-// xdx = x/dx, ydy = y/dy and zc the clamped z.
-__device__ inline void sample3_exact(const Grid& g, const TrajA& V, double xdx, double ydy,
-                                     double zc, double& us, double& vs, double& ws) {
-    double split;
-    const int c = face_cell_fast(g, zc, split);
-    const int mc = locate_split<0>(c, split, zc);
-    us = trilinear_m<0>(g, V, xdx, ydy, zc, mc);
-    vs = trilinear_m<1>(g, V, xdx, ydy, zc, mc);
-    ws = trilinear_m<2>(g, V, xdx, ydy, zc, c);
+// Two consecutive doubles as one 16-byte load (8-byte aligned).
+struct __attribute__((packed, aligned(8))) Pair {
+    double a, b;
+};
+
+template <bool BIG>
+__device__ inline Pair pair_at(const double* p, unsigned i) {
+    return *reinterpret_cast<const Pair*>(elem<BIG>(p, i));
 }
 
-// Column values of component C at levels k0, k0+1 of its four trilinear
-// columns, with the x/y weights of trilinear_m.
-template <int C>
-__device__ inline void trilinear_cols(const Grid& g, const TrajA& V, double xdx, double ydy,
-                                      int k0, double* wx, double* wy, double (&v)[2][2][2]) {
-    int ix[2], iy[2];
-    trilinear_xy<C>(g, xdx, ydy, wx, wy, ix, iy);
+// The two trilinear columns of one axis: wrapped node indices i0, i1 of the
+// cell and the fraction t in it.
+struct Cell {
+    int i0, i1;
+    double t;
+};
+
+// Wrap by unsigned minima: for f in [-n, 2n) the first one adds a period to
+// a negative f, the second takes one from an f >= n (the other candidate is
+// then beyond 2^31).  *far collects lanes where f lies farther out.
+__device__ inline Cell cell_of(double s, int n) {
+    const double fl = floor(s);
+    const unsigned un = (unsigned)n, f = (unsigned)floor_int(fl);
+    unsigned r = min(f, f + un);
+    r = min(r, r - un);
+    const unsigned r1 = min(r + 1u, r + 1u - un);
+    return Cell{(int)r, (int)r1, s - fl};
+}
+
+__device__ inline void cell_far(double s, int n, Cell& c) {
+    const int f = floor_int(floor(s));
+    c.i0 = wrap_far(f, n);
+    c.i1 = c.i0 + 1 == n ? 0 : c.i0 + 1;
+}
+
+// x and y cells of a point for nodes on faces (shift 0) and centres (shift
+// -1/2): u sits at (x face, y centre), v at (x centre, y face), w at (x
+// centre, y centre), so four cells serve the three components.
+struct XYCells {
+    Cell xf, xc, yf, yc;
+};
+
+__device__ inline XYCells xy_cells(const Grid& g, double xdx, double ydy) {
+    XYCells q;
+    const double xh = xdx + -0.5, yh = ydy + -0.5;
+    q.xf = cell_of(xdx, g.nx);
+    q.xc = cell_of(xh, g.nx);
+    q.yf = cell_of(ydy, g.ny);
+    q.yc = cell_of(yh, g.ny);
+    const bool far = max((unsigned)q.xf.i0, (unsigned)q.xc.i0) >= (unsigned)g.nx ||
+                     max((unsigned)q.yf.i0, (unsigned)q.yc.i0) >= (unsigned)g.ny;
+    if (__builtin_expect(far, 0)) {
+        // a point more than one period outside the domain, or not finite
+        cell_far(xdx, g.nx, q.xf);
+        cell_far(xh, g.nx, q.xc);
+        cell_far(ydy, g.ny, q.yf);
+        cell_far(yh, g.ny, q.yc);
+    }
+    return q;
+}
+
+// The eight corner values of component C's trilinear cell: (i, j) columns,
+// levels k0, k0 + 1.  Without BIG the indices and strides are below 2^24
+// (big_index), so the products are full-rate 24-bit ones (a 32-bit product
+// takes four times as long).
+template <int C, bool BIG>
+__device__ inline void cell_cols(const Grid& g, const double* F, const Cell& x, const Cell& y,
+                                 int k0, Pair (&v)[2][2]) {
+    const unsigned SZ = (unsigned)Comp<C>::SZ(g), PS = (unsigned)Comp<C>::SY(g) * SZ;
+    const double* base = F + ((size_t)Comp<C>::ox * PS + (size_t)Comp<C>::oy * SZ);
+    auto mul = [](int a, unsigned b) { return BIG ? (unsigned)a * b : __umul24((unsigned)a, b); };
+    const unsigned x0 = mul(x.i0, PS), x1 = mul(x.i1, PS);
+    const unsigned y0 = mul(y.i0, SZ) + (unsigned)k0, y1 = mul(y.i1, SZ) + (unsigned)k0;
+    v[0][0] = pair_at<BIG>(base, x0 + y0);
+    v[0][1] = pair_at<BIG>(base, x0 + y1);
+    v[1][0] = pair_at<BIG>(base, x1 + y0);
+    v[1][1] = pair_at<BIG>(base, x1 + y1);
+}
+
+// The sequential (i, j, k) sum of the trilinear sample (semilag.py:44-59) with
+// the order-2 weights (1 - t, t) of the cells: the terms and the order of
+// trilinear<C> (slc_device.h), so the same doubles.
+__device__ inline double cell_sum(const Cell& x, const Cell& y, const double (&wz)[2],
+                                  const Pair (&v)[2][2]) {
+    const double wx[2] = {1.0 - x.t, x.t}, wy[2] = {1.0 - y.t, y.t};
+    double out = 0.0;
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-            const int base = node_addr<C, false>(g, ix[i], iy[j], k0);
-            v[i][j][0] = V.a[C][base];
-            v[i][j][1] = V.a[C][base + 1];
+            const double wij = wx[i] * wy[j];
+            const double t0 = (wij * wz[0]) * v[i][j].a, t1 = (wij * wz[1]) * v[i][j].b;
+            out = (i == 0 && j == 0) ? t0 : out + t0;
+            out = out + t1;
         }
-}
-
-// trilinear_m's sum, over column values read by trilinear_cols.
-__device__ inline double trilinear_sum(const double* wx, const double* wy, const double* wz,
-                                       const double (&v)[2][2][2]) {
-    double out = 0.0;
-    bool first = true;
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            double wij = wx[i] * wy[j];
-#pragma unroll
-            for (int k = 0; k < 2; ++k) {
-                double term = (wij * wz[k]) * v[i][j][k];
-                out = first ? term : out + term;
-                first = false;
-            }
-        }
-    }
     return out;
 }
 
-// sample3_exact in one round of loads, for a point traced from the arrival
+// Trajectory samples of the three U* components at (xdx, ydy) = (x/dx, y/dy)
+// and the clamped z, whose face interval c and centre node interval m are
+// known (semilag.py:512-528 recomputes them per component with identical
+// results).
+template <bool BIG>
+__device__ inline void sample3_at(const Grid& g, const TrajA& V, double xdx, double ydy,
+                                  double zc, int c, int m, double& us, double& vs, double& ws) {
+    const XYCells q = xy_cells(g, xdx, ydy);
+    const Pair nf = pair_at<false>(g.z_f, (unsigned)c), nc = pair_at<false>(g.z_c, (unsigned)m);
+    const Pair pc = pair_at<false>(g.dinv_c2, 2u * (unsigned)m);
+    const Pair pf = pair_at<false>(g.dinv_f2, 2u * (unsigned)c);
+    Pair uv[2][2], vv[2][2], wv[2][2];
+    cell_cols<0, BIG>(g, V.a[0], q.xf, q.yc, m, uv);
+    cell_cols<1, BIG>(g, V.a[1], q.xc, q.yf, m, vv);
+    cell_cols<2, BIG>(g, V.a[2], q.xc, q.yc, c, wv);
+    const double wzc[2] = {(zc - nc.b) * pc.a, (zc - nc.a) * pc.b};
+    const double wzf[2] = {(zc - nf.b) * pf.a, (zc - nf.a) * pf.b};
+    us = cell_sum(q.xf, q.yc, wzc, uv);
+    vs = cell_sum(q.xc, q.yf, wzc, vv);
+    ws = cell_sum(q.xc, q.yc, wzf, wv);
+}
+
+// sample3_at for a point whose z interval is not known, in one round of
+// loads, for a point traced from the arrival
 // (za, K) of component C.  The face interval c and the centred components'
 // node interval m = c + s (s: z >= z_c[c+1]) are predicted without loads, and
 // the faces, centre nodes, inverse denominators and the three components'
@@ -194,14 +280,14 @@ __device__ inline double trilinear_sum(const double* wx, const double* wy, const
 // the prediction and z is outside the faces' 1e-10 band, c is the interval
 // face_cell_fast returns (the one interval bracketing z) and m the node
 // interval of locate_split.  Otherwise (a few lanes in 1e5 on stretched
-// production grids) c and m are located as sample3_exact does and the values
-// read again.  Either way the sums are trilinear_m's operations on the same
-// values, so the result is sample3_exact's.
-template <int C>
+// production grids) c and m are located as face_cell_fast does and the values
+// read again.  Either way the sums are the same operations on the same
+// values as with a located interval.
+template <int C, bool BIG>
 __device__ inline void sample3(const Grid& g, const TrajA& V, double x, double y, double z,
                                double za, int K, double& us, double& vs, double& ws) {
     const double zc = clampd(z, g.z_lo, g.z_hi);
-    const double xdx = x / g.dx, ydy = y / g.dy;
+    const XYCells q = xy_cells(g, over_dx(g, x), over_dy(g, y));
     float kfe, a;
     int c = face_estimate(g, zc, kfe, a);
     if (!Comp<C>::centers && (c == K - 1 || c == K)) c = zc >= za ? K : K - 1;
@@ -209,40 +295,27 @@ __device__ inline void sample3(const Grid& g, const TrajA& V, double x, double y
     if (Comp<C>::centers && c == K - 1) s = zc >= za;
     int m = c + (s ? 1 : 0);
     for (bool located = false;; located = true) {
-        const double lo = g.z_f[c], hi = g.z_f[c + 1];
-        const double n0 = g.z_c[m], n1 = g.z_c[m + 1];
-        const double p0 = g.dinv_c2[2 * m], p1 = g.dinv_c2[2 * m + 1];
-        const double f0 = g.dinv_f2[2 * c], f1 = g.dinv_f2[2 * c + 1];
-        double uwx[2], uwy[2], vwx[2], vwy[2], wwx[2], wwy[2];
-        double uv[2][2][2], vv[2][2][2], wv[2][2][2];
-        trilinear_cols<0>(g, V, xdx, ydy, m, uwx, uwy, uv);
-        trilinear_cols<1>(g, V, xdx, ydy, m, vwx, vwy, vv);
-        trilinear_cols<2>(g, V, xdx, ydy, c, wwx, wwy, wv);
-        const double split = m > c ? n0 : n1;  // z_c[c + 1]
-        if (located || (face_estimate_holds(g, c, zc, lo, hi) && (zc >= split) == (m > c))) {
-            const double wzc[2] = {(zc - n1) * p0, (zc - n0) * p1};
-            const double wzf[2] = {(zc - hi) * f0, (zc - lo) * f1};
-            us = trilinear_sum(uwx, uwy, wzc, uv);
-            vs = trilinear_sum(vwx, vwy, wzc, vv);
-            ws = trilinear_sum(wwx, wwy, wzf, wv);
+        const Pair nf = pair_at<false>(g.z_f, (unsigned)c);
+        const Pair nc = pair_at<false>(g.z_c, (unsigned)m);
+        const Pair pc = pair_at<false>(g.dinv_c2, 2u * (unsigned)m);
+        const Pair pf = pair_at<false>(g.dinv_f2, 2u * (unsigned)c);
+        Pair uv[2][2], vv[2][2], wv[2][2];
+        cell_cols<0, BIG>(g, V.a[0], q.xf, q.yc, m, uv);
+        cell_cols<1, BIG>(g, V.a[1], q.xc, q.yf, m, vv);
+        cell_cols<2, BIG>(g, V.a[2], q.xc, q.yc, c, wv);
+        const double split = m > c ? nc.a : nc.b;  // z_c[c + 1]
+        if (located || (face_estimate_holds(g, c, zc, nf.a, nf.b) && (zc >= split) == (m > c))) {
+            const double wzc[2] = {(zc - nc.b) * pc.a, (zc - nc.a) * pc.b};
+            const double wzf[2] = {(zc - nf.b) * pf.a, (zc - nf.a) * pf.b};
+            us = cell_sum(q.xf, q.yc, wzc, uv);
+            vs = cell_sum(q.xc, q.yf, wzc, vv);
+            ws = cell_sum(q.xc, q.yc, wzf, wv);
             return;
         }
         double sp;
         c = face_cell_fast(g, zc, sp);
         m = locate_split<0>(c, sp, zc);
     }
-}
-
-// Arrival-point trajectory sample with precomputed x/dx, y/dy and z location
-// (csel = 2 * face cell + centre split: the values sample3_exact computes; see
-// ArrivalTabs).
-__device__ inline void sample3_at(const Grid& g, const TrajA& V, double xdx, double ydy,
-                                  double z, int csel, double& us, double& vs, double& ws) {
-    const double zc = clampd(z, g.z_lo, g.z_hi);
-    const int c = csel >> 1, mc = c + (csel & 1);
-    us = trilinear_m<0>(g, V, xdx, ydy, zc, mc);
-    vs = trilinear_m<1>(g, V, xdx, ydy, zc, mc);
-    ws = trilinear_m<2>(g, V, xdx, ydy, zc, c);
 }
 
 // Per-foot stencil data kept between the phases.
@@ -259,186 +332,399 @@ __device__ inline void make_st(const Grid& g, double x, double y, double z, Foot
     stencil_base<C, P>(g, x, y, f.z, f.bx, f.by, f.bk, f.tx, f.ty);
 }
 
-// Stages the stencil bounding box `b` of a tile's feet (field S) into `lds`,
-// using at most cap_bytes: the box (z fastest), then one int per (x, y) row,
-// its global base.  Returns false (nothing staged) when the box does not fit.
-// b.kmin becomes the z index of the box's first level.  Ends with a barrier.
+// How a tile's stencil box reaches the contraction (uniform over the block):
+//   whole   the box in LDS with row stride kLZ: the usual case (the stencils of
+//           a 16-level tile span 20-23 levels at the usual CFL)
+//   slabs   the box goes through LDS in runs of x planes, each staged with
+//           the box's own z extent; a lane adds its stencil planes as they
+//           come by.  Boxes over the LDS budget (high CFL, rough fields)
+//   direct  loads from memory, when not even one plane fits (feet far apart
+//           or not finite)
+// Every way adds the same products in the same order, so the doubles agree.
 //
-// Double fields whose z rows have an even length and whose base is 16-byte
-// aligned are staged with gfx950's direct global-to-LDS loads of 16-byte
-// pairs (global_load_lds_dwordx4: no register round trip, no LDS write
-// instruction): the box then starts at an even level and has an even
-// z extent, so every pair lies inside one row (the rounded-up end is at most
-// the row length, which is even) and is aligned.  The barrier's release
-// fence waits for the loads.  Other fields (the w component at even nz, FP32
-// storage) are staged through registers.
-#ifndef SLC_STAGE_DMA
-#define SLC_STAGE_DMA 1
-#endif
+// kLZ = 32 doubles: a multiple of the 64 LDS banks, so the bank of a value
+// depends on its level alone and the 16 consecutive levels that 16 lanes read
+// do not collide when some of their columns lie in another row (a stride of
+// 24 took 1.57 ms per fused pass of u at 256^3, order 6, this one 1.45 ms; the
+// unpadded box extent 1.54 ms).
+constexpr int kLZ = 32;
+
+enum { BOX_NONE = 0, BOX_WHOLE, BOX_SLABS, BOX_DIRECT };
+
+constexpr int kFar = 1 << 30;  // bases beyond: x0 + x could leave 32 bits
+
+struct BoxPlan {
+    int how;
+    int x0, y0, k0;   // first node of the box (x, y before the periodic wrap)
+    int BX, BY, BZ;   // extents
+    int LD;           // row stride in LDS: kLZ (whole), else the slabs' own
+    int ns;           // planes per slab
+    int pairs;        // staged in 16-byte pieces (double fields)
+    int ax, ay, c;    // level k of row (x, y) sits at k - k0 + ((ax x + ay y + c) & 1)
+};
+
+// Double fields are staged in aligned 16-byte pieces, two levels each.  Row
+// (x, y) starts at element (rowidx SZ + k0) of the field, whose parity (and
+// that of the field's base address) decides whether its pieces start at level
+// k0 or k0 - 1; the row is shifted in LDS accordingly.  Rows of even length
+// (u, v at even nz) all shift alike, rows of odd length (w there) by turns in
+// y, and in x too when a plane holds an odd number of rows; a wrapped box
+// keeps the turns where the period is even.  A piece may reach one or two
+// elements out of its row, into a neighbouring row of the field (the first
+// and last rows of a field are ghost rows, never staged).
 template <typename T, int C, int P>
-__device__ inline bool stage_box(const Grid& g, const T* __restrict__ S, SBox& b,
-                                 T* __restrict__ lds, long cap_bytes, int& BY, int& BZ) {
-    bool dma = false;
-    if constexpr (SLC_STAGE_DMA && sizeof(T) == 8)
-        dma = (Comp<C>::SZ(g) % 2 == 0) && ((reinterpret_cast<uintptr_t>(S) & 15) == 0);
-    // extents in 64 bits, each bounded before the product: feet far outside
+__device__ inline BoxPlan plan_box(const Grid& g, const T* S, const SBox& b, int cap_bytes) {
+    BoxPlan r{BOX_NONE, b.xmin, b.ymin, b.kmin, 0, 1, 1, 1, 0, 0, 0, 0, 0};
+    if (b.xmin > b.xmax) return r;  // no live point
+    r.how = BOX_DIRECT;
+    // extents in 64 bits, each bounded before a product: feet far outside
     // the domain (or non-finite ones, whose floors saturate) would overflow
-    // int extents and must take the direct-load path
+    // int extents and take the direct loads
     const long ex = (long)b.xmax - b.xmin + P, ey = (long)b.ymax - b.ymin + P;
-    auto fits_z = [&](long ez) {
-        return b.xmin <= b.xmax && ex <= cap_bytes && ey <= cap_bytes && ez <= cap_bytes &&
-               ex * ey * ez * (long)sizeof(T) + ex * ey * 4 <= cap_bytes;
-    };
-    // the even start and extent can add two levels: a box that fits only
-    // without them is staged through registers
-    if (dma) {
-        const long ezd = (long)b.kmax - (b.kmin & ~1) + P;
-        dma = fits_z(ezd + (ezd & 1));
-    }
-    const int k0 = dma ? (b.kmin & ~1) : b.kmin;
-    long ez = (long)b.kmax - k0 + P;
-    if (dma) ez += ez & 1;
-    const bool fits = fits_z(ez);
-    const int BX = fits ? (int)ex : 0;
-    BY = fits ? (int)ey : 1;
-    BZ = fits ? (int)ez : 1;
-    const int rows = BX * BY;
-    const int nbox = rows * BZ;
-    if (fits) {
-        b.kmin = k0;
-        int* rowbase = reinterpret_cast<int*>(lds + nbox);
-        for (int r = threadIdx.x; r < rows; r += kSB) {
-            const int x = r / BY, y = r - (r / BY) * BY;
-            rowbase[r] = node_addr<C>(g, wrap_idx(b.xmin + x, g.nx),
-                                      wrap_idx(b.ymin + y, g.ny), k0);
-        }
-        __syncthreads();
-        if (dma) {
-            // pair q = 2 elements; a wavefront's 64 lanes load 64 consecutive
-            // pairs into 1 KB of consecutive LDS per instruction; (row, zz) of
-            // element 2q carried from one iteration to the next as below
-            const int npairs = nbox / 2;
-            const int lane = (int)threadIdx.x & 63;
-            const int step = 2 * kSB;  // elements per iteration
-            const int dq = step / BZ, dr = step - dq * BZ;
-            int q = (int)threadIdx.x;
-            int row = 2 * q / BZ;
-            int zz = 2 * q - row * BZ;
-#ifndef SLC_STAGE_DMA_UNROLL
-#define SLC_STAGE_DMA_UNROLL 2  // 1, 2, 4 measured the same at 256^3
-#endif
-#pragma unroll SLC_STAGE_DMA_UNROLL
-            for (int base = q - lane; base < npairs; base += kSB) {
-                if (q < npairs)
-                    __builtin_amdgcn_global_load_lds(
-                        (const __attribute__((address_space(1))) void*)(S + rowbase[row] + zz),
-                        (__attribute__((address_space(3))) void*)(lds + 2 * base), 16, 0, 0);
-                q += kSB;
-                row += dq;
-                zz += dr;
-                if (zz >= BZ) {
-                    zz -= BZ;
-                    ++row;
-                }
-            }
-        } else {
-            // flat element loop (z fastest: coalesced rows), e = row BZ + zz
-            // carried from one iteration to the next: e grows by kSB = dq BZ + dr
-            // with dr < BZ, so zz + dr < 2 BZ needs at most one carry
-            const int dq = kSB / BZ, dr = kSB - dq * BZ;
-            int row = (int)threadIdx.x / BZ;
-            int zz = (int)threadIdx.x - row * BZ;
-            // unrolled: the iterations are independent, so several row-base
-            // reads and global loads are in flight before the first wait
-            // (measured at 256^3 order 6: fused pass 2.05 -> 1.92 ms)
-#ifndef SLC_STAGE_UNROLL
-#define SLC_STAGE_UNROLL 4
-#endif
-#pragma unroll SLC_STAGE_UNROLL
-            for (int e = threadIdx.x; e < nbox; e += kSB) {
-                lds[e] = S[rowbase[row] + zz];
-                row += dq;
-                zz += dr;
-                if (zz >= BZ) {
-                    zz -= BZ;
-                    ++row;
-                }
-            }
+    const int ez = b.kmax - b.kmin + P;  // bases are clamped to the column
+    const long cap = cap_bytes / (int)sizeof(T);
+    if (ex > 65536 || ey > cap || b.xmin < -kFar || b.xmax > kFar || b.ymin < -kFar ||
+        b.ymax > kFar)
+        return r;
+    r.BX = (int)ex;
+    r.BY = (int)ey;
+    r.BZ = ez;
+    int ld = ez;
+    if (sizeof(T) == 8) {
+        const int SZ = (int)Comp<C>::SZ(g), SY = (int)Comp<C>::SY(g);
+        const int ay = SZ & 1, ax = SZ & SY & 1;
+        const bool oky = !ay || g.ny % 2 == 0 || (b.ymin >= 0 && b.ymin + r.BY <= g.ny);
+        const bool okx = !ax || g.nx % 2 == 0 || (b.xmin >= 0 && b.xmin + r.BX <= g.nx);
+        if (okx && oky) {
+            r.pairs = 1;
+            r.ax = ax;
+            r.ay = ay;
+            const int row0 = (wrap_idx(b.xmin, g.nx) + Comp<C>::ox) * SY +
+                             wrap_idx(b.ymin, g.ny) + Comp<C>::oy;
+            r.c = (int)((reinterpret_cast<uintptr_t>(S) >> 3) + (unsigned)(row0 * SZ + b.kmin)) & 1;
+            ld = (ez + (ay | r.c) + 1) & ~1;
         }
     }
-    __syncthreads();
-    return fits;
+    if (ld <= kLZ && ex * ey * kLZ <= cap) {
+        r.how = BOX_WHOLE;
+        r.LD = kLZ;
+        r.ns = r.BX;
+        return r;
+    }
+    // past eight slabs the box holds about as many values as the stencils do
+    if (ey * ld > cap || ex * ey * ld > 8 * cap) return r;
+    r.how = BOX_SLABS;
+    r.LD = ld;
+    // planes per slab: floor by a float reciprocal, corrected by one (both
+    // below 2^24, so the error is below one)
+    const int pl = r.BY * ld;
+    int ns = (int)((float)cap / (float)pl);
+    if ((long)ns * pl > cap) --ns;
+    r.ns = min(max(ns, 1), r.BX);
+    return r;
 }
 
-// z weights of one foot's order-P stencil against the node tables
-// (semilag.py:441-454): the part of the weights that reads memory.
+// Boxes of doubles are staged by gfx950's direct global-to-LDS loads (no
+// register round trip, no vector arithmetic per load): lane l of a wavefront's
+// load lands 16 l (4 l) bytes behind the wave-uniform LDS address.  staged()
+// waits for them.
+__device__ inline void load16_to_lds(const void* src, void* lds) {
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                     (__attribute__((address_space(3))) void*)lds, 16, 0, 0);
+}
+
+__device__ inline void load4_to_lds(const void* src, void* lds) {
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                     (__attribute__((address_space(3))) void*)lds, 4, 0, 0);
+}
+
+__device__ inline void staged() {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+}
+
+// Planes [s0, s0 + n) of the box in 16-byte pieces.  A wavefront takes every
+// kTileWaves-th plane, RPI rows of LD / 2 pieces per load (lane = rr LD / 2 +
+// zp; the pieces that hold levels of the box are loaded), so a plane's address
+// is scalar and a row's offset is formed once for all planes (twice where the
+// shift turns in x).
+template <int C, bool BIG>
+__device__ inline void stage_pairs(const Grid& g, const double* __restrict__ S, const BoxPlan& b,
+                                   int s0, int n, int LD, int RPI, int tid, int rr, int zp,
+                                   double* __restrict__ lds) {
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const unsigned SZ = (unsigned)Comp<C>::SZ(g), SY = (unsigned)Comp<C>::SY(g);
+    for (int y0 = 0; y0 < b.BY; y0 += RPI) {
+        const int y = y0 + rr;
+        const int sh = (b.ay * y + b.c + b.ax * (s0 + wave)) & 1;  // kTileWaves is even
+        if (rr >= RPI || y >= b.BY || 2 * zp >= b.BZ + sh) continue;
+        const int yg = wrap_idx(b.y0 + y, g.ny);
+        const unsigned off = (BIG ? (unsigned)yg * SZ : __umul24((unsigned)yg, SZ)) +
+                             (unsigned)(2 * zp - sh);
+        for (int x = wave; x < n; x += kTileWaves) {
+            const int xg = wrap_idx(b.x0 + s0 + x, g.nx);
+            const double* plane = S + (((unsigned)(xg + Comp<C>::ox) * SY + Comp<C>::oy) * SZ +
+                                       (unsigned)b.k0);
+            load16_to_lds(plane + (long)(int)off, lds + (x * b.BY + y0) * LD);
+        }
+    }
+}
+
+// Planes [s0, s0 + n) of the box into rows of LD elements, in 4-byte pieces: a
+// row of up to 64 of them per load (any alignment and extent), rows dealt
+// round robin to the wavefronts, addresses scalar but for the lane's place in
+// the row.
+template <typename T, int C>
+__device__ inline void stage_rows(const Grid& g, const T* __restrict__ S, const BoxPlan& b,
+                                  int s0, int n, int LD, T* __restrict__ lds) {
+    const int tid = phase_tid();
+    const unsigned lane = (unsigned)tid & 63u;
+    const unsigned nd = (unsigned)b.BZ * (unsigned)(sizeof(T) / 4);
+    const unsigned SZ = (unsigned)Comp<C>::SZ(g), SY = (unsigned)Comp<C>::SY(g);
+    for (unsigned d = 0; d < nd; d += 64) {  // one turn but for boxes over 32 levels
+        if (d + lane >= nd) break;
+        // row (x, y): y advances by kTileWaves <= P <= BY, one carry
+        int x = 0, y = __builtin_amdgcn_readfirstlane(tid >> 6);
+        while (x < n) {
+            const int xg = wrap_idx(b.x0 + s0 + x, g.nx), yg = wrap_idx(b.y0 + y, g.ny);
+            const T* row = S + (((unsigned)(xg + Comp<C>::ox) * SY +
+                                 (unsigned)(yg + Comp<C>::oy)) * SZ + (unsigned)b.k0);
+            load4_to_lds(reinterpret_cast<const unsigned*>(row) + (d + lane),
+                         reinterpret_cast<unsigned*>(lds + (x * b.BY + y) * LD) + d);
+            y += kTileWaves;
+            if (y >= b.BY) {
+                y -= b.BY;
+                ++x;
+            }
+        }
+    }
+}
+
+// A whole box of floats, four levels per lane and load (the last may reach out
+// of its row, as the pieces above), through registers
+// (unaligned 16-byte loads; in 4-byte direct loads the fused pass of u took
+// 590 us at 256x192x160, order 4, against 548).
+template <int C, bool BIG>
+__device__ inline void stage_quads(const Grid& g, const float* __restrict__ S, const BoxPlan& b,
+                                   float* __restrict__ lds) {
+    constexpr int NP = kLZ / 4, RPI = 64 / NP;
+    const int tid = phase_tid(), lane = tid & 63, rr = lane / NP, zp = lane % NP;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const unsigned SZ = (unsigned)Comp<C>::SZ(g), SY = (unsigned)Comp<C>::SY(g);
+    struct __attribute__((packed, aligned(4))) Quad {
+        float a, b, c, d;
+    };
+    for (int y0 = 0; y0 < b.BY; y0 += RPI) {
+        const int y = y0 + rr;
+        if (y >= b.BY || 4 * zp >= b.BZ) continue;
+        const int yg = wrap_idx(b.y0 + y, g.ny);
+        const unsigned off =
+            (BIG ? (unsigned)yg * SZ : __umul24((unsigned)yg, SZ)) + (unsigned)(4 * zp);
+        // three loads in flight per lane
+#pragma unroll 3
+        for (int x = wave; x < b.BX; x += kTileWaves) {
+            const int xg = wrap_idx(b.x0 + x, g.nx);
+            const float* plane = S + (((unsigned)(xg + Comp<C>::ox) * SY + Comp<C>::oy) * SZ +
+                                      (unsigned)b.k0);
+            const Quad q = *reinterpret_cast<const Quad*>(elem<BIG>(plane, off));
+            *reinterpret_cast<float4*>(lds + (x * b.BY + y) * kLZ + 4 * zp) =
+                make_float4(q.a, q.b, q.c, q.d);
+        }
+    }
+}
+
+template <typename T, int C, bool BIG>
+__device__ inline void stage_whole(const Grid& g, const T* __restrict__ S, const BoxPlan& b,
+                                   T* __restrict__ lds) {
+    if constexpr (sizeof(T) == 4) {
+        stage_quads<C, BIG>(g, S, b, lds);
+    } else if (b.pairs) {
+        constexpr int NP = kLZ / 2;
+        const int tid = phase_tid(), lane = tid & 63;
+        stage_pairs<C, BIG>(g, S, b, 0, b.BX, kLZ, 64 / NP, tid, lane / NP, lane % NP, lds);
+    } else {
+        stage_rows<T, C>(g, S, b, 0, b.BX, kLZ, lds);
+    }
+}
+
+template <typename T, int C, bool BIG>
+__device__ inline void stage_slab(const Grid& g, const T* __restrict__ S, const BoxPlan& b,
+                                  int s0, int n, T* __restrict__ lds) {
+    if constexpr (sizeof(T) == 8) {
+        if (b.pairs && b.LD <= 128) {
+            // lane / NP and 64 / NP by a float reciprocal: the operands are small
+            // integers, and half a unit keeps the quotient off the integers
+            const int tid = phase_tid(), lane = tid & 63, NP = b.LD >> 1;
+            const float rz = 1.0f / (float)NP;
+            const int RPI = __builtin_amdgcn_readfirstlane((int)(64.5f * rz));
+            const int rr = (int)(((float)lane + 0.5f) * rz);
+            stage_pairs<C, BIG>(g, S, b, s0, n, b.LD, RPI, tid, rr, lane - rr * NP, lds);
+            return;
+        }
+    }
+    stage_rows<T, C>(g, S, b, s0, n, b.LD, lds);
+}
+
+// Weights of one foot's order-P stencil (z against the node tables,
+// semilag.py:441-454).
+// The x weights are formed after the planes' sums, which take their place in
+// the registers.
 template <int P>
-struct ZWeights {
-    double wz[P];
+struct Weights {
+    double y[P], z[P];
 };
 
 template <int C, int P>
-__device__ inline void zweights(const Grid& g, const FootSt& f, ZWeights<P>& w) {
+__device__ inline void weights(const Grid& g, const FootSt& f, Weights<P>& w) {
     const double* zn = znodes<C>(g);
     const double* dinv = Comp<C>::centers ? g.dinv_cP : g.dinv_fP;
-    z_weights<P>(zn, dinv, f.z, f.bk, w.wz);
+    z_weights<P>(zn, dinv, f.z, f.bk, w.z);
+    uniform_weights<P>(f.ty, w.y);
 }
 
-// Order-P gather of one foot given its z weights: the x and y weights, then
-// the staged z -> y -> x contraction with FMAs, from the LDS box when it was
-// staged, else from S.
-template <typename T, int C, int P>
-__device__ inline double contract_w(const Grid& g, const FootSt& f, const ZWeights<P>& w,
-                                    const SBox& b, bool fits, const T* __restrict__ lds,
-                                    int BY, int BZ, const T* __restrict__ S) {
-    double wx[P], wy[P];
+// The x sum over the stencil planes' values a.
+template <int P>
+__device__ inline double x_sum(const FootSt& f, const double (&a)[P]) {
+    double wx[P], acc = 0.0;
     uniform_weights<P>(f.tx, wx);
-    uniform_weights<P>(f.ty, wy);
-    const double* wz = w.wz;
+#pragma unroll
+    for (int i = 0; i < P; ++i) acc = fma(wx[i], a[i], acc);
+    return acc;
+}
+
+// One stencil plane, z then y, from LDS with row stride LD: even rows from c0,
+// odd rows from c1 (their levels may sit one place apart, BoxPlan).
+template <typename T, int P>
+__device__ inline double plane_sum(const Weights<P>& w, const T* __restrict__ c0,
+                                   const T* __restrict__ c1, int LD) {
+    double ai = 0.0;
+#pragma unroll
+    for (int j = 0; j < P; ++j) {
+        const T* col = (j & 1 ? c1 : c0) + j * LD;
+        double sj = 0.0;
+#pragma unroll
+        for (int k = 0; k < P; ++k) sj = fma(w.z[k], (double)col[k], sj);
+        ai = fma(w.y[j], sj, ai);
+    }
+    return ai;
+}
+
+// First values of the even and odd rows of the stencil's planes in a staged
+// box whose plane s0 comes first: c[0], c[1] in its even planes, c[2], c[3] in
+// its odd ones (plane 0 of the stencil may lie before the box).
+template <typename T>
+__device__ inline void stencil_rows(const FootSt& f, const BoxPlan& b, int ox, int LD,
+                                    const T* __restrict__ lds, const T* (&c)[4]) {
+    const int oy = f.by - b.y0;
+    const T* col = lds + ((ox * b.BY + oy) * LD + (f.bk - b.k0));
+    const int sh = (b.ax * (f.bx - b.x0) + b.ay * oy + b.c) & 1;
+    c[0] = col + sh;
+    c[1] = col + (sh ^ b.ay);
+    c[2] = col + (sh ^ b.ax);
+    c[3] = col + (sh ^ b.ay ^ b.ax);
+}
+
+// The staged z -> y -> x contraction with FMAs from a whole box.  The row
+// stride is a compile-time constant: a plane's rows are read at immediate
+// offsets from two lane addresses.
+template <typename T, int P>
+__device__ inline double contract_whole(const FootSt& f, const Weights<P>& w, const BoxPlan& b,
+                                        const T* __restrict__ lds) {
+    const T* c[4];
+    stencil_rows<T>(f, b, f.bx - b.x0, kLZ, lds, c);
+    const int step = b.BY * kLZ;
+    double a[P];
+#pragma unroll
+    for (int i = 0; i < P; ++i)
+        a[i] = plane_sum<T, P>(w, c[2 * (i & 1)] + i * step, c[2 * (i & 1) + 1] + i * step, kLZ);
+    return x_sum<P>(f, a);
+}
+
+// The planes of the slab [s0, s0 + n) that belong to the lane's stencil, into
+// their places of a.
+template <typename T, int P>
+__device__ inline void contract_slab(const FootSt& f, const Weights<P>& w, const BoxPlan& b,
+                                     int s0, int n, const T* __restrict__ lds, double (&a)[P]) {
+    const int ox = f.bx - b.x0 - s0;
+    const T* c[4];
+    stencil_rows<T>(f, b, ox, b.LD, lds, c);
+    const int step = b.BY * b.LD;
+#pragma unroll
+    for (int i = 0; i < P; ++i)
+        if ((unsigned)(ox + i) < (unsigned)n)
+            a[i] = plane_sum<T, P>(w, c[2 * (i & 1)] + i * step, c[2 * (i & 1) + 1] + i * step,
+                                   b.LD);
+}
+
+// The same sum by loads from the field S; rolled over the planes.
+template <typename T, int C, int P>
+__device__ inline double contract_direct(const Grid& g, const FootSt& f, const Weights<P>& w,
+                                         const T* __restrict__ S) {
+    // the base wrapped, then a step at a time, as build_stencil does (a
+    // saturated base must not leave 32 bits)
     double acc = 0.0;
-    if (fits) {
-        const int ox = f.bx - b.xmin, oy = f.by - b.ymin, oz = f.bk - b.kmin;
-#pragma unroll
-        for (int i = 0; i < P; ++i) {
-            double ai = 0.0;
-#pragma unroll
-            for (int j = 0; j < P; ++j) {
-                const T* col = lds + ((ox + i) * BY + (oy + j)) * BZ + oz;
-                double sj = 0.0;
-#pragma unroll
-                for (int k = 0; k < P; ++k) sj = fma(wz[k], (double)col[k], sj);
-                ai = fma(wy[j], sj, ai);
-            }
-            acc = fma(wx[i], ai, acc);
-        }
-    } else {
+    int gx = wrap_idx(f.bx, g.nx);
+    const int gy0 = wrap_idx(f.by, g.ny);
 #pragma unroll 1
-        for (int i = 0; i < P; ++i) {
-            const int gx = wrap_idx(f.bx + i, g.nx);
-            double ai = 0.0;
+    for (int i = 0; i < P; ++i) {
+        double ai = 0.0;
+        int gy = gy0;
 #pragma unroll
-            for (int j = 0; j < P; ++j) {
-                const int gy = wrap_idx(f.by + j, g.ny);
-                const T* col = S + node_addr<C>(g, gx, gy, f.bk);
-                double sj = 0.0;
+        for (int j = 0; j < P; ++j) {
+            const T* col = S + node_addr<C>(g, gx, gy, f.bk);
+            double sj = 0.0;
 #pragma unroll
-                for (int k = 0; k < P; ++k) sj = fma(wz[k], (double)col[k], sj);
-                ai = fma(wy[j], sj, ai);
-            }
-            acc = fma(uniform_weight_m<P>(f.tx, i), ai, acc);
+            for (int k = 0; k < P; ++k) sj = fma(w.z[k], (double)col[k], sj);
+            ai = fma(w.y[j], sj, ai);
+            gy = gy + 1 == g.ny ? 0 : gy + 1;
         }
+        acc = fma(uniform_weight_m<P>(f.tx, i), ai, acc);
+        gx = gx + 1 == g.nx ? 0 : gx + 1;
     }
     return acc;
 }
 
-// Weights, then the contraction.
-template <typename T, int C, int P>
-__device__ inline double contract(const Grid& g, const FootSt& f, const SBox& b, bool fits,
-                                  const T* __restrict__ lds, int BY, int BZ,
-                                  const T* __restrict__ S) {
-    ZWeights<P> w;
-    zweights<C, P>(g, f, w);
-    return contract_w<T, C, P>(g, f, w, b, fits, lds, BY, BZ, S);
+// Arrival point of interior index (i, j, k) (arrival<C> without the linear
+// index).
+template <int C>
+__device__ inline void arrival_at(const Grid& g, int i, int j, int k, double& xa, double& ya,
+                                  double& za) {
+    const double ar = (double)(i + 1), aj = (double)(j + 1);
+    xa = (C == 0 ? ar : ar - 0.5) * g.dx;
+    ya = (C == 1 ? aj : aj - 0.5) * g.dy;
+    za = *elem<false>(znodes<C>(g), (unsigned)(k + 1));
+}
+
+// Element (i+1, j+1, k+1) of component C's ghost-shaped array.
+template <int C>
+__device__ inline unsigned field_elem(const Grid& g, int i, int j, int k) {
+    const unsigned SZ = (unsigned)Comp<C>::SZ(g), SY = (unsigned)Comp<C>::SY(g);
+    return ((unsigned)(i + 1) * SY + (unsigned)(j + 1)) * SZ + (unsigned)(k + 1);
+}
+
+// Elements of the five-point xy stencil around interior point (i, j, .) at
+// element o (operators.py:293-367; periodic extension for u in x, v in y).
+struct XYStar {
+    unsigned o, xp, xm, yp, ym;
+};
+
+template <int C>
+__device__ inline XYStar xy_star(const Grid& g, int i, int j, unsigned o) {
+    const unsigned SZ = (unsigned)Comp<C>::SZ(g), PS = (unsigned)Comp<C>::SY(g) * SZ;
+    XYStar q{o, o + PS, o - PS, o + SZ, o - SZ};
+    if (C == 0 && i == g.nx - 1) q.xp = o - (unsigned)(g.nx - 1) * PS;
+    if (C == 1 && j == g.ny - 1) q.yp = o - (unsigned)(g.ny - 1) * SZ;
+    return q;
+}
+
+// rhs_xy (slc_device.h) over those elements.
+template <bool BIG>
+__device__ inline double rhs_star(const Grid& g, const double* __restrict__ F, const XYStar& q,
+                                  double rdx2, double rdy2) {
+    const double c = *elem<BIG>(F, q.o);
+    const double d2x = ((*elem<BIG>(F, q.xp) - 2.0 * c) + *elem<BIG>(F, q.xm)) * rdx2;
+    const double d2y = ((*elem<BIG>(F, q.yp) - 2.0 * c) + *elem<BIG>(F, q.ym)) * rdy2;
+    return g.nu * (d2x + d2y);
 }
 
 __device__ inline void box_add(SBox& l, const FootSt& f) {
@@ -449,7 +735,7 @@ __device__ inline void box_add(SBox& l, const FootSt& f) {
 
 // Iterated midpoint (semilag.py:534-552) from the arrival point with its
 // shared first sample (u0, v0, w0); returns the unclamped foot.
-template <int C>
+template <int C, bool BIG>
 __device__ inline void trace_foot(const Grid& g, const TrajA& V, double xa, double ya,
                                   double za, int K, double u0, double v0, double w0, double h,
                                   double& x, double& y, double& z) {
@@ -457,7 +743,7 @@ __device__ inline void trace_foot(const Grid& g, const TrajA& V, double xa, doub
     double zm = clampd(za - h * w0, g.z_lo, g.z_hi);
     for (int it = 1; it < g.n_iters; ++it) {
         double us, vs, ws;
-        sample3<C>(g, V, xm, ym, zm, za, K, us, vs, ws);
+        sample3<C, BIG>(g, V, xm, ym, zm, za, K, us, vs, ws);
         xm = xa - h * us;
         ym = ya - h * vs;
         zm = clampd(za - h * ws, g.z_lo, g.z_hi);
@@ -473,8 +759,7 @@ __device__ inline void trace_foot(const Grid& g, const TrajA& V, double xa, doub
 // FP64).  F / Fm are always the FP64 fields (explicit xy-diffusion);
 // Sn / Sm are the gathered copies (== F / Fm when T is double).
 // One tile of the step kernel (tile = linear tile index, k fastest).  The
-// caller provides the block's LDS: lds (LDS_BYTES), sh (6 ints; 12 for
-// MODE_BDF2), s_cnt, and for MODE_BDF2 nst (one FootSt per tile point).
+// caller provides the block's LDS (TileLds).
 // defer (MODE_GATHER): when non-null, one flag per tile: 1 for a tile whose
 // box does not fit the LDS budget (it is not gathered here but left for a
 // pass with a larger budget), 0 for the others.
@@ -492,153 +777,196 @@ __device__ inline bool redo_point(const Redo& r, const Grid& g, int nzi, int i, 
     return r.flags[((long)(i / r.ti) * rtj + j / r.tj) * rtk + k / r.tk] != 0u;
 }
 
-template <typename T, int C, int P, int MODE, int TI, int TJ, int TK, int LDS_BYTES>
+// LDS of a tile workgroup.
+template <typename T, int MODE, int NPT, int LDS_BYTES>
+struct TileLds {
+    static constexpr int NN = MODE == MODE_BDF2 ? NPT : 1;
+    __align__(16) T box[LDS_BYTES / sizeof(T)];
+    __align__(16) BoxRed red;
+    // near stencils (MODE_BDF2), waiting for the far gather
+    double ntx[NN], nty[NN], nz[NN];
+    int nbx[NN], nby[NN], nbk[NN];
+};
+
+template <typename T, int C, int P, int MODE, int TI, int TJ, int TK, int LDS_BYTES, bool BIG>
 __device__ __forceinline__ void sl_tile_body(
     const Grid& g, const ArrivalTabs& A, const TrajVel& V, const double* __restrict__ F,
     const double* __restrict__ Fm, const T* __restrict__ Sn, const T* __restrict__ Sm,
-    double dt, double* __restrict__ out, const Feet& ft, unsigned long long* nclamp, long tile,
-    T* __restrict__ lds, int* sh, int* s_cnt, FootSt* nst = nullptr,
-    unsigned* defer = nullptr, Redo redo = Redo{}) {
+    double dt, double* __restrict__ out, const Feet& ft, unsigned long long* nclamp, unsigned tile,
+    TileLds<T, MODE, TI * TJ * TK, LDS_BYTES>& L, unsigned* defer = nullptr,
+    Redo redo = Redo{}) {
     constexpr int NPT = TI * TJ * TK;
     static_assert(NPT % kSB == 0, "tile must be a multiple of the block");
     constexpr int PT = NPT / kSB;
+    constexpr bool BOTH = MODE == MODE_FAR || MODE == MODE_BDF2;  // both feet traced
+    constexpr bool RHS = MODE == MODE_BDF1 || MODE == MODE_NEAR || MODE == MODE_BDF2;
     const int nzi = Comp<C>::NZI(g);
-    const int ntk = (nzi + TK - 1) / TK, ntj = (g.ny + TJ - 1) / TJ;
+    const unsigned ntk = (unsigned)(nzi + TK - 1) / TK, ntj = (unsigned)(g.ny + TJ - 1) / TJ;
     // the step kernels' trajectory velocity is always a stored field
     const TrajA VA{{V.a[0], V.a[1], V.a[2]}};
-    const int tk = (int)(tile % ntk);
-    const long r0 = tile / ntk;
-    const int tj = (int)(r0 % ntj), ti = (int)(r0 / ntj);
-    const int i0 = ti * TI, j0 = tj * TJ, k0t = tk * TK;
+    const unsigned r0 = tile / ntk, tk = tile - r0 * ntk;
+    const unsigned ti = r0 / ntj, tj = r0 - ti * ntj;
+    const int i0 = (int)ti * TI, j0 = (int)tj * TJ, k0t = (int)tk * TK;
 
     // ---- phase 1: feet and stencils --------------------------------------
-    long idx[PT];
+    // lane's point p: (i, j, k), z fastest
+    auto point = [&](int tid, int p, int& i, int& j, int& k) {
+        const int q = tid + kSB * p;
+        i = i0 + q / (TK * TJ);
+        j = j0 + (q / TK) % TJ;
+        k = k0t + q % TK;
+    };
+    bool live[PT];
     FootSt st[PT];
     SBox l{INT_MAX, INT_MIN, INT_MAX, INT_MIN, INT_MAX, INT_MIN};
     SBox ln{INT_MAX, INT_MIN, INT_MAX, INT_MIN, INT_MAX, INT_MIN};  // MODE_BDF2 near box
     int ncl = 0;
 #pragma unroll
     for (int p = 0; p < PT; ++p) {
-        const int q = threadIdx.x + kSB * p;
-        const int kk = q % TK, t2 = q / TK;
-        const int jj = t2 % TJ, ii = t2 / TJ;
-        const int i = i0 + ii, j = j0 + jj, k = k0t + kk;
-        idx[p] = -1;
-        if (i < g.nx && j < g.ny && k < nzi &&
-            (MODE != MODE_GATHER || redo_point(redo, g, nzi, i, j, k))) {
-            const long n = ((long)i * g.ny + j) * nzi + k;
-            idx[p] = n;
-            double xa, ya, za;
-            int I, J, K;
-            arrival<C>(g, n, xa, ya, za, I, J, K);
+        int i, j, k;
+        point((int)threadIdx.x, p, i, j, k);
+        live[p] = i < g.nx && j < g.ny && k < nzi &&
+                  (MODE != MODE_GATHER || redo_point(redo, g, nzi, i, j, k));
+        if (live[p]) {
+            const unsigned n = ((unsigned)i * g.ny + j) * nzi + k;
             double x, y, z;
             if (MODE == MODE_NEAR || MODE == MODE_GATHER) {
-                x = ft.x[n];
-                y = ft.y[n];
-                z = ft.z[n];
+                x = *elem<BIG>(ft.x, n);
+                y = *elem<BIG>(ft.y, n);
+                z = *elem<BIG>(ft.z, n);
             } else {
+                const int K = k + 1;
+                double xa, ya, za;
+                arrival_at<C>(g, i, j, k, xa, ya, za);
                 // the first sample is at the arrival point for every foot depth
                 double u0, v0, w0;
-                sample3_at(g, VA, A.xdx[I - 1], A.ydy[J - 1], za, A.csel[K - 1], u0, v0, w0);
-                if (MODE == MODE_FAR || MODE == MODE_BDF2) {
+                const int csel = A.csel[k], c = csel >> 1;
+                sample3_at<BIG>(g, VA, over_dx(g, xa), over_dy(g, ya),
+                                clampd(za, g.z_lo, g.z_hi), c, c + (csel & 1), u0, v0, w0);
+                if (BOTH) {
                     // the near foot first: it leaves the registers (to LDS or
                     // to the feet arrays) before the far foot is traced
                     double xn, yn, zn;
-                    trace_foot<C>(g, VA, xa, ya, za, K, u0, v0, w0, 0.5 * dt, xn, yn, zn);
+                    trace_foot<C, BIG>(g, VA, xa, ya, za, K, u0, v0, w0, 0.5 * dt, xn, yn, zn);
                     if (MODE == MODE_FAR) {
-                        ft.x[n] = xn;
-                        ft.y[n] = yn;
-                        ft.z[n] = zn;
+                        *elem<BIG>(ft.x, n) = xn;
+                        *elem<BIG>(ft.y, n) = yn;
+                        *elem<BIG>(ft.z, n) = zn;
                     } else {
                         FootSt sn;
                         make_st<C, P>(g, xn, yn, zn, sn, ncl);
                         box_add(ln, sn);
-                        nst[q] = sn;
+                        const int q = threadIdx.x + kSB * p;
+                        L.ntx[q] = sn.tx;
+                        L.nty[q] = sn.ty;
+                        L.nz[q] = sn.z;
+                        L.nbx[q] = sn.bx;
+                        L.nby[q] = sn.by;
+                        L.nbk[q] = sn.bk;
                     }
                 }
-                trace_foot<C>(g, VA, xa, ya, za, K, u0, v0, w0,
-                           (MODE == MODE_FAR || MODE == MODE_BDF2) ? 0.5 * (2.0 * dt) : 0.5 * dt,
-                           x, y, z);
+                trace_foot<C, BIG>(g, VA, xa, ya, za, K, u0, v0, w0,
+                                   BOTH ? 0.5 * (2.0 * dt) : 0.5 * dt, x, y, z);
             }
             make_st<C, P>(g, x, y, z, st[p], ncl);
             box_add(l, st[p]);
         }
     }
+    box_reduce(l, L.red.v[0]);
+    if (MODE == MODE_BDF2) box_reduce(ln, L.red.v[1]);
+    __syncthreads();
 
-    // ---- stage the tile's stencil box in LDS -------------------------------
-    // With one point per lane, the z weights are formed before the box is
-    // staged, so their table loads are in flight with the staging's.
-    constexpr bool HOIST = PT == 1;
-    ZWeights<P> w0;
-    if (HOIST && idx[0] >= 0) zweights<C, P>(g, st[0], w0);
-    const T* __restrict__ S = (MODE == MODE_FAR || MODE == MODE_BDF2) ? Sm : Sn;
-    // MODE_BDF2: the near box is reduced with the far one and waits in
-    // sh[6..11], so no lane holds it through the far contraction
-    SBox b = (MODE == MODE_BDF2) ? s_block_box2(l, ln, sh) : s_block_box(l, sh);
-    int BY = 0, BZ = 0;
-    const bool fits = stage_box<T, C, P>(g, S, b, lds, LDS_BYTES, BY, BZ);
-    if (MODE == MODE_GATHER && defer) {  // fits is uniform over the block
-        if (threadIdx.x == 0) defer[tile] = fits ? 0u : 1u;
-        if (!fits) return;
-    }
-
-    // ---- phase 2: contract -------------------------------------------------
-    const double rdx2 = 1.0 / (g.dx * g.dx), rdy2 = 1.0 / (g.dy * g.dy);
-    double farv[PT];
-    if (MODE == MODE_BDF2) {
-        // far value of every point, then the near box into the same buffer
+    // ---- phase 2: stage a foot's box, contract; far foot, then near ---------
+    constexpr int NF = MODE == MODE_BDF2 ? 2 : 1;
+    double val[PT], farv[PT];
+#pragma unroll 1
+    for (int f = 0; f < NF; ++f) {
+        const T* __restrict__ S = (MODE == MODE_FAR || (MODE == MODE_BDF2 && f == 0)) ? Sm : Sn;
+        const BoxPlan b = plan_box<T, C, P>(g, S, box_union(L.red.v[f]), LDS_BYTES);
+        if (MODE == MODE_GATHER && defer) {
+            const bool later = b.how == BOX_DIRECT || (b.how == BOX_SLABS && b.BX > b.ns);
+            if (threadIdx.x == 0) defer[tile] = later ? 1u : 0u;
+            if (later) return;
+        }
+        if (b.how == BOX_WHOLE) stage_whole<T, C, BIG>(g, S, b, L.box);
+        // in flight with the box: the near stencils and the z tables
+        if (MODE == MODE_BDF2 && f == 1) {
+            const int tid = phase_tid();
+#pragma unroll
+            for (int p = 0; p < PT; ++p) {
+                const int q = tid + kSB * p;
+                if (live[p])
+                    st[p] = FootSt{L.nbx[q], L.nby[q], L.nbk[q], L.ntx[q], L.nty[q], L.nz[q]};
+            }
+        }
+        Weights<P> w[PT];
 #pragma unroll
         for (int p = 0; p < PT; ++p)
-            farv[p] = idx[p] < 0 ? 0.0
-                      : HOIST ? contract_w<T, C, P>(g, st[p], w0, b, fits, lds, BY, BZ, S)
-                              : contract<T, C, P>(g, st[p], b, fits, lds, BY, BZ, S);
-        __syncthreads();  // every lane is done with the far box
-        // the near stencils' weights, before the near box is staged
-        if (HOIST && idx[0] >= 0) zweights<C, P>(g, nst[threadIdx.x], w0);
+            if (live[p]) weights<C, P>(g, st[p], w[p]);
+        if (b.how == BOX_WHOLE) {
+            staged();
+#pragma unroll
+            for (int p = 0; p < PT; ++p)
+                if (live[p]) val[p] = contract_whole<T, P>(st[p], w[p], b, L.box);
+        } else if (b.how == BOX_SLABS) {
+            double a[PT][P] = {};
+            for (int s0 = 0; s0 < b.BX; s0 += b.ns) {
+                const int n = min(b.ns, b.BX - s0);
+                if (s0) __syncthreads();  // every lane is done with the last slab
+                stage_slab<T, C, BIG>(g, S, b, s0, n, L.box);
+                staged();
+#pragma unroll
+                for (int p = 0; p < PT; ++p)
+                    if (live[p]) contract_slab<T, P>(st[p], w[p], b, s0, n, L.box, a[p]);
+            }
+#pragma unroll
+            for (int p = 0; p < PT; ++p) val[p] = x_sum<P>(st[p], a[p]);
+        } else {
+#pragma unroll
+            for (int p = 0; p < PT; ++p)
+                if (live[p]) val[p] = contract_direct<T, C, P>(g, st[p], w[p], S);
+        }
+        if (f + 1 < NF) {
+#pragma unroll
+            for (int p = 0; p < PT; ++p) farv[p] = val[p];
+            __syncthreads();  // every lane is done with the far box
+        }
     }
-    SBox bn = (MODE == MODE_BDF2) ? SBox{sh[6], sh[7], sh[8], sh[9], sh[10], sh[11]} : b;
-    const bool fits_n = (MODE == MODE_BDF2) ? stage_box<T, C, P>(g, Sn, bn, lds, LDS_BYTES, BY, BZ)
-                                            : fits;
+    const int tid = phase_tid();
 #pragma unroll
     for (int p = 0; p < PT; ++p) {
-        if (idx[p] < 0) continue;
-        const long n = idx[p];
-        const double acc =
-            HOIST ? ((MODE == MODE_BDF2)
-                         ? contract_w<T, C, P>(g, nst[threadIdx.x], w0, bn, fits_n, lds, BY, BZ,
-                                               Sn)
-                         : contract_w<T, C, P>(g, st[p], w0, b, fits, lds, BY, BZ, S))
-            : (MODE == MODE_BDF2)
-                ? contract<T, C, P>(g, nst[threadIdx.x + kSB * p], bn, fits_n, lds, BY, BZ, Sn)
-                : contract<T, C, P>(g, st[p], b, fits, lds, BY, BZ, S);
-        // arrival ghost index of n
-        const unsigned un = (unsigned)n;
-        const int K = (int)(un % (unsigned)nzi) + 1;
-        const unsigned rr = un / (unsigned)nzi;
-        const int J = (int)(rr % (unsigned)g.ny) + 1, I = (int)(rr / (unsigned)g.ny) + 1;
-        const long o = ((long)I * Comp<C>::SY(g) + J) * Comp<C>::SZ(g) + K;
-        if (MODE == MODE_GATHER) {
-            out[n] = acc;
-        } else if (MODE == MODE_ADVECT || MODE == MODE_FAR) {
-            out[o] = acc;
-        } else if (MODE == MODE_BDF1) {
-            out[o] = acc + dt * rhs_xy<C>(g, F, I, J, K, rdx2, rdy2);
-        } else {
-            const double far = (MODE == MODE_BDF2) ? farv[p] : out[o];
-            const double rn = rhs_xy<C>(g, F, I, J, K, rdx2, rdy2);
+        if (!live[p]) continue;
+        int i, j, k;
+        point(tid, p, i, j, k);
+        const unsigned o = field_elem<C>(g, i, j, k);
+        double rh = 0.0;
+        if (RHS) {
+            const double rdx2 = 1.0 / (g.dx * g.dx), rdy2 = 1.0 / (g.dy * g.dy);
+            const XYStar q = xy_star<C>(g, i, j, o);
+            rh = rhs_star<BIG>(g, F, q, rdx2, rdy2);
             // Rh: 2R^n - R^{n-1} ('extrap') or R^n ('lagged'), solver.py:848-854
-            const double rh = g.xy_lagged ? rn : 2.0 * rn - rhs_xy<C>(g, Fm, I, J, K, rdx2, rdy2);
+            if (MODE != MODE_BDF1 && !g.xy_lagged)
+                rh = 2.0 * rh - rhs_star<BIG>(g, Fm, q, rdx2, rdy2);
+        }
+        if (MODE == MODE_GATHER) {
+            *elem<BIG>(out, ((unsigned)i * g.ny + j) * nzi + k) = val[p];
+        } else if (MODE == MODE_ADVECT || MODE == MODE_FAR) {
+            *elem<BIG>(out, o) = val[p];
+        } else if (MODE == MODE_BDF1) {
+            *elem<BIG>(out, o) = val[p] + dt * rh;
+        } else {
+            const double far = (MODE == MODE_BDF2) ? farv[p] : *elem<BIG>(out, o);
             const double dt_eff = (2.0 / 3.0) * dt;
-            const double pred = fma(far, -1.0 / 3.0, acc * (4.0 / 3.0));
-            out[o] = pred + dt_eff * rh;
+            const double pred = fma(far, -1.0 / 3.0, val[p] * (4.0 / 3.0));
+            *elem<BIG>(out, o) = pred + dt_eff * rh;
         }
     }
     if (nclamp) {
-        if (threadIdx.x == 0) *s_cnt = 0;
-        __syncthreads();
-        if (ncl) atomicAdd(s_cnt, ncl);
-        __syncthreads();
-        if (threadIdx.x == 0 && *s_cnt) atomicAdd(nclamp, (unsigned long long)*s_cnt);
+        // one or two clamped feet per lane, counted over the wavefront
+        int tot = 0;
+#pragma unroll
+        for (int c = 0; c < PT * (BOTH ? 2 : 1); ++c) tot += __popcll(__ballot(ncl > c));
+        if (tot && (threadIdx.x & 63) == 0) atomicAdd(nclamp, (unsigned long long)tot);
     }
 }
 
