@@ -15,7 +15,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OUT = os.path.join(HERE, "libslc_hip.so")
 BUILD = os.path.join(HERE, "_build")
-SOURCES = ["slc_api.hip", "slc_sl.hip", "slc_ops.hip", "slc_tiled.hip", "slc_step.hip",
+SOURCES = ["slc_api.hip", "slc_sl.hip", "slc_ops.hip", "slc_tiled.hip", "slc_step.hip", "slc_step3.hip",
            "slc_ens.hip", "slc_ens_kernels.hip", "slc_ens_tile_d4.hip", "slc_ens_tile_d6.hip",
            "slc_ens_tile_f4.hip", "slc_ens_tile_f6.hip", "slc_stats.hip",
            "slc_diag.hip", "slc_imex.hip", "slc_init.hip"]

@@ -302,7 +302,7 @@ int slc::plan_create(const slc_grid_desc* d, int device, bool spectral, slc_plan
         p->nfoot = (double*)ptr;
         {
             long tiles = 0;
-            for (int c = 0; c < 3; ++c) tiles = std::max(tiles, gather_tiles(g, c));
+            for (int c = 0; c < 3; ++c) tiles = std::max(tiles, step_tiles(g, c));
             if ((rc = dev_alloc(p, sizeof(unsigned) * (size_t)tiles, &ptr))) {
                 slc_plan_destroy(p);
                 return rc;
@@ -514,6 +514,25 @@ int slc_locate_z(slc_plan* p, int comp, const double* z, int64_t n, int32_t* m0_
     return SLC_OK;
 }
 
+// The tiled passes of the three components: one launch where the grid is small
+// (and the launch timer, which labels them one by one, is off).
+static int tile_passes(slc_plan* p, int mode, const TrajVel& V, const double* const F[3],
+                       const double* const Fm[3], const float* const Fn32[3],
+                       const float* const Fm32[3], double dt, double* const O[3],
+                       unsigned long long* ncl, const char* const labels[3], void* stream) {
+    if (!p->prof && step_tiles(p->g, 0) <= kMergeTiles && !big_index(p->g)) {
+        HIP_OK(run_tile_step3(p->g, mode, p->at, V, F, Fm, Fn32, Fm32, dt, O, ncl, S(stream)));
+        return SLC_OK;
+    }
+    for (int c = 0; c < 3; ++c) {
+        Timed t(p, labels[c], stream);
+        HIP_OK(run_tile_step(p->g, c, mode, p->at[c], V, F[c], Fm ? Fm[c] : nullptr,
+                             Fn32 ? Fn32[c] : nullptr, Fm32 ? Fm32[c] : nullptr, dt, O[c],
+                             nullptr, nullptr, nullptr, ncl, S(stream)));
+    }
+    return SLC_OK;
+}
+
 // The LDS-tiled step kernels trace with trilinear trajectories; tricubic ones
 // (traj_interp_order 4) run the direct-load kernels.
 static bool tiled_steps(const slc_plan* p) {
@@ -536,14 +555,14 @@ int slc_advect(slc_plan* p, const double* u, const double* v, const double* w, c
         Timed t(p, "to_f32", stream);
         HIP_OK(run_to_f32(p->g, p->f32n, F, S(stream)));
     }
+    if (tiled_steps(p)) {
+        const char* const labels[3] = {kLabel[0][3], kLabel[1][3], kLabel[2][3]};
+        return tile_passes(p, 0, V, F, nullptr, f32 ? p->f32n : nullptr, nullptr, dt, O, ncl,
+                           labels, stream);
+    }
     for (int c = 0; c < 3; ++c) {
         Timed t(p, kLabel[c][3], stream);
-        if (tiled_steps(p))
-            HIP_OK(run_tile_step(p->g, c, 0, p->at[c], V, F[c], nullptr,
-                                 f32 ? p->f32n[c] : nullptr, nullptr, dt, O[c], nullptr,
-                                 nullptr, nullptr, ncl, S(stream)));
-        else
-            HIP_OK(run_advect(p->g, c, V, F[c], dt, O[c], ncl, S(stream)));
+        HIP_OK(run_advect(p->g, c, V, F[c], dt, O[c], ncl, S(stream)));
     }
     return SLC_OK;
 }
@@ -563,14 +582,14 @@ int slc_bdf1_predict(slc_plan* p, const double* u, const double* v, const double
         Timed t(p, "to_f32", stream);
         HIP_OK(run_to_f32(p->g, p->f32n, F, S(stream)));
     }
+    if (tiled_steps(p)) {
+        const char* const labels[3] = {kLabel[0][2], kLabel[1][2], kLabel[2][2]};
+        return tile_passes(p, 1, V, F, nullptr, f32 ? p->f32n : nullptr, nullptr, dt, O, ncl,
+                           labels, stream);
+    }
     for (int c = 0; c < 3; ++c) {
         Timed t(p, kLabel[c][2], stream);
-        if (tiled_steps(p))
-            HIP_OK(run_tile_step(p->g, c, 1, p->at[c], V, F[c], nullptr,
-                                 f32 ? p->f32n[c] : nullptr, nullptr, dt, O[c], nullptr,
-                                 nullptr, nullptr, ncl, S(stream)));
-        else
-            HIP_OK(run_bdf1(p->g, c, V, F[c], dt, O[c], ncl, S(stream)));
+        HIP_OK(run_bdf1(p->g, c, V, F[c], dt, O[c], ncl, S(stream)));
     }
     return SLC_OK;
 }
@@ -597,13 +616,8 @@ int slc_bdf2_predict(slc_plan* p, const double* u, const double* v, const double
         TrajVel V{{p->us[0], p->us[1], p->us[2]}, {nullptr, nullptr, nullptr}};
         const long N = (long)p->nx * p->ny * p->nz;
         if (p->bdf2_fused) {
-            for (int c = 0; c < 3; ++c) {
-                Timed t(p, kBdf2Label[c], stream);
-                HIP_OK(run_tile_step(p->g, c, 5, p->at[c], V, Fn[c], Fm[c],
-                                     f32 ? p->f32n[c] : nullptr, f32 ? p->f32m[c] : nullptr, dt,
-                                     O[c], nullptr, nullptr, nullptr, ncl, S(stream)));
-            }
-            return SLC_OK;
+            return tile_passes(p, 5, V, Fn, Fm, f32 ? p->f32n : nullptr, f32 ? p->f32m : nullptr,
+                               dt, O, ncl, kBdf2Label, stream);
         }
         for (int c = 0; c < 3; ++c)
             for (int pass = 0; pass < 2; ++pass) {

@@ -678,10 +678,9 @@ __device__ inline double rhs_xy(const Grid& g, const double* __restrict__ F, int
     return g.nu * (d2x + d2y);
 }
 
-// blockIdx -> tile remap that keeps consecutive tiles on one XCD (blocks are
-// dispatched round-robin over the 8 XCDs; each XCD has its own L2).
-__device__ inline long xcd_block(long nblocks) {
-    long b = blockIdx.x;
+// Block b of nblocks -> tile, so that consecutive tiles stay on one XCD (blocks
+// are dispatched round-robin over the 8 XCDs; each XCD has its own L2).
+__device__ inline long xcd_block(long b, long nblocks) {
     const long nx = 8;
     long per = nblocks / nx;
     long rem = nblocks % nx;
@@ -690,6 +689,35 @@ __device__ inline long xcd_block(long nblocks) {
     long start = x * per + (x < rem ? x : rem);
     long count = per + (x < rem ? 1 : 0);
     return q < count ? start + q : b;
+}
+
+__device__ inline long xcd_block(long nblocks) { return xcd_block((long)blockIdx.x, nblocks); }
+
+// One launch over the units of three components (u's n[0] first): component
+// c and unit u of block b, or c = 3 for a block that only fills a component's
+// count up to a multiple of 8, so that every component starts on the first
+// XCD and xcd order holds inside it.
+__host__ __device__ inline unsigned pad8(unsigned n) { return (n + 7u) & ~7u; }
+
+struct Comp3 {
+    int c;
+    unsigned u;
+};
+
+__device__ inline Comp3 comp3_unit(unsigned b, const unsigned (&n)[3]) {
+    int c = 0;
+    if (b >= pad8(n[0])) {
+        b -= pad8(n[0]);
+        c = 1;
+        if (b >= pad8(n[1])) {
+            b -= pad8(n[1]);
+            c = 2;
+        }
+    }
+    const unsigned nc = c == 0 ? n[0] : c == 1 ? n[1] : n[2];
+    const unsigned x = b & 7u, q = b >> 3, per = nc >> 3, rem = nc & 7u;
+    if (q >= per + (x < rem ? 1u : 0u)) return Comp3{3, 0u};
+    return Comp3{c, x * per + min(x, rem) + q};
 }
 
 }  // namespace slc

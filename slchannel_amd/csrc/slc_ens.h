@@ -104,8 +104,14 @@ struct EnsLaunch {
     const unsigned* start;  // this kind's nmem + 1 prefix
     int nmem;
     unsigned total;
-    const int* umap;        // member of every unit (SL tile kinds only)
-    bool big;               // a member needs 64-bit addressing (big_index)
+};
+
+// SL tile units of the three components (n = 0: left out).
+struct EnsTiles {
+    const unsigned* start[3];
+    const int* umap[3];  // member of every unit
+    unsigned n[3];
+    bool big;            // a member needs 64-bit addressing (big_index)
 };
 
 // SL tile shapes the ensemble kernels are compiled for (autotuned):
@@ -125,16 +131,12 @@ hipError_t run_ens_bcp(const EnsLaunch& L, unsigned grid, hipStream_t s);
 hipError_t run_ens_bcu(const EnsLaunch& L, unsigned grid, hipStream_t s);
 hipError_t run_ens_ustar(const EnsLaunch& L, unsigned grid, hipStream_t s);
 // pass 0: far (BDF2 members), 1: near (BDF2) / bootstrap (BDF1)
-hipError_t run_ens_tile(const EnsLaunch& L, int comp, int pass, int order, int f32, int shape,
-                        unsigned grid, hipStream_t s);
-void run_ens_tile_d4(const EnsLaunch& L, int comp, int pass, int shape, unsigned grid,
-                     hipStream_t s);
-void run_ens_tile_d6(const EnsLaunch& L, int comp, int pass, int shape, unsigned grid,
-                     hipStream_t s);
-void run_ens_tile_f4(const EnsLaunch& L, int comp, int pass, int shape, unsigned grid,
-                     hipStream_t s);
-void run_ens_tile_f6(const EnsLaunch& L, int comp, int pass, int shape, unsigned grid,
-                     hipStream_t s);
+hipError_t run_ens_tile(const EnsMember* mem, const EnsTiles& t, int pass, int order, int f32,
+                        int shape, hipStream_t s);
+void run_ens_tile_d4(const EnsMember* mem, const EnsTiles& t, int pass, int shape, hipStream_t s);
+void run_ens_tile_d6(const EnsMember* mem, const EnsTiles& t, int pass, int shape, hipStream_t s);
+void run_ens_tile_f4(const EnsMember* mem, const EnsTiles& t, int pass, int shape, hipStream_t s);
+void run_ens_tile_f6(const EnsMember* mem, const EnsTiles& t, int pass, int shape, hipStream_t s);
 hipError_t run_ens_zsolve(const EnsLaunch& L, int comp, size_t lds_bytes, unsigned grid,
                           bool short_cols, hipStream_t s);
 hipError_t run_ens_div_planes(const EnsLaunch& L, unsigned grid, hipStream_t s);

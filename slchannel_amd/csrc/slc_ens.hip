@@ -426,16 +426,27 @@ int rebuild(slc_ens* e) {
     return SLC_OK;
 }
 
-EnsLaunch launch(const slc_ens* e, int kind, int comp = -1) {
+EnsLaunch launch(const slc_ens* e, int kind) {
     const int n = (int)e->members.size();
     EnsLaunch L;
     L.mem = e->d_mem;
     L.start = e->d_start + (size_t)kind * (n + 1);
     L.nmem = n;
     L.total = e->totals[kind];
-    L.umap = comp >= 0 ? e->d_umap[comp] : nullptr;
-    L.big = e->big;
     return L;
+}
+
+// SL tiles of the components in the bit set comps
+EnsTiles tiles(const slc_ens* e, int comps) {
+    const int n = (int)e->members.size();
+    EnsTiles t;
+    for (int c = 0; c < 3; ++c) {
+        t.start[c] = e->d_start + (size_t)(EK_TILE0 + c) * (n + 1);
+        t.umap[c] = e->d_umap[c];
+        t.n[c] = (comps >> c & 1) ? e->totals[EK_TILE0 + c] : 0u;
+    }
+    t.big = e->big;
+    return t;
 }
 
 unsigned pgrid(const slc_ens* e, int kind) {
@@ -461,17 +472,13 @@ int fft_all(slc_ens* e, bool forward) {
 int sl_passes(slc_ens* e) {
     const int f32 = e->storage == 32 ? 1 : 0;
     if (e->bdf2_fused) {
-        for (int c = 0; c < 3; ++c) {
-            EnsLaunch L = launch(e, EK_TILE0 + c, c);
-            HIP_OK(run_ens_tile(L, c, 2, e->order, f32, e->tile_shape, L.total, e->es));
-        }
+        HIP_OK(run_ens_tile(e->d_mem, tiles(e, 7), 2, e->order, f32, e->tile_shape, e->es));
         return SLC_OK;
     }
-    for (int c = 0; c < 3; ++c)
-        for (int pass = 0; pass < 2; ++pass) {
-            EnsLaunch L = launch(e, EK_TILE0 + c, c);
-            HIP_OK(run_ens_tile(L, c, pass, e->order, f32, e->tile_shape, L.total, e->es));
-        }
+    for (int c = 0; c < 3; ++c)  // the near feet's buffer serves one component at a time
+        for (int pass = 0; pass < 2; ++pass)
+            HIP_OK(run_ens_tile(e->d_mem, tiles(e, 1 << c), pass, e->order, f32, e->tile_shape,
+                                e->es));
     return SLC_OK;
 }
 

@@ -109,15 +109,15 @@ hipError_t run_ens_ustar(const EnsLaunch& L, unsigned grid, hipStream_t s) {
 // slc_ens_tile_{d4,d6,f4,f6}.hip so they compile in parallel)
 // ---------------------------------------------------------------------------
 
-hipError_t run_ens_tile(const EnsLaunch& L, int comp, int pass, int order, int f32, int shape,
-                        unsigned grid, hipStream_t s) {
-    if (L.total == 0) return hipSuccess;
+hipError_t run_ens_tile(const EnsMember* mem, const EnsTiles& t, int pass, int order, int f32,
+                        int shape, hipStream_t s) {
+    if (t.n[0] + t.n[1] + t.n[2] == 0) return hipSuccess;
     if (f32) {
-        if (order == 4) run_ens_tile_f4(L, comp, pass, shape, grid, s);
-        else run_ens_tile_f6(L, comp, pass, shape, grid, s);
+        if (order == 4) run_ens_tile_f4(mem, t, pass, shape, s);
+        else run_ens_tile_f6(mem, t, pass, shape, s);
     } else {
-        if (order == 4) run_ens_tile_d4(L, comp, pass, shape, grid, s);
-        else run_ens_tile_d6(L, comp, pass, shape, grid, s);
+        if (order == 4) run_ens_tile_d4(mem, t, pass, shape, s);
+        else run_ens_tile_d6(mem, t, pass, shape, s);
     }
     return hipGetLastError();
 }

@@ -10,22 +10,18 @@
 
 namespace slc {
 
-// One workgroup per tile: unit = xcd-ordered block index, its member from the
-// per-unit member map (the persistent chunk walk of the other batched kernels
-// keeps ~25 more registers live here and halves the occupancy).
-template <typename T, int C, int P, int PASS, int TI, int TJ, int TK, int kEnsLds, int WAVES,
-          bool BIG>
-__global__ __launch_bounds__(kSB) __attribute__((amdgpu_waves_per_eu(WAVES))) void
-ens_tile_kernel(const EnsMember* __restrict__ mem,
-                                                       const unsigned* __restrict__ start,
-                                                       const int* __restrict__ umap) {
+// One workgroup per tile, the three components (or one, n[c] = 0 for the
+// others) in one launch: its member from the per-unit member map (the
+// persistent chunk walk of the other batched kernels keeps ~25 more registers
+// live here and halves the occupancy).
+template <typename T, int C, int P, int PASS, int TI, int TJ, int TK, int kEnsLds, bool BIG,
+          typename LdsT>
+__device__ __forceinline__ void ens_tile_unit(const EnsMember* __restrict__ mem,
+                                              const unsigned* __restrict__ start,
+                                              const int* __restrict__ umap, unsigned uu, LdsT& L) {
     // one of the two tile bodies runs: the bootstrap's LDS is the fused pass's
-    constexpr int NPT = TI * TJ * TK;
-    constexpr int M0 = PASS == 0 ? MODE_FAR : PASS == 1 ? MODE_NEAR : MODE_BDF2;
-    __shared__ TileLds<T, M0, NPT, kEnsLds> L;
-    TileLds<T, MODE_BDF1, NPT, kEnsLds>& L1 =
-        reinterpret_cast<TileLds<T, MODE_BDF1, NPT, kEnsLds>&>(L);
-    const unsigned uu = (unsigned)xcd_block(gridDim.x);
+    TileLds<T, MODE_BDF1, TI * TJ * TK, kEnsLds>& L1 =
+        reinterpret_cast<TileLds<T, MODE_BDF1, TI * TJ * TK, kEnsLds>&>(L);
     // member and state are the same for the whole workgroup: broadcast them
     // so the member table is read with scalar loads and its pointers stay in
     // scalar registers
@@ -65,41 +61,49 @@ ens_tile_kernel(const EnsMember* __restrict__ mem,
     }
 }
 
-template <typename T, int C, int P, int PASS>
-inline void launch_tile_shape(const EnsLaunch& L, int shape, unsigned grid, hipStream_t s) {
-    if (L.big) {  // a member past the 32-bit offsets: one shape
-        hipLaunchKernelGGL((ens_tile_kernel<T, C, P, PASS, 4, 4, 16, 31104, 4, true>), dim3(grid),
-                           dim3(kSB), 0, s, L.mem, L.start, L.umap);
+template <typename T, int P, int PASS, int TI, int TJ, int TK, int kEnsLds, int WAVES, bool BIG>
+__global__ __launch_bounds__(kSB) __attribute__((amdgpu_waves_per_eu(WAVES))) void
+ens_tile_kernel(const EnsMember* __restrict__ mem, EnsTiles t) {
+    constexpr int M0 = PASS == 0 ? MODE_FAR : PASS == 1 ? MODE_NEAR : MODE_BDF2;
+    __shared__ TileLds<T, M0, TI * TJ * TK, kEnsLds> L;
+    const Comp3 w = comp3_unit(blockIdx.x, t.n);
+    if (w.c == 0)
+        ens_tile_unit<T, 0, P, PASS, TI, TJ, TK, kEnsLds, BIG>(mem, t.start[0], t.umap[0], w.u, L);
+    else if (w.c == 1)
+        ens_tile_unit<T, 1, P, PASS, TI, TJ, TK, kEnsLds, BIG>(mem, t.start[1], t.umap[1], w.u, L);
+    else if (w.c == 2)
+        ens_tile_unit<T, 2, P, PASS, TI, TJ, TK, kEnsLds, BIG>(mem, t.start[2], t.umap[2], w.u, L);
+}
+
+template <typename T, int P, int PASS>
+inline void launch_tile_shape(const EnsMember* mem, const EnsTiles& t, int shape, hipStream_t s) {
+    const dim3 grid(pad8(t.n[0]) + pad8(t.n[1]) + pad8(t.n[2])), blk(kSB);
+    if (t.big) {  // a member past the 32-bit offsets: one shape
+        hipLaunchKernelGGL((ens_tile_kernel<T, P, PASS, 4, 4, 16, 31104, 4, true>), grid, blk, 0, s,
+                           mem, t);
         return;
     }
     switch (shape) {
         case 1:
-            hipLaunchKernelGGL((ens_tile_kernel<T, C, P, PASS, 4, 4, 32, 40960, 1, false>), dim3(grid),
-                               dim3(kSB), 0, s, L.mem, L.start, L.umap);
+            hipLaunchKernelGGL((ens_tile_kernel<T, P, PASS, 4, 4, 32, 40960, 1, false>), grid, blk,
+                               0, s, mem, t);
             break;
         case 2:
-            hipLaunchKernelGGL((ens_tile_kernel<T, C, P, PASS, 2, 8, 16, 31104, 4, false>), dim3(grid),
-                               dim3(kSB), 0, s, L.mem, L.start, L.umap);
+            hipLaunchKernelGGL((ens_tile_kernel<T, P, PASS, 2, 8, 16, 31104, 4, false>), grid, blk,
+                               0, s, mem, t);
             break;
         default:
-            hipLaunchKernelGGL((ens_tile_kernel<T, C, P, PASS, 4, 4, 16, 31104, 4, false>), dim3(grid),
-                               dim3(kSB), 0, s, L.mem, L.start, L.umap);
+            hipLaunchKernelGGL((ens_tile_kernel<T, P, PASS, 4, 4, 16, 31104, 4, false>), grid, blk,
+                               0, s, mem, t);
     }
 }
 
-template <typename T, int C, int P>
-inline void launch_tile_pass(const EnsLaunch& L, int pass, int shape, unsigned grid, hipStream_t s) {
-    if (pass == 0) launch_tile_shape<T, C, P, 0>(L, shape, grid, s);
-    else if (pass == 1) launch_tile_shape<T, C, P, 1>(L, shape, grid, s);
-    else launch_tile_shape<T, C, P, 2>(L, shape, grid, s);
-}
-
 template <typename T, int P>
-inline void launch_tile_comp(const EnsLaunch& L, int comp, int pass, int shape, unsigned grid,
+inline void launch_tile_pass(const EnsMember* mem, const EnsTiles& t, int pass, int shape,
                              hipStream_t s) {
-    if (comp == 0) launch_tile_pass<T, 0, P>(L, pass, shape, grid, s);
-    else if (comp == 1) launch_tile_pass<T, 1, P>(L, pass, shape, grid, s);
-    else launch_tile_pass<T, 2, P>(L, pass, shape, grid, s);
+    if (pass == 0) launch_tile_shape<T, P, 0>(mem, t, shape, s);
+    else if (pass == 1) launch_tile_shape<T, P, 1>(mem, t, shape, s);
+    else launch_tile_shape<T, P, 2>(mem, t, shape, s);
 }
 
 }  // namespace slc

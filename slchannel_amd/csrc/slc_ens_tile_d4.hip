@@ -3,9 +3,9 @@
 
 namespace slc {
 
-void run_ens_tile_d4(const EnsLaunch& L, int comp, int pass, int shape, unsigned grid,
+void run_ens_tile_d4(const EnsMember* mem, const EnsTiles& t, int pass, int shape,
                      hipStream_t s) {
-    launch_tile_comp<double, 4>(L, comp, pass, shape, grid, s);
+    launch_tile_pass<double, 4>(mem, t, pass, shape, s);
 }
 
 }  // namespace slc

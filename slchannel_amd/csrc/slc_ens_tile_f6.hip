@@ -3,9 +3,9 @@
 
 namespace slc {
 
-void run_ens_tile_f6(const EnsLaunch& L, int comp, int pass, int shape, unsigned grid,
+void run_ens_tile_f6(const EnsMember* mem, const EnsTiles& t, int pass, int shape,
                      hipStream_t s) {
-    launch_tile_comp<float, 6>(L, comp, pass, shape, grid, s);
+    launch_tile_pass<float, 6>(mem, t, pass, shape, s);
 }
 
 }  // namespace slc

@@ -58,8 +58,9 @@ inline bool big_index(const Grid& g) {
     return pl * (g.nx + 2) >= 536870912.0 || pl >= 16777216.0 || g.nx + 2 >= (1 << 24);
 }
 
-// LDS-tiled step kernels (slc_step.hip); mode: 0 advect, 1 bdf1, 2 far,
-// 3 near, 4 gather (feet given), 5 far + near in one pass (no feet arrays)
+// LDS-tiled step kernels (slc_step.hip) of one component; mode: 0 advect,
+// 1 bdf1, 2 far, 3 near, 4 gather (feet given), 5 far + near in one pass (no
+// feet arrays)
 // Fn32 / Fm32: float copies of F / Fm to gather from (FP32 storage), or null.
 // defer (mode 4 only): (tiles of the component) unsigned of device scratch,
 // one flag per tile; when given, tiles whose box exceeds the LDS budget are
@@ -69,8 +70,16 @@ hipError_t run_tile_step(const Grid& g, int comp, int mode, const ArrivalTabs& A
                          const float* Fm32, double dt, double* out, double* fx, double* fy,
                          double* fz, unsigned long long* ncl, hipStream_t s,
                          unsigned* defer = nullptr);
-// Tiles of the gather at given feet for component comp (the defer flags' count).
-long gather_tiles(const Grid& g, int comp);
+// Modes 0, 1 and 5 for the three components in one launch (slc_step3.hip).
+hipError_t run_tile_step3(const Grid& g, int mode, const ArrivalTabs A[3], const TrajVel& V,
+                          const double* const F[3], const double* const Fm[3],
+                          const float* const Fn32[3], const float* const Fm32[3], double dt,
+                          double* const out[3], unsigned long long* ncl, hipStream_t s);
+// Tiles of the step kernels for component comp (the defer flags' count).
+long step_tiles(const Grid& g, int comp);
+// Tiles of a component up to which the three components share a launch: where
+// two launches and tails (15-20 us) outweigh the merged kernel's 2-3%.
+constexpr long kMergeTiles = 8192;
 hipError_t run_arrival_tabs(const Grid& g, int comp, double* xdx, double* ydy, int* cell,
                             hipStream_t s);
 hipError_t run_ustar(const Grid& g, double* const o[3], const double* const a[3],

@@ -2,29 +2,9 @@
 // channel per launch); the tile itself is sl_tile_body in slc_tile.h.
 #include <atomic>
 
-#include "slc_tile.h"
+#include "slc_step.h"
 
 namespace slc {
-
-// Tile of the step kernels: 4 x 4 x 16 arrival points, one per thread (measured
-// at 256^3 order 6 against 4x4x32, 2x8x16, 8x4x8 and 4x8x8 tiles).  Compile-time
-// overridable with -DSLC_TILE_TI=... for tile-shape sweeps.  The box budgets
-// fill a CU's 160 KB of LDS at the occupancy the registers allow: four
-// workgroups per CU (four waves per SIMD), less the workgroup's other LDS.
-#ifndef SLC_TILE_TI
-#define SLC_TILE_TI 4
-#define SLC_TILE_TJ 4
-#define SLC_TILE_TK 16
-#endif
-constexpr int kTI = SLC_TILE_TI, kTJ = SLC_TILE_TJ, kTK = SLC_TILE_TK;
-constexpr int kTileLds = 40576;
-constexpr int kTileLdsBdf2 = 31104;  // beside the near stencils' 9 KB
-constexpr int kTileWavesPerSimd = 4;
-// The gather at given feet and the near pass at order 4 fit seven waves per
-// SIMD (72 VGPRs) with a 21 KB budget (an order-4 box of a 4x4x16 tile at the
-// usual CFL takes 16-20 KB); at order 6 five or more spill.
-constexpr int kGatherWaves4 = 7;
-constexpr int kGatherLds4 = 21504;
 
 template <typename T, int C, int P, int MODE, int TI, int TJ, int TK, int LDS_BYTES, int WAVES,
           bool BIG>
@@ -335,9 +315,9 @@ static void launch_t(const Grid& g, int comp, int mode, const ArrivalTabs& A, co
     switch (mode) {
         case MODE_ADVECT: launch_c<T, MODE_ADVECT>(g, comp, A, V, a, s); break;
         case MODE_BDF1: launch_c<T, MODE_BDF1>(g, comp, A, V, a, s); break;
+        case MODE_BDF2: launch_c<T, MODE_BDF2>(g, comp, A, V, a, s); break;
         case MODE_FAR: launch_c<T, MODE_FAR>(g, comp, A, V, a, s); break;
         case MODE_NEAR: launch_c<T, MODE_NEAR>(g, comp, A, V, a, s); break;
-        case MODE_BDF2: launch_c<T, MODE_BDF2>(g, comp, A, V, a, s); break;
         default: launch_c<T, MODE_GATHER>(g, comp, A, V, a, s); break;
     }
 }
@@ -357,7 +337,7 @@ hipError_t run_tile_step(const Grid& g, int comp, int mode, const ArrivalTabs& A
     return hipGetLastError();
 }
 
-long gather_tiles(const Grid& g, int comp) {
+long step_tiles(const Grid& g, int comp) {
     const long nzi = (comp == 2) ? g.nz - 1 : g.nz;
     return ((long)(g.nx + kTI - 1) / kTI) *
            ((g.ny + kTJ - 1) / kTJ) * ((nzi + kTK - 1) / kTK);
