@@ -182,6 +182,15 @@ int slc_pressure_combine(slc_plan* plan, double* out, double a, const double* x,
 int slc_project_step(slc_plan* plan, double* u, double* v, double* w, double rhs_scale,
                      double dt_proj, double* p, void* stream);
 
+/* The implicit and projection part of one step: the theta-method z-solves of
+ * u, v and w over dt_z (slc_zsolve of each) and slc_project_step with
+ * (rhs_scale, dt_proj, p).  The fields come with no ghosts filled and leave
+ * with all of them filled: the results are those of slc_apply_bc before
+ * (where theta < 1) and after the z-solves.  Needs nz >= 3.
+ * Replaces solver.py:766-801 + 809 and 949-998 + 1015. */
+int slc_implicit_project(slc_plan* plan, double* u, double* v, double* w, double dt_z,
+                         double theta, double rhs_scale, double dt_proj, double* p, void* stream);
+
 /* Bulk velocity sum(u dx dy dz_f)/V of u's interior into out[3] (out: 4
  * device doubles of scratch).  Replaces compute_bulk_velocity
  * (slchannel/utils.py:147-163). */
@@ -260,8 +269,8 @@ int slc_bulk_force(slc_plan* plan, double* u, double* v, double* w, double U_bul
 /* slc_bulk_force without the plan's workspace: no counterpart in the
  * reference.  For callers that cannot allocate device memory (code under
  * hipGraph capture, tight serving loops, harnesses that forbid hipMalloc):
- * the call allocates nothing.  Its partial sums (at most 2048 doubles, the
- * most any grid needs) live in a static device array of the library, one per
+ * the call allocates nothing.  Its partial sums (at most 4096 doubles and a
+ * counter, the most any grid needs) live in a static device array of the library, one per
  * GPU, held until the process ends.  Calls that overlap on one GPU share that
  * array and race: order them on one stream.  Same kernels, same results as
  * slc_bulk_force. */

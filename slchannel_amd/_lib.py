@@ -18,7 +18,7 @@ EXPORTS = (
     "slc_version", "slc_last_error", "slc_plan_create", "slc_plan_destroy",
     "slc_plan_workspace_bytes", "slc_apply_bc", "slc_departure", "slc_gather",
     "slc_stencil", "slc_locate_z", "slc_advect", "slc_bdf1_predict", "slc_bdf2_predict",
-    "slc_zsolve", "slc_divergence", "slc_poisson", "slc_project", "slc_project_step",
+    "slc_zsolve", "slc_divergence", "slc_poisson", "slc_project", "slc_project_step", "slc_implicit_project",
     "slc_pressure_combine",
     "slc_bulk_velocity", "slc_bulk_force", "slc_bulk_force_noalloc", "slc_diagnostics",
     "slc_init_solenoidal", "slc_init_solenoidal_work", "slc_interp_trilinear",
@@ -85,6 +85,7 @@ def load():
         "slc_project": ([vp, vp, vp, vp, vp, d, vp], i),
         "slc_pressure_combine": ([vp, vp, d, vp, d, vp, vp], i),
         "slc_project_step": ([vp, vp, vp, vp, d, d, vp, vp], i),
+        "slc_implicit_project": ([vp, vp, vp, vp, d, d, d, d, vp, vp], i),
         "slc_bulk_velocity": ([vp, vp, vp, vp], i),
         "slc_bulk_force": ([vp, vp, vp, vp, d, d, vp, vp], i),
         "slc_bulk_force_noalloc": ([vp, vp, vp, vp, d, d, vp, vp], i),

@@ -328,8 +328,7 @@ int slc::plan_create(const slc_grid_desc* d, int device, bool spectral, slc_plan
             }
         }
     }
-    p->max_partials = bulk_partials_needed(g);
-    if ((rc = dev_alloc(p, sizeof(double) * p->max_partials, &ptr))) { slc_plan_destroy(p); return rc; }
+    if ((rc = dev_alloc(p, sizeof(double) * bulk_scratch(bulk_partials_needed(g)), &ptr))) { slc_plan_destroy(p); return rc; }
     p->partials = (double*)ptr;
     if ((rc = dev_alloc(p, sizeof(double) * 5 * kDiagMaxBlocks, &ptr))) { slc_plan_destroy(p); return rc; }
     p->diag_part = (double*)ptr;
@@ -381,7 +380,7 @@ constexpr int kNoAllocPartials = 2048;  // the most bulk_partials_needed() retur
 constexpr int kNoAllocDevices = 64;
 }  // namespace
 
-static __device__ __align__(256) double scratch[kNoAllocPartials];
+static __device__ __align__(256) double scratch[bulk_scratch(kNoAllocPartials)];
 
 namespace {
 std::mutex g_scratch_mu;
@@ -638,6 +637,16 @@ int slc_bdf2_predict(slc_plan* p, const double* u, const double* v, const double
     return SLC_OK;
 }
 
+// The factorisation of a component's z-solve depends only on (dt, theta):
+// whether the plan's is for others, which it then counts as rebuilt.
+static bool zrefactor(slc_plan* p, int comp, double dt, double theta) {
+    const bool same = p->zvalid[comp] && p->zkey[comp][0] == dt && p->zkey[comp][1] == theta;
+    p->zvalid[comp] = true;
+    p->zkey[comp][0] = dt;
+    p->zkey[comp][1] = theta;
+    return !same;
+}
+
 int slc_zsolve(slc_plan* p, int comp, double* field, double dt, double theta, void* stream) {
     if (int rc = check_plan(p)) return rc;
     if (comp < 0 || comp > 2) return fail(SLC_EINVAL, "comp must be 0, 1 or 2");
@@ -645,11 +654,7 @@ int slc_zsolve(slc_plan* p, int comp, double* field, double dt, double theta, vo
     if (!(theta > 0.0 && theta <= 1.0)) return fail(SLC_EINVAL, "theta must be in (0, 1]");
     if (comp == 2 && p->nz < 3) return fail(SLC_EINVAL, "w z-solve needs nz >= 3");
     DeviceGuard dg(p->device);
-    // the factorisation depends only on (dt, theta): rebuilt when they change
-    bool refactor = !(p->zvalid[comp] && p->zkey[comp][0] == dt && p->zkey[comp][1] == theta);
-    p->zvalid[comp] = true;
-    p->zkey[comp][0] = dt;
-    p->zkey[comp][1] = theta;
+    const bool refactor = zrefactor(p, comp, dt, theta);
     Timed t(p, kZLabel[comp], stream);
     HIP_OK(run_zsolve(p->g, comp, field, dt, theta, p->d_dzc, p->d_dzf,
                       p->ztab + (size_t)comp * 3 * (p->nz + 2), refactor, S(stream)));
@@ -674,7 +679,6 @@ int slc_poisson(slc_plan* p, const double* div, double rhs_scale, double* pr, vo
     const double inv_n = 1.0 / ((double)p->nx * (double)p->ny);
     HIP_OK(run_project_planes(p->g, nullptr, nullptr, nullptr, p->planes, inv_n, 0.0, p->d_dzc,
                               pr, S(stream)));
-    HIP_OK(run_bc_p(p->g, pr, S(stream)));
     return SLC_OK;
 }
 
@@ -697,34 +701,67 @@ int slc_pressure_combine(slc_plan* p, double* out, double a, const double* x, do
     return SLC_OK;
 }
 
+// div/rhs_scale -> rocFFT -> per-mode solve -> rocFFT -> gradient update and
+// ghosts.  wrap: the fields' ghosts are not filled yet.
+static int projection(slc_plan* p, double* u, double* v, double* w, double rhs_scale,
+                      double dt_proj, double* pr, bool wrap, void* stream) {
+    {
+        Timed t(p, "divergence_planes", stream);
+        HIP_OK(run_div_planes(p->g, u, v, w, p->d_dzf, rhs_scale, p->planes, wrap, S(stream)));
+    }
+    if (int rc = poisson_planes(p, stream)) return rc;
+    const double inv_n = 1.0 / ((double)p->nx * (double)p->ny);
+    Timed t(p, "project_planes", stream);
+    HIP_OK(run_project_planes(p->g, u, v, w, p->planes, inv_n, dt_proj, p->d_dzc, pr,
+                              S(stream)));
+    return SLC_OK;
+}
+
 int slc_project_step(slc_plan* p, double* u, double* v, double* w, double rhs_scale,
                      double dt_proj, double* pr, void* stream) {
     if (int rc = check_plan(p)) return rc;
     if (!u || !v || !w) return fail(SLC_EINVAL, "null array");
     DeviceGuard dg(p->device);
-    {
-        Timed t(p, "divergence_planes", stream);
-        HIP_OK(run_div_planes(p->g, u, v, w, p->d_dzf, rhs_scale, p->planes, S(stream)));
+    return projection(p, u, v, w, rhs_scale, dt_proj, pr, false, stream);
+}
+
+int slc_implicit_project(slc_plan* p, double* u, double* v, double* w, double dt_z, double theta,
+                         double rhs_scale, double dt_proj, double* pr, void* stream) {
+    if (int rc = check_plan(p)) return rc;
+    if (!u || !v || !w) return fail(SLC_EINVAL, "null array");
+    if (!(theta > 0.0 && theta <= 1.0)) return fail(SLC_EINVAL, "theta must be in (0, 1]");
+    if (p->nz < 3) return fail(SLC_EINVAL, "w z-solve needs nz >= 3");
+    DeviceGuard dg(p->device);
+    // ghosts enter the z-solves only in the explicit part of a theta < 1
+    // right-hand side
+    if (theta != 1.0) {
+        Timed t(p, "ghost_fill_uvw", stream);
+        HIP_OK(run_bc(p->g, u, v, w, S(stream)));
     }
-    if (int rc = poisson_planes(p, stream)) return rc;
-    const double inv_n = 1.0 / ((double)p->nx * (double)p->ny);
-    {
-        Timed t(p, "project_planes", stream);
-        HIP_OK(run_project_planes(p->g, u, v, w, p->planes, inv_n, dt_proj, p->d_dzc, pr,
-                                  S(stream)));
+    double* const F[3] = {u, v, w};
+    double* tab[3];
+    bool refactor[3];
+    for (int c = 0; c < 3; ++c) {
+        tab[c] = p->ztab + (size_t)c * 3 * (p->nz + 2);
+        refactor[c] = zrefactor(p, c, dt_z, theta);
     }
-    Timed t(p, "ghost_fill_p_uvw", stream);
-    if (pr) HIP_OK(run_bc_p(p->g, pr, S(stream)));
-    HIP_OK(run_bc(p->g, u, v, w, S(stream)));
-    return SLC_OK;
+    if (p->prof) {
+        for (int c = 0; c < 3; ++c) {
+            Timed t(p, kZLabel[c], stream);
+            HIP_OK(run_zsolve(p->g, c, F[c], dt_z, theta, p->d_dzc, p->d_dzf, tab[c], refactor[c],
+                              S(stream)));
+        }
+    } else {
+        HIP_OK(run_zsolve3(p->g, F, dt_z, theta, p->d_dzc, p->d_dzf, tab, refactor, S(stream)));
+    }
+    return projection(p, u, v, w, rhs_scale, dt_proj, pr, true, stream);
 }
 
 int slc_bulk_velocity(slc_plan* p, const double* u, double* out, void* stream) {
     if (int rc = check_plan(p)) return rc;
     if (!u || !out) return fail(SLC_EINVAL, "null array");
     DeviceGuard dg(p->device);
-    HIP_OK(run_bulk_velocity(p->g, u, p->d_cv, p->total_volume, p->partials, p->max_partials, out,
-                             S(stream)));
+    HIP_OK(run_bulk_velocity(p->g, u, p->d_cv, p->total_volume, p->partials, out, S(stream)));
     return SLC_OK;
 }
 
@@ -733,10 +770,11 @@ int slc_bulk_force(slc_plan* p, double* u, double* v, double* w, double U_bulk, 
     if (int rc = check_plan(p)) return rc;
     if (!u || !out) return fail(SLC_EINVAL, "null array");
     if (!(dt != 0.0)) return fail(SLC_EINVAL, "dt must be non-zero");
+    (void)v;
+    (void)w;
     DeviceGuard dg(p->device);
     Timed t(p, "bulk_force", stream);
-    HIP_OK(run_bulk(p->g, u, v, w, p->d_cv, p->total_volume, U_bulk, dt, 1, p->partials,
-                    p->max_partials, out, S(stream)));
+    HIP_OK(run_bulk(p->g, u, p->d_cv, p->total_volume, U_bulk, dt, p->partials, out, S(stream)));
     return SLC_OK;
 }
 
@@ -745,6 +783,8 @@ int slc_bulk_force_noalloc(slc_plan* p, double* u, double* v, double* w, double 
     if (int rc = check_plan(p)) return rc;
     if (!u || !out) return fail(SLC_EINVAL, "null array");
     if (!(dt != 0.0)) return fail(SLC_EINVAL, "dt must be non-zero");
+    (void)v;
+    (void)w;
     const int np = bulk_partials_needed(p->g);
     if (np > kNoAllocPartials)
         return fail(SLC_EINVAL, "%d bulk partial sums exceed the static scratch of %d", np,
@@ -752,9 +792,8 @@ int slc_bulk_force_noalloc(slc_plan* p, double* u, double* v, double* w, double 
     DeviceGuard dg(p->device);
     double* partials = nullptr;
     if (int rc = scratch_on(p->device, &partials)) return rc;
-    // every partial is written before it is read: nothing to clear
-    HIP_OK(run_bulk(p->g, u, v, w, p->d_cv, p->total_volume, U_bulk, dt, 1, partials,
-                    kNoAllocPartials, out, S(stream)));
+    // the first pass writes all that the second reads: nothing to clear
+    HIP_OK(run_bulk(p->g, u, p->d_cv, p->total_volume, U_bulk, dt, partials, out, S(stream)));
     return SLC_OK;
 }
 

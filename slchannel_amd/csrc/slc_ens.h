@@ -77,14 +77,12 @@ struct EnsMember {
     int npart;
     int zcols[3];  // columns per z-solve work unit
     int zch[3];    // register z-solve unknowns per lane (0: LDS column path)
-    long nghost[4];  // ghost entries of u, v, w, p
+    long nghost[3];  // ghost entries of u, v, w
 };
 
 // Work-unit kinds; start[kind * (nmem + 1) + m] is the first unit of member m.
 enum EnsKind {
     EK_BC3 = 0,  // ghost fill of u, v, w (256-entry blocks, u then v then w)
-    EK_BCP,      // ghost fill of p
-    EK_BCU,      // ghost fill of u only
     EK_ELEM,     // 256-element blocks over the largest velocity component
     EK_TILE0,    // SL tiles of u, v, w
     EK_TILE1,
@@ -95,7 +93,6 @@ enum EnsKind {
     EK_PLANE,    // 32 x 32 transpose tiles (divergence, projection)
     EK_THOMAS,   // 256-mode Poisson Thomas blocks
     EK_BULK,     // bulk-reduction partials
-    EK_ONE,      // one unit per member
     EK_COUNT
 };
 
@@ -126,9 +123,7 @@ __host__ __device__ inline void ens_tile_shape(int s, int& ti, int& tj, int& tk)
 
 // launchers: `grid` is the persistent grid size (workgroups); the SL tile
 // launcher runs one workgroup per unit and ignores it
-hipError_t run_ens_bc3(const EnsLaunch& L, int role, unsigned grid, hipStream_t s);
-hipError_t run_ens_bcp(const EnsLaunch& L, unsigned grid, hipStream_t s);
-hipError_t run_ens_bcu(const EnsLaunch& L, unsigned grid, hipStream_t s);
+hipError_t run_ens_bc3(const EnsLaunch& L, unsigned grid, hipStream_t s);
 hipError_t run_ens_ustar(const EnsLaunch& L, unsigned grid, hipStream_t s);
 // pass 0: far (BDF2 members), 1: near (BDF2) / bootstrap (BDF1)
 hipError_t run_ens_tile(const EnsMember* mem, const EnsTiles& t, int pass, int order, int f32,
@@ -142,9 +137,8 @@ hipError_t run_ens_zsolve(const EnsLaunch& L, int comp, size_t lds_bytes, unsign
 hipError_t run_ens_div_planes(const EnsLaunch& L, unsigned grid, hipStream_t s);
 hipError_t run_ens_thomas(const EnsLaunch& L, unsigned grid, hipStream_t s);
 hipError_t run_ens_project(const EnsLaunch& L, unsigned grid, hipStream_t s);
-hipError_t run_ens_bulk_partial(const EnsLaunch& L, int shift, unsigned grid, hipStream_t s);
-hipError_t run_ens_bulk_final(const EnsLaunch& L, int mode, unsigned grid, hipStream_t s);
-hipError_t run_ens_advance(const EnsLaunch& L, hipStream_t s);
+hipError_t run_ens_bulk_before(const EnsLaunch& L, unsigned grid, hipStream_t s);
+hipError_t run_ens_bulk_shift(const EnsLaunch& L, unsigned grid, hipStream_t s);
 hipError_t run_ens_clear_ncl(const EnsLaunch& L, hipStream_t s);
 // *p = v, stream-ordered (no host memory involved)
 hipError_t run_ens_set_int(int* p, int v, hipStream_t s);

@@ -350,18 +350,16 @@ int rebuild(slc_ens* e) {
         M.U_bulk = m->U_bulk;
         M.total_volume = pl->total_volume;
         M.inv_n = 1.0 / ((double)m->nx * (double)m->ny);
-        M.npart = pl->max_partials;
+        M.npart = bulk_partials_needed(pl->g);
         for (int k = 0; k < 3; ++k) {
             M.zch[k] = zsolve_scan_ch(k, m->nz);
             M.zcols[k] = M.zch[k] > 0 ? kZScanCols * zscan_k(M.zch[k]) : zsolve_cols(k, m->nz);
             e->zs_short[k] = e->zs_short[k] && (M.zch[k] == 1 || M.zch[k] == 2);
         }
-        for (int k = 0; k < 4; ++k) M.nghost[k] = ghost_count(k, m->nx, m->ny, m->nz);
+        for (int k = 0; k < 3; ++k) M.nghost[k] = ghost_count(k, m->nx, m->ny, m->nz);
         // work units
         unsigned units[EK_COUNT];
         units[EK_BC3] = ublocks(M.nghost[0]) + ublocks(M.nghost[1]) + ublocks(M.nghost[2]);
-        units[EK_BCP] = ublocks(M.nghost[3]);
-        units[EK_BCU] = ublocks(M.nghost[0]);
         long nmax = 0;
         for (int k = 0; k < 3; ++k) nmax = std::max(nmax, field_elems(k, m->nx, m->ny, m->nz));
         units[EK_ELEM] = ublocks(nmax);
@@ -379,7 +377,6 @@ int rebuild(slc_ens* e) {
                                             spike_modes(m->nz))
                                : ublocks((long)m->nx * nky);
         units[EK_BULK] = (unsigned)M.npart;
-        units[EK_ONE] = 1;
         for (int k = 0; k < EK_COUNT; ++k)
             e->h_start[(size_t)k * (n + 1) + i + 1] = e->h_start[(size_t)k * (n + 1) + i] + units[k];
         for (int k = 0; k < 3; ++k) umap[k].insert(umap[k].end(), units[EK_TILE0 + k], i);
@@ -485,27 +482,21 @@ int sl_passes(slc_ens* e) {
 // the whole step, enqueued on e->es
 int enqueue_step(slc_ens* e) {
     hipStream_t s = e->es;
-    HIP_OK(run_ens_bc3(launch(e, EK_BC3), 0, pgrid(e, EK_BC3), s));
+    HIP_OK(run_ens_bc3(launch(e, EK_BC3), pgrid(e, EK_BC3), s));
     HIP_OK(run_ens_ustar(launch(e, EK_ELEM), pgrid(e, EK_ELEM), s));
     if (int rc = sl_passes(e)) return rc;
-    HIP_OK(run_ens_bc3(launch(e, EK_BC3), 1, pgrid(e, EK_BC3), s));
+    // nothing up to the divergence reads the predictor's ghosts; the
+    // projection and the bulk shift write them with the interior
     for (int c = 0; c < 3; ++c)
         HIP_OK(run_ens_zsolve(launch(e, EK_ZS0 + c), c, e->zs_lds[c], pgrid(e, EK_ZS0 + c),
                               e->zs_short[c], s));
-    HIP_OK(run_ens_bc3(launch(e, EK_BC3), 1, pgrid(e, EK_BC3), s));
     HIP_OK(run_ens_div_planes(launch(e, EK_PLANE), pgrid(e, EK_PLANE), s));
     if (int rc = fft_all(e, true)) return rc;
     HIP_OK(run_ens_thomas(launch(e, EK_THOMAS), pgrid(e, EK_THOMAS), s));
     if (int rc = fft_all(e, false)) return rc;
     HIP_OK(run_ens_project(launch(e, EK_PLANE), pgrid(e, EK_PLANE), s));
-    HIP_OK(run_ens_bcp(launch(e, EK_BCP), pgrid(e, EK_BCP), s));
-    HIP_OK(run_ens_bc3(launch(e, EK_BC3), 1, pgrid(e, EK_BC3), s));
-    HIP_OK(run_ens_bulk_partial(launch(e, EK_BULK), 0, pgrid(e, EK_BULK), s));
-    HIP_OK(run_ens_bulk_final(launch(e, EK_ONE), 0, pgrid(e, EK_ONE), s));
-    HIP_OK(run_ens_bulk_partial(launch(e, EK_BULK), 1, pgrid(e, EK_BULK), s));
-    HIP_OK(run_ens_bulk_final(launch(e, EK_ONE), 1, pgrid(e, EK_ONE), s));
-    HIP_OK(run_ens_bcu(launch(e, EK_BCU), pgrid(e, EK_BCU), s));
-    HIP_OK(run_ens_advance(launch(e, EK_ONE), s));
+    HIP_OK(run_ens_bulk_before(launch(e, EK_BULK), pgrid(e, EK_BULK), s));
+    HIP_OK(run_ens_bulk_shift(launch(e, EK_BULK), pgrid(e, EK_BULK), s));
     return SLC_OK;
 }
 
@@ -534,7 +525,7 @@ int64_t member_bytes(int nx, int ny, int nz, int order, int storage) {
     // tables: z (2 P + 4 columns of nz+2), arrival, Poisson, z-solve factors,
     // bulk and diagnostics partials
     b += 8L * (nz + 2) * (2 * order + 8 + 19) + 8L * (nx + ny) * 4 + 4L * 3 * nz +
-         8L * bulk_blocks(nx, ny, nz) + 8L * 5 * kDiagMaxBlocks + 4096;
+         8L * bulk_scratch(bulk_blocks(nx, ny, nz)) + 8L * 5 * kDiagMaxBlocks + 4096;
     return b;
 }
 
@@ -973,7 +964,7 @@ static int autotune_sweeps(slc_ens* e, int reps, hipEvent_t t0, hipEvent_t t1,
         e->grid_per_cu = grids[gi];
         auto substeps = [&]() -> int {
             hipStream_t s = e->es;
-            HIP_OK(run_ens_bc3(launch(e, EK_BC3), 0, pgrid(e, EK_BC3), s));
+            HIP_OK(run_ens_bc3(launch(e, EK_BC3), pgrid(e, EK_BC3), s));
             HIP_OK(run_ens_ustar(launch(e, EK_ELEM), pgrid(e, EK_ELEM), s));
             for (int c = 0; c < 3; ++c)
                 HIP_OK(run_ens_zsolve(launch(e, EK_ZS0 + c), c, e->zs_lds[c],
@@ -1001,7 +992,7 @@ static int autotune_sweeps(slc_ens* e, int reps, hipEvent_t t0, hipEvent_t t1,
     }
     e->grid_per_cu = best_grid;
     // the timed passes accumulated clamp counts: clear them
-    HIP_OK(run_ens_clear_ncl(launch(e, EK_ONE), e->es));
+    HIP_OK(run_ens_clear_ncl(launch(e, EK_BULK), e->es));
     return SLC_OK;
 }
 

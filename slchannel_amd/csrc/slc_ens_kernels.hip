@@ -13,14 +13,13 @@ namespace slc {
 
 
 // ---------------------------------------------------------------------------
-// ghost fills
+// ghost fill of V^n
 // ---------------------------------------------------------------------------
 
-__global__ __launch_bounds__(256) void ens_bc3_kernel(ENS_PARAMS, int role) {
+__global__ __launch_bounds__(256) void ens_bc3_kernel(ENS_PARAMS) {
     ens_for(start, nmem, total, [&](int m, unsigned u) {
         const EnsMember& M = mem[m];
-        const int st = *M.state;
-        const int set = role == 0 ? ens_a(st) : ens_c(st);
+        const int set = ens_a(*M.state);
         const unsigned b0 = ublocks(M.nghost[0]), b1 = ublocks(M.nghost[1]);
         int c;
         unsigned lb;
@@ -31,36 +30,9 @@ __global__ __launch_bounds__(256) void ens_bc3_kernel(ENS_PARAMS, int role) {
     });
 }
 
-hipError_t run_ens_bc3(const EnsLaunch& L, int role, unsigned grid, hipStream_t s) {
+hipError_t run_ens_bc3(const EnsLaunch& L, unsigned grid, hipStream_t s) {
     if (L.total == 0) return hipSuccess;
-    hipLaunchKernelGGL(ens_bc3_kernel, dim3(grid), dim3(256), 0, s, ENS_ARGS(L), role);
-    return hipGetLastError();
-}
-
-__global__ __launch_bounds__(256) void ens_bcp_kernel(ENS_PARAMS) {
-    ens_for(start, nmem, total, [&](int m, unsigned u) {
-        const EnsMember& M = mem[m];
-        bc_body(M.g, M.p, 3, (long)u * 256 + threadIdx.x);
-    });
-}
-
-hipError_t run_ens_bcp(const EnsLaunch& L, unsigned grid, hipStream_t s) {
-    if (L.total == 0) return hipSuccess;
-    hipLaunchKernelGGL(ens_bcp_kernel, dim3(grid), dim3(256), 0, s, ENS_ARGS(L));
-    return hipGetLastError();
-}
-
-// u of the predictor set only (after the bulk shift, solver.py:720)
-__global__ __launch_bounds__(256) void ens_bcu_kernel(ENS_PARAMS) {
-    ens_for(start, nmem, total, [&](int m, unsigned u) {
-        const EnsMember& M = mem[m];
-        bc_body(M.g, M.fld[ens_c(*M.state)][0], 0, (long)u * 256 + threadIdx.x);
-    });
-}
-
-hipError_t run_ens_bcu(const EnsLaunch& L, unsigned grid, hipStream_t s) {
-    if (L.total == 0) return hipSuccess;
-    hipLaunchKernelGGL(ens_bcu_kernel, dim3(grid), dim3(256), 0, s, ENS_ARGS(L));
+    hipLaunchKernelGGL(ens_bc3_kernel, dim3(grid), dim3(256), 0, s, ENS_ARGS(L));
     return hipGetLastError();
 }
 
@@ -192,7 +164,7 @@ hipError_t run_ens_zsolve(const EnsLaunch& L, int comp, size_t lds_bytes, unsign
 }
 
 // ---------------------------------------------------------------------------
-// projection: divergence -> planes, Thomas, gradient update
+// projection: divergence -> planes, Thomas, gradient update with the ghosts
 // ---------------------------------------------------------------------------
 
 __device__ inline double ens_dt_eff(const EnsMember& M, int st) {
@@ -207,8 +179,8 @@ __global__ __launch_bounds__(256) void ens_div_planes_kernel(ENS_PARAMS) {
         const int c = ens_c(st);
         int i, j0, k0;
         plane_tile(M.g, u, i, j0, k0);
-        div_planes_body(M.g, M.fld[c][0], M.fld[c][1], M.fld[c][2], M.dzf, ens_dt_eff(M, st),
-                        M.planes, i, j0, k0, tile);
+        div_planes_body<true>(M.g, M.fld[c][0], M.fld[c][1], M.fld[c][2], M.dzf, ens_dt_eff(M, st),
+                              M.planes, i, j0, k0, tile);
     });
 }
 
@@ -263,57 +235,47 @@ hipError_t run_ens_project(const EnsLaunch& L, unsigned grid, hipStream_t s) {
 // bulk constraint and the end-of-step state advance
 // ---------------------------------------------------------------------------
 
-__global__ __launch_bounds__(kRedBlock) void ens_bulk_partial_kernel(ENS_PARAMS, int shift) {
+__global__ __launch_bounds__(kRedBlock) void ens_bulk_before_kernel(ENS_PARAMS) {
     __shared__ double red[kRedBlock];
     ens_for(start, nmem, total, [&](int m, unsigned u) {
         const EnsMember& M = mem[m];
-        const int st = *M.state;
-        bulk_partial_body(M.g, M.fld[ens_c(st)][0], M.cv, shift ? M.scal[0] : 0.0, shift,
-                          M.partials, u, M.npart, red);
+        bulk_before_body(M.g, M.fld[ens_c(*M.state)][0], M.cv, M.partials, (int)u, M.npart, red);
     });
 }
 
-hipError_t run_ens_bulk_partial(const EnsLaunch& L, int shift, unsigned grid, hipStream_t s) {
+hipError_t run_ens_bulk_before(const EnsLaunch& L, unsigned grid, hipStream_t s) {
     if (L.total == 0) return hipSuccess;
-    hipLaunchKernelGGL(ens_bulk_partial_kernel, dim3(grid), dim3(kRedBlock), 0, s, ENS_ARGS(L), shift);
+    hipLaunchKernelGGL(ens_bulk_before_kernel, dim3(grid), dim3(kRedBlock), 0, s, ENS_ARGS(L));
     return hipGetLastError();
 }
 
-__global__ __launch_bounds__(kRedBlock) void ens_bulk_final_kernel(ENS_PARAMS, int mode) {
+// The member's last block also publishes the step's statistics, clears the
+// clamp counter and rotates the buffer sets (its other blocks have read the
+// state by then).
+__global__ __launch_bounds__(kRedBlock) void ens_bulk_shift_kernel(ENS_PARAMS) {
     __shared__ double red[kRedBlock];
-    ens_for(start, nmem, total, [&](int m, unsigned) {
+    __shared__ bool last;
+    ens_for(start, nmem, total, [&](int m, unsigned u) {
         const EnsMember& M = mem[m];
-        bulk_finalize_body(M.partials, M.npart, M.total_volume, M.U_bulk, M.dt, mode, M.scal,
-                           red);
+        const int st = *M.state;
+        const bool done =
+            bulk_shift_body(M.g, M.fld[ens_c(st)][0], M.cv, M.partials, (int)u, M.npart,
+                            M.total_volume, M.U_bulk, M.dt, M.scal, red, &last);
+        if (!done || threadIdx.x != 0) return;
+        double* S = M.stats;
+        S[ES_UBULK] = M.scal[2];
+        S[ES_FORCING] = M.scal[1];
+        S[ES_NCLAMP] = (double)*M.ncl;
+        S[ES_STEPS] = S[ES_STEPS] + 1.0;
+        S[ES_UBULK_PRE] = M.scal[3];
+        *M.ncl = 0ull;
+        *M.state = ens_next(st);
     });
 }
 
-hipError_t run_ens_bulk_final(const EnsLaunch& L, int mode, unsigned grid, hipStream_t s) {
+hipError_t run_ens_bulk_shift(const EnsLaunch& L, unsigned grid, hipStream_t s) {
     if (L.total == 0) return hipSuccess;
-    hipLaunchKernelGGL(ens_bulk_final_kernel, dim3(grid), dim3(kRedBlock), 0, s, ENS_ARGS(L), mode);
-    return hipGetLastError();
-}
-
-// one thread per member: publish the step's statistics, clear the clamp
-// counter, rotate the buffer sets
-__global__ void ens_advance_kernel(const EnsMember* __restrict__ mem, int nmem) {
-    const int m = blockIdx.x * blockDim.x + threadIdx.x;
-    if (m >= nmem) return;
-    const EnsMember& M = mem[m];
-    double* S = M.stats;
-    S[ES_UBULK] = M.scal[2];
-    S[ES_FORCING] = M.scal[1];
-    S[ES_NCLAMP] = (double)*M.ncl;
-    S[ES_STEPS] = S[ES_STEPS] + 1.0;
-    S[ES_UBULK_PRE] = M.scal[3];
-    *M.ncl = 0ull;
-    *M.state = ens_next(*M.state);
-}
-
-hipError_t run_ens_advance(const EnsLaunch& L, hipStream_t s) {
-    if (L.nmem == 0) return hipSuccess;
-    hipLaunchKernelGGL(ens_advance_kernel, dim3((L.nmem + 63) / 64), dim3(64), 0, s, L.mem,
-                       L.nmem);
+    hipLaunchKernelGGL(ens_bulk_shift_kernel, dim3(grid), dim3(kRedBlock), 0, s, ENS_ARGS(L));
     return hipGetLastError();
 }
 

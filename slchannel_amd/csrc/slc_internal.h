@@ -92,30 +92,40 @@ hipError_t run_to_f32(const Grid& g, float* const o[3], const double* const a[3]
 hipError_t run_fill_u64(unsigned long long* p, long n, unsigned long long v, hipStream_t s);
 hipError_t run_fill_f64(double* p, long n, double v, hipStream_t s);
 hipError_t run_bc(const Grid& g, double* u, double* v, double* w, hipStream_t s);
-hipError_t run_bc_p(const Grid& g, double* p, hipStream_t s);
 hipError_t run_zfactor(const Grid& g, int comp, double dt, double theta, const double* dz_c,
                        const double* dz_f, double* tab, hipStream_t s);
 hipError_t run_zsolve(const Grid& g, int comp, double* f, double dt, double theta,
                       const double* dz_c, const double* dz_f, double* tab, bool refactor,
                       hipStream_t s);
+// the three components' z-solves (tab, refactor: per component) in one launch
+hipError_t run_zsolve3(const Grid& g, double* const f[3], double dt, double theta,
+                       const double* dz_c, const double* dz_f, double* const tab[3],
+                       const bool refactor[3], hipStream_t s);
+// wrap: read no ghost entry (the fields' ghosts need not be filled)
 hipError_t run_div_planes(const Grid& g, const double* u, const double* v, const double* w,
-                          const double* dz_f, double scale, double* planes, hipStream_t s);
+                          const double* dz_f, double scale, double* planes, bool wrap,
+                          hipStream_t s);
 hipError_t run_div_field(const Grid& g, const double* u, const double* v, const double* w,
                          const double* dz_f, double* div, hipStream_t s);
 hipError_t run_field_to_planes(const Grid& g, const double* f, double scale, double* planes,
                                hipStream_t s);
 hipError_t run_poisson_thomas(const PoissonTabs& t, double* dhat, double* cp, hipStream_t s);
+// writes the ghosts of u, v, w and p too
 hipError_t run_project_planes(const Grid& g, double* u, double* v, double* w,
                               const double* planes, double inv_n, double dt,
                               const double* dz_c, double* p, hipStream_t s);
 hipError_t run_project_p(const Grid& g, double* u, double* v, double* w, const double* p,
                          double dt, const double* dz_c, hipStream_t s);
-hipError_t run_bulk(const Grid& g, double* u, double* v, double* w, const double* cv,
-                    double total_volume, double U_bulk, double dt, int shift, double* partials,
-                    int max_partials, double* scal, hipStream_t s);
+// Doubles of scratch of the bulk constraint over np partial sums: the sums
+// before and after the shift, and the ticket of the blocks that have finished.
+constexpr int bulk_scratch(int np) { return 2 * np + 1; }
+// partials: bulk_scratch(bulk_partials_needed(g)) doubles; scal: [0] correction,
+// [1] forcing, [2] mean after the shift, [3] before it
+hipError_t run_bulk(const Grid& g, double* u, const double* cv, double total_volume,
+                    double U_bulk, double dt, double* partials, double* scal, hipStream_t s);
+// the mean to out[3]
 hipError_t run_bulk_velocity(const Grid& g, const double* u, const double* cv,
-                             double total_volume, double* partials, int max_partials,
-                             double* out, hipStream_t s);
+                             double total_volume, double* partials, double* out, hipStream_t s);
 hipError_t run_axpby(double* out, const double* a, const double* b, double alpha, double beta,
                      long n, hipStream_t s);
 int bulk_partials_needed(const Grid& g);

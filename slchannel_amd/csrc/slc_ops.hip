@@ -62,9 +62,9 @@ hipError_t run_axpby(double* out, const double* a, const double* b, double alpha
 // ghost fill
 // ---------------------------------------------------------------------------
 
-__global__ void bc_kernel(Grid g, double* f0, double* f1, double* f2, int kind0) {
-    const int kind = kind0 == 3 ? 3 : (int)blockIdx.y;
-    double* F = kind0 == 3 ? f0 : (blockIdx.y == 0 ? f0 : (blockIdx.y == 1 ? f1 : f2));
+__global__ void bc_kernel(Grid g, double* u, double* v, double* w) {
+    const int kind = (int)blockIdx.y;
+    double* F = kind == 0 ? u : kind == 1 ? v : w;
     if (!F) return;
     bc_body(g, F, kind, (long)blockIdx.x * blockDim.x + threadIdx.x);
 }
@@ -76,14 +76,7 @@ hipError_t run_bc(const Grid& g, double* u, double* v, double* w, hipStream_t st
         if (n > nmax) nmax = n;
     }
     hipLaunchKernelGGL(bc_kernel, dim3((unsigned)((nmax + 255) / 256), 3), dim3(256), 0, st, g, u,
-                       v, w, 0);
-    return hipGetLastError();
-}
-
-hipError_t run_bc_p(const Grid& g, double* p, hipStream_t st) {
-    long n = ghost_count(3, g.nx, g.ny, g.nz);
-    hipLaunchKernelGGL(bc_kernel, dim3((unsigned)((n + 255) / 256), 1), dim3(256), 0, st, g, p,
-                       nullptr, nullptr, 3);
+                       v, w);
     return hipGetLastError();
 }
 
@@ -229,10 +222,80 @@ hipError_t run_zsolve(const Grid& g, int comp, double* f, double dt, double thet
     return hipGetLastError();
 }
 
+// The three components' solves in one launch (blocks of u, then v, then w): CHW
+// unknowns per lane for w's columns, which are one shorter.  Small grids leave
+// a component's launch mostly latency (3 x 5.5 -> 10.7 us at 64^3); large ones
+// lose two tails (3 x 82 -> 226 us at 256^3, 3.6 TB/s).
+struct ZSolve3 {
+    double* f[3];
+    const double* tab[3];
+    const double* dz_c;
+    const double* dz_f;
+    double beta;
+    unsigned nb;  // blocks per component
+};
+
+template <int CHU, int CHW>
+__global__ __launch_bounds__(256) void zsolve3_kernel(Grid g, ZSolve3 a) {
+    constexpr bool X = CHU >= SLC_ZSCAN_LDS_MIN_CH;
+    __shared__ double xl[kZScanCols][X ? zscan_lds<CHU>() : 1];
+    unsigned b = blockIdx.x;
+    const int c = b < a.nb ? 0 : b < 2 * a.nb ? 1 : 2;
+    b -= (unsigned)c * a.nb;
+    const long ncols = (long)g.nx * g.ny;
+    const long col = (long)b * kZScanCols + (threadIdx.x >> 6);
+    if (col >= ncols) return;
+    double* x = X ? xl[threadIdx.x >> 6] : nullptr;
+    double* xw = CHW >= SLC_ZSCAN_LDS_MIN_CH ? x : nullptr;
+    if (c == 0)
+        zsolve_scan_cols<0, CHU, 1>(g, a.f[0], a.tab[0], col, ncols, a.beta, a.dz_c, a.dz_f, x);
+    else if (c == 1)
+        zsolve_scan_cols<1, CHU, 1>(g, a.f[1], a.tab[1], col, ncols, a.beta, a.dz_c, a.dz_f, x);
+    else
+        zsolve_scan_cols<2, CHW, 1>(g, a.f[2], a.tab[2], col, ncols, a.beta, a.dz_c, a.dz_f, xw);
+}
+
+hipError_t run_zsolve3(const Grid& g, double* const f[3], double dt, double theta,
+                       const double* dz_c, const double* dz_f, double* const tab[3],
+                       const bool refactor[3], hipStream_t s) {
+    const int cu = zsolve_scan_ch(0, g.nz), cw = zsolve_scan_ch(2, g.nz);
+    if (cu == 0 || cw == 0) {
+        for (int c = 0; c < 3; ++c) {
+            hipError_t e = run_zsolve(g, c, f[c], dt, theta, dz_c, dz_f, tab[c], refactor[c], s);
+            if (e != hipSuccess) return e;
+        }
+        return hipSuccess;
+    }
+    ZSolve3 a;
+    for (int c = 0; c < 3; ++c) {
+        if (refactor[c])
+            hipLaunchKernelGGL(zfactor_kernel, dim3(1), dim3(64), 0, s, g, c, dt, theta, dz_c, dz_f,
+                               tab[c]);
+        a.f[c] = f[c];
+        a.tab[c] = tab[c];
+    }
+    a.dz_c = dz_c;
+    a.dz_f = dz_f;
+    a.beta = theta < 1.0 ? (1.0 - theta) * dt * g.nu : 0.0;
+    a.nb = (unsigned)(((long)g.nx * g.ny + kZScanCols - 1) / kZScanCols);
+    const dim3 grid(3 * a.nb), blk(256);
+#define SLC_ZS3(CU, CW) hipLaunchKernelGGL((zsolve3_kernel<CU, CW>), grid, blk, 0, s, g, a)
+    switch (cu) {
+        case 1: SLC_ZS3(1, 1); break;
+        case 2: if (cw == 2) SLC_ZS3(2, 2); else SLC_ZS3(2, 1); break;
+        case 4: if (cw == 4) SLC_ZS3(4, 4); else SLC_ZS3(4, 2); break;
+        case 8: if (cw == 8) SLC_ZS3(8, 8); else SLC_ZS3(8, 4); break;
+        default: if (cw == 16) SLC_ZS3(16, 16); else SLC_ZS3(16, 8);
+    }
+#undef SLC_ZS3
+    return hipGetLastError();
+}
+
 // ---------------------------------------------------------------------------
 // divergence -> plane-major (k, i, j) Poisson right-hand side
 // ---------------------------------------------------------------------------
 
+template <bool WRAP>
 __global__ __launch_bounds__(256) void div_planes_kernel(Grid g, const double* __restrict__ u,
                                                          const double* __restrict__ v,
                                                          const double* __restrict__ w,
@@ -240,14 +303,20 @@ __global__ __launch_bounds__(256) void div_planes_kernel(Grid g, const double* _
                                                          double scale,
                                                          double* __restrict__ planes) {
     __shared__ double tile[kT][kT + 1];
-    div_planes_body(g, u, v, w, dz_f, scale, planes, blockIdx.z, blockIdx.y * kT,
-                    blockIdx.x * kT, tile);
+    div_planes_body<WRAP>(g, u, v, w, dz_f, scale, planes, blockIdx.z, blockIdx.y * kT,
+                          blockIdx.x * kT, tile);
 }
 
 hipError_t run_div_planes(const Grid& g, const double* u, const double* v, const double* w,
-                          const double* dz_f, double scale, double* planes, hipStream_t s) {
+                          const double* dz_f, double scale, double* planes, bool wrap,
+                          hipStream_t s) {
     dim3 grid((g.nz + kT - 1) / kT, (g.ny + kT - 1) / kT, g.nx);
-    hipLaunchKernelGGL(div_planes_kernel, grid, dim3(256), 0, s, g, u, v, w, dz_f, scale, planes);
+    if (wrap)
+        hipLaunchKernelGGL(div_planes_kernel<true>, grid, dim3(256), 0, s, g, u, v, w, dz_f, scale,
+                           planes);
+    else
+        hipLaunchKernelGGL(div_planes_kernel<false>, grid, dim3(256), 0, s, g, u, v, w, dz_f, scale,
+                           planes);
     return hipGetLastError();
 }
 
@@ -261,7 +330,7 @@ __global__ void div_field_kernel(Grid g, const double* __restrict__ u,
     int k = (int)(un % (unsigned)g.nz);
     unsigned r = un / (unsigned)g.nz;
     int j = (int)(r % (unsigned)g.ny), i = (int)(r / (unsigned)g.ny);
-    div[n] = divergence_at(g, u, v, w, dz_f, i + 1, j + 1, k + 1);
+    div[n] = divergence_at<false>(g, u, v, w, dz_f, i + 1, j + 1, k + 1);
 }
 
 hipError_t run_div_field(const Grid& g, const double* u, const double* v, const double* w,
@@ -412,54 +481,49 @@ hipError_t run_project_p(const Grid& g, double* u, double* v, double* w, const d
 
 int bulk_partials_needed(const Grid& g) { return bulk_blocks(g.nx, g.ny, g.nz); }
 
-// shift 0: partial sums of u*cv; shift 1: u += corr (scal[0]) then partial sums
-__global__ __launch_bounds__(kRedBlock) void bulk_partial_kernel(Grid g, double* __restrict__ u,
-                                                                 const double* __restrict__ cv,
-                                                                 const double* __restrict__ scal,
-                                                                 int shift,
-                                                                 double* __restrict__ partials) {
+__global__ __launch_bounds__(kRedBlock) void bulk_before_kernel(Grid g, const double* u,
+                                                                const double* __restrict__ cv,
+                                                                double* partials) {
     __shared__ double red[kRedBlock];
-    bulk_partial_body(g, u, cv, shift ? scal[0] : 0.0, shift, partials, blockIdx.x, gridDim.x,
-                      red);
+    bulk_before_body(g, u, cv, partials, blockIdx.x, gridDim.x, red);
 }
 
-__global__ __launch_bounds__(kRedBlock) void bulk_finalize_kernel(
-    const double* __restrict__ partials, int np, double total_volume, double U_bulk, double dt,
-    int mode, double* __restrict__ scal) {
+__global__ __launch_bounds__(kRedBlock) void bulk_shift_kernel(Grid g, double* __restrict__ u,
+                                                               const double* __restrict__ cv,
+                                                               double* partials,
+                                                               double total_volume, double U_bulk,
+                                                               double dt,
+                                                               double* __restrict__ scal) {
     __shared__ double red[kRedBlock];
-    bulk_finalize_body(partials, np, total_volume, U_bulk, dt, mode, scal, red);
+    __shared__ bool last;
+    bulk_shift_body(g, u, cv, partials, blockIdx.x, gridDim.x, total_volume, U_bulk, dt, scal, red,
+                    &last);
 }
 
-hipError_t run_bulk(const Grid& g, double* u, double* v, double* w, const double* cv,
-                    double total_volume, double U_bulk, double dt, int shift, double* partials,
-                    int max_partials, double* scal, hipStream_t s) {
-    int np = bulk_partials_needed(g);
-    if (np > max_partials) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(bulk_partial_kernel, dim3(np), dim3(kRedBlock), 0, s, g, u, cv, scal, 0,
-                       partials);
-    hipLaunchKernelGGL(bulk_finalize_kernel, dim3(1), dim3(kRedBlock), 0, s, partials, np,
-                       total_volume, U_bulk, dt, 0, scal);
-    if (!shift) return hipGetLastError();
-    hipLaunchKernelGGL(bulk_partial_kernel, dim3(np), dim3(kRedBlock), 0, s, g, u, cv, scal, 1,
-                       partials);
-    hipLaunchKernelGGL(bulk_finalize_kernel, dim3(1), dim3(kRedBlock), 0, s, partials, np,
-                       total_volume, U_bulk, dt, 1, scal);
-    // u's ghosts follow the shifted interior (solver.py:720; v, w unchanged)
-    (void)v;
-    (void)w;
-    return run_bc(g, u, nullptr, nullptr, s);
+__global__ __launch_bounds__(kRedBlock) void bulk_mean_kernel(const double* __restrict__ partials,
+                                                              int np, double total_volume,
+                                                              double* __restrict__ out) {
+    __shared__ double red[kRedBlock];
+    const double ub = bulk_mean(partials, np, total_volume, red);
+    if (threadIdx.x == 0) *out = ub;
+}
+
+// u's ghosts follow the shifted interior (solver.py:720; v, w unchanged).
+hipError_t run_bulk(const Grid& g, double* u, const double* cv, double total_volume,
+                    double U_bulk, double dt, double* partials, double* scal, hipStream_t s) {
+    const int np = bulk_partials_needed(g);
+    hipLaunchKernelGGL(bulk_before_kernel, dim3(np), dim3(kRedBlock), 0, s, g, u, cv, partials);
+    hipLaunchKernelGGL(bulk_shift_kernel, dim3(np), dim3(kRedBlock), 0, s, g, u, cv, partials,
+                       total_volume, U_bulk, dt, scal);
+    return hipGetLastError();
 }
 
 hipError_t run_bulk_velocity(const Grid& g, const double* u, const double* cv,
-                             double total_volume, double* partials, int max_partials,
-                             double* out, hipStream_t s) {
-    int np = bulk_partials_needed(g);
-    if (np > max_partials) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(bulk_partial_kernel, dim3(np), dim3(kRedBlock), 0, s, g,
-                       const_cast<double*>(u), cv, out, 0, partials);
-    // out[0..3] is used as scratch by mode 0; the bulk value lands in out[3]
-    hipLaunchKernelGGL(bulk_finalize_kernel, dim3(1), dim3(kRedBlock), 0, s, partials, np,
-                       total_volume, 0.0, 1.0, 0, out);
+                             double total_volume, double* partials, double* out, hipStream_t s) {
+    const int np = bulk_partials_needed(g);
+    hipLaunchKernelGGL(bulk_before_kernel, dim3(np), dim3(kRedBlock), 0, s, g, u, cv, partials);
+    hipLaunchKernelGGL(bulk_mean_kernel, dim3(1), dim3(kRedBlock), 0, s, partials, np,
+                       total_volume, out + 3);
     return hipGetLastError();
 }
 

@@ -108,6 +108,44 @@ __device__ inline void bc_body(const Grid& g, double* F, int kind, long t) {
     F[((long)I * s.NJ + J) * s.NK + K] = v;
 }
 
+// Every ghost entry that takes its value from interior point (I, J, K), whose
+// value is v (for w at K = nz, which has no interior face: the top wall face):
+// with a call per interior point, the ghost fill of bc_body.  The wall entries
+// of the own column are two predicated stores; the images of the column in x
+// and y are for a few columns of a field.  A fill of its own costs a launch
+// and a pass of strided reads per set of fields: with the projection writing
+// the ghosts of u, v, w and p, its kernel went from 11.6 to 14.9 us at 64^3
+// and from 242 to 274 us at 256^3, and the two fills (2 x 4.8 and 2 x 13 us
+// and their launch gaps) went.
+__device__ inline void put_ghosts(const Grid& g, double* __restrict__ F, int kind, int I, int J,
+                                  int K, double v) {
+    const int NJ = kind == 1 ? g.ny + 1 : g.ny + 2, NK = kind == 2 ? g.nz + 1 : g.nz + 2;
+    const double lo = kind == 2 ? 0.0 : kind == 3 ? v : -v;
+    const double hi = kind == 2 ? 0.0 : kind == 3 || g.top_neumann ? v : -v;
+    double* col = F + ((long)I * NJ + J) * NK;
+    if (K == 1) col[0] = lo;
+    if (K == g.nz) col[NK - 1] = hi;
+    const bool x0 = I == g.nx, x1 = kind != 0 && I == 1;
+    const bool y0 = J == g.ny, y1 = kind != 1 && J == 1;
+    if (!(x0 || x1 || y0 || y1)) return;
+    auto image = [&](int X, int Y) {
+        double* img = F + ((long)X * NJ + Y) * NK;
+        if (kind != 2 || K < g.nz) img[K] = v;
+        if (K == 1) img[0] = lo;
+        if (K == g.nz) img[NK - 1] = hi;
+    };
+    if (x0) image(0, J);
+    if (x1) image(g.nx + 1, J);
+    if (y0) image(I, 0);
+    if (y1) image(I, g.ny + 1);
+    if ((x0 || x1) && (y0 || y1)) {
+        if (x0 && y0) image(0, 0);
+        if (x0 && y1) image(0, g.ny + 1);
+        if (x1 && y0) image(g.nx + 1, 0);
+        if (x1 && y1) image(g.nx + 1, g.ny + 1);
+    }
+}
+
 // ---------------------------------------------------------------------------
 // implicit z-diffusion: (I - theta dt nu Dzz) x = d + (1-theta) dt nu Dzz d
 // ---------------------------------------------------------------------------
@@ -526,6 +564,9 @@ __device__ inline void plane_tile(const Grid& g, long t, int& i, int& j0, int& k
     i = (int)(r / ntj);
 }
 
+// WRAP: the ghost columns and the wall faces of w are not read but taken from
+// where a ghost fill takes them (the same values without the fill).
+template <bool WRAP>
 __device__ inline double divergence_at(const Grid& g, const double* __restrict__ u,
                                        const double* __restrict__ v,
                                        const double* __restrict__ w,
@@ -533,14 +574,18 @@ __device__ inline double divergence_at(const Grid& g, const double* __restrict__
     const long uSY = g.ny + 2, uSZ = g.nz + 2;
     const long vSY = g.ny + 1, vSZ = g.nz + 2;
     const long wSY = g.ny + 2, wSZ = g.nz + 1;
-    double du = (u[((long)I * uSY + J) * uSZ + K] - u[((long)(I - 1) * uSY + J) * uSZ + K]) / g.dx;
-    double dv = (v[((long)I * vSY + J) * vSZ + K] - v[((long)I * vSY + (J - 1)) * vSZ + K]) / g.dy;
+    const int Im = WRAP && I == 1 ? g.nx : I - 1, Jm = WRAP && J == 1 ? g.ny : J - 1;
+    double du = (u[((long)I * uSY + J) * uSZ + K] - u[((long)Im * uSY + J) * uSZ + K]) / g.dx;
+    double dv = (v[((long)I * vSY + J) * vSZ + K] - v[((long)I * vSY + Jm) * vSZ + K]) / g.dy;
     long wb = ((long)I * wSY + J) * wSZ;
-    double dw = (w[wb + K] - w[wb + K - 1]) / dz_f[K - 1];
+    const double wt = WRAP && K == g.nz ? 0.0 : w[wb + K];
+    const double wl = WRAP && K == 1 ? 0.0 : w[wb + K - 1];
+    double dw = (wt - wl) / dz_f[K - 1];
     return du + dv + dw;
 }
 
 // tile: kT x (kT+1) doubles of LDS
+template <bool WRAP>
 __device__ inline void div_planes_body(const Grid& g, const double* __restrict__ u,
                                        const double* __restrict__ v,
                                        const double* __restrict__ w,
@@ -553,7 +598,7 @@ __device__ inline void div_planes_body(const Grid& g, const double* __restrict__
         for (int jj = t / kT; jj < kT; jj += 256 / kT) {
             int j = j0 + jj, k = k0 + kk;
             if (j < g.ny && k < g.nz) {
-                double d = divergence_at(g, u, v, w, dz_f, i + 1, j + 1, k + 1);
+                double d = divergence_at<WRAP>(g, u, v, w, dz_f, i + 1, j + 1, k + 1);
                 tile[jj][kk] = d / scale;
             }
         }
@@ -811,7 +856,9 @@ __device__ inline void poisson_spike_body(const PoissonTabs& t, double2* __restr
 // projection u -= dt grad p from the plane-major (unnormalised) inverse FFT
 // ---------------------------------------------------------------------------
 // Also writes the interior of the ghost-shaped pressure p = P / (nx ny).
-// t0: (kT+1) x (kT+2), t1: kT x (kT+1) doubles of LDS.
+// t0: (kT+1) x (kT+2), t1: kT x (kT+1) doubles of LDS.  Each point
+// also writes the ghost entries that take their values from it, in place of
+// a ghost fill afterwards.
 
 __device__ inline void project_planes_body(const Grid& g, double* __restrict__ u,
                                            double* __restrict__ v, double* __restrict__ w,
@@ -847,18 +894,28 @@ __device__ inline void project_planes_body(const Grid& g, double* __restrict__ u
         double pc = t0[jj][kk] * inv_n;
         double pxp = t1[jj][kk] * inv_n;
         double pyp = t0[jj + 1][kk] * inv_n;
+        double un = 0.0, vn = 0.0, wn = 0.0;
         if (u) {
             long ui = ((long)I * (ny + 2) + J) * (nz + 2) + K;
-            u[ui] = u[ui] - dt * ((pxp - pc) / g.dx);
+            un = u[ui] - dt * ((pxp - pc) / g.dx);
+            u[ui] = un;
             long vi = ((long)I * (ny + 1) + J) * (nz + 2) + K;
-            v[vi] = v[vi] - dt * ((pyp - pc) / g.dy);
+            vn = v[vi] - dt * ((pyp - pc) / g.dy);
+            v[vi] = vn;
         }
         if (u && k < nz - 1) {
             double pzp = t0[jj][kk + 1] * inv_n;
             long wi = ((long)I * (ny + 2) + J) * (nz + 1) + K;
-            w[wi] = w[wi] - dt * ((pzp - pc) / dz_c[K]);
+            wn = w[wi] - dt * ((pzp - pc) / dz_c[K]);
+            w[wi] = wn;
         }
         if (p) p[((long)I * (ny + 2) + J) * (nz + 2) + K] = pc;
+        if (u) {
+            put_ghosts(g, u, 0, I, J, K, un);
+            put_ghosts(g, v, 1, I, J, K, vn);
+            put_ghosts(g, w, 2, I, J, K, wn);
+        }
+        if (p) put_ghosts(g, p, 3, I, J, K, pc);
     }
 }
 
@@ -889,11 +946,12 @@ __device__ inline double block_sum(double v, double* red) {
     return red[0];
 }
 
-// Partial sum number blk of nb over u*cv; with shift, u += corr first.
-__device__ inline void bulk_partial_body(const Grid& g, double* __restrict__ u,
-                                         const double* __restrict__ cv, double corr, int shift,
-                                         double* __restrict__ partials, long blk, long nb,
-                                         double* red) {
+// Partial sum number blk of nb over u*cv, on every thread; SHIFT: u += corr
+// first, and the ghost entries of the shifted values are written.
+template <bool SHIFT>
+__device__ inline double bulk_partial_body(const Grid& g, double* __restrict__ u,
+                                           const double* __restrict__ cv, double corr, long blk,
+                                           long nb, double* red) {
     const long N = (long)g.nx * g.ny * g.nz;
     const long chunk = (N + nb - 1) / nb;
     const long beg = blk * chunk;
@@ -911,51 +969,109 @@ __device__ inline void bulk_partial_body(const Grid& g, double* __restrict__ u,
         int j = (int)(r % (unsigned)g.ny), i = (int)(r / (unsigned)g.ny);
         const int dk = kRedBlock % g.nz, t = kRedBlock / g.nz;
         const int dj = t % g.ny, di = t / g.ny;
-#pragma unroll 4
-        for (; n < end; n += kRedBlock) {
-            const long ui = ((long)(i + 1) * (g.ny + 2) + (j + 1)) * (g.nz + 2) + (k + 1);
-            double val = u[ui];
-            if (shift) {
-                val = val + corr;
-                u[ui] = val;
+        // kB elements at a time, so that their loads are in flight together
+        // (the shift's stores would hold back each next load)
+        constexpr int kB = 4;
+        while (n < end) {
+            double val[kB];
+            long ui[kB];
+            int ii[kB], jj[kB], kk[kB];
+#pragma unroll
+            for (int b = 0; b < kB; ++b) {
+                ii[b] = i;
+                jj[b] = j;
+                kk[b] = k;
+                ui[b] = ((long)(i + 1) * (g.ny + 2) + (j + 1)) * (g.nz + 2) + (k + 1);
+                val[b] = n + b * kRedBlock < end ? u[ui[b]] : 0.0;
+                k += dk;
+                if (k >= g.nz) {
+                    k -= g.nz;
+                    ++j;
+                }
+                j += dj;
+                if (j >= g.ny) {
+                    j -= g.ny;
+                    ++i;
+                }
+                i += di;
             }
-            acc += val * cv[k];
-            k += dk;
-            if (k >= g.nz) {
-                k -= g.nz;
-                ++j;
+#pragma unroll
+            for (int b = 0; b < kB; ++b) {
+                if (n + b * kRedBlock >= end) break;
+                if (SHIFT) {
+                    val[b] = val[b] + corr;
+                    u[ui[b]] = val[b];
+                    put_ghosts(g, u, 0, ii[b] + 1, jj[b] + 1, kk[b] + 1, val[b]);
+                }
+                acc += val[b] * cv[kk[b]];
             }
-            j += dj;
-            if (j >= g.ny) {
-                j -= g.ny;
-                ++i;
-            }
-            i += di;
+            n += kB * kRedBlock;
         }
     }
-    double s = block_sum(acc, red);
-    if (threadIdx.x == 0) partials[blk] = s;
+    return block_sum(acc, red);
 }
 
-// mode 0: scal[3] = ub*, scal[0] = U_b - ub*, scal[1] = scal[0] / dt
-// mode 1: scal[2] = ub
-__device__ inline void bulk_finalize_body(const double* __restrict__ partials, int np,
-                                          double total_volume, double U_bulk, double dt,
-                                          int mode, double* __restrict__ scal, double* red) {
+// The count of the blocks that have finished the shift, behind both sums.
+__device__ inline unsigned* bulk_ticket(double* partials, int np) {
+    return reinterpret_cast<unsigned*>(partials + 2 * np);
+}
+
+// First pass, block blk of np.
+__device__ inline void bulk_before_body(const Grid& g, const double* u,
+                                        const double* __restrict__ cv, double* partials, int blk,
+                                        int np, double* red) {
+    const double s = bulk_partial_body<false>(g, const_cast<double*>(u), cv, 0.0, blk, np, red);
+    if (threadIdx.x != 0) return;
+    partials[blk] = s;
+    if (blk == 0) *bulk_ticket(partials, np) = 0u;
+}
+
+// The np partial sums over the volume, on every thread (a fixed tree).  AGENT:
+// the partials were written by other blocks of this launch.
+template <bool AGENT = false>
+__device__ inline double bulk_mean(const double* partials, int np, double total_volume,
+                                   double* red) {
     double acc = 0.0;
-    for (int b = threadIdx.x; b < np; b += kRedBlock) acc += partials[b];
-    double s = block_sum(acc, red);
+    for (int b = threadIdx.x; b < np; b += kRedBlock)
+        acc += AGENT ? __hip_atomic_load(partials + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+                     : partials[b];
+    return block_sum(acc, red) / total_volume;
+}
+
+// Second pass, block blk of np: every block forms the mean from the partial
+// sums (a few thousand cached loads in place of a launch of its own), shifts
+// its chunk and the ghost entries that follow it, and sums the shifted
+// values.  The last block to finish forms the mean after the shift, fills
+// scal -- [0] correction, [1] forcing, [2] mean after the shift, [3] before
+// it -- and returns true (on every thread).  The sums cross blocks as
+// agent-scope accesses, each ahead of its block's ticket: a release fence
+// would write back the shifted values of the whole L2 with every block.
+// Two launches in place of five (sums, mean, shift and sums, mean, ghosts):
+// 24 -> 14 us at 64^3, 120 -> 117 us at 256^3 (bound by memory there).
+__device__ inline bool bulk_shift_body(const Grid& g, double* __restrict__ u,
+                                       const double* __restrict__ cv, double* partials, int blk,
+                                       int np, double total_volume, double U_bulk, double dt,
+                                       double* __restrict__ scal, double* red, bool* last) {
+    const double ub = bulk_mean(partials, np, total_volume, red);
+    const double corr = U_bulk - ub;
+    double* after = partials + np;
+    const double s = bulk_partial_body<true>(g, u, cv, corr, blk, np, red);
     if (threadIdx.x == 0) {
-        double ub = s / total_volume;
-        if (mode == 0) {
-            double corr = U_bulk - ub;
-            scal[3] = ub;
-            scal[0] = corr;
-            scal[1] = corr / dt;
-        } else {
-            scal[2] = ub;
-        }
+        __hip_atomic_store(after + blk, s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        *last = __hip_atomic_fetch_add(bulk_ticket(partials, np), 1u, __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_AGENT) == (unsigned)np - 1u;
     }
+    __syncthreads();
+    if (!*last) return false;
+    const double ua = bulk_mean<true>(after, np, total_volume, red);
+    if (threadIdx.x == 0) {
+        scal[0] = corr;
+        scal[1] = corr / dt;
+        scal[2] = ua;
+        scal[3] = ub;
+    }
+    return true;
 }
 
 }  // namespace slc

@@ -67,7 +67,6 @@ struct slc_plan {
     double zkey[3][2] = {};     // (dt, theta) the factor of each component was built for
     bool zvalid[3] = {false, false, false};
     double* partials = nullptr;
-    int max_partials = 0;
     double* diag_part = nullptr;  // slc_diagnostics partials (5 per workgroup)
     double* us[3] = {nullptr, nullptr, nullptr};  // U* = 2V^n - V^{n-1} (ghost-shaped)
     double* nfoot = nullptr;                      // near feet of one component (3 x N)

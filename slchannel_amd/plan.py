@@ -283,6 +283,16 @@ class HipPlan:
                                               float(rhs_scale), float(dt_proj), _ptr(p),
                                               self._stream()), "slc_project_step")
 
+    def implicit_project(self, u, v, w, dt_z, theta, rhs_scale, dt_proj, p=None):
+        """The z-solves of u, v, w and the projection, ghosts included
+        (slc_implicit_project)."""
+        self._uvw(u, v, w)
+        if p is not None:
+            self._chk(p, self.shapes["p"], "p")
+        _lib.check(self._lib.slc_implicit_project(
+            self._h, _ptr(u), _ptr(v), _ptr(w), float(dt_z), float(theta), float(rhs_scale),
+            float(dt_proj), _ptr(p), self._stream()), "slc_implicit_project")
+
     def bulk_velocity(self, u, out):
         self._chk(u, self.shapes["u"], "u")
         self._chk(out, (4,), "out")

@@ -11,10 +11,9 @@ and re-bootstrap with one BDF1 step; statistics are
 slchannel_amd.TurbulenceStats.  The run loop and plotting of the reference
 are not part of this layer.
 
-Per step the device does: ghost fill; the fused two-foot BDF2 predictor (far
-pass + near pass per component); ghost fill; three Thomas z-solves; ghost fill;
-divergence -> rocFFT -> per-mode Thomas -> inverse rocFFT -> gradient
-projection -> ghost fill; the deterministic bulk shift.  No host
+Per step the device does: ghost fill; the fused two-foot BDF2 predictor; the
+Thomas z-solves; divergence -> rocFFT -> per-mode Thomas -> inverse rocFFT ->
+gradient projection with the ghosts; the deterministic bulk shift.  No host
 synchronisation: u_bulk and forcing come back as 0-D device tensors, as in the
 reference.
 """
@@ -132,7 +131,6 @@ class SLChannelFlow:
         self.time = 0.0
         self.initial_step = 0
         self.initial_time = 0.0
-        self._nclamp = torch.zeros(1, dtype=torch.int64, device=self.device)
         self._bulk = torch.zeros(4, dtype=torch.float64, device=self.device)
 
         init = cfg.get("initialization") or {}
@@ -248,25 +246,16 @@ class SLChannelFlow:
     def _apply_bulk_forcing(self, dt):
         """solver.py:694-723: exact uniform shift of u onto U_bulk; forcing is
         the correction / dt.  Returns 0-D device tensors."""
+        self._bulk = torch.empty(4, dtype=torch.float64, device=self.device)
         self.plan.bulk_force(self.u, self.v, self.w, self.U_bulk, dt, self._bulk)
-        self.forcing = self._bulk[1].clone()
-        return self._bulk[2].clone(), self.forcing
+        self.forcing = self._bulk[1]
+        return self._bulk[2], self.forcing
 
     def _implicit_and_project(self, dt_z, rhs_scale, dt_proj, theta=1.0, sl=True):
-        """(Ghosts,) z-solves, ghosts, projection; returns the buffer holding
-        phi: self.p, or for SL steps with the 'inc' option a separate phi
-        buffer (self.p then ends as the full pressure p^{n+1})."""
-        plan = self.plan
-        # the z-solves read ghost values only for the explicit part of a
-        # theta < 1 right-hand side; at theta = 1 the fill the reference makes
-        # here (solver.py:766, 949) is overwritten by the one after the solves
-        # before anything reads it
-        if theta != 1.0:
-            plan.apply_bc(self.u, self.v, self.w)
-        plan.zsolve("u", self.u, dt_z, theta)
-        plan.zsolve("v", self.v, dt_z, theta)
-        plan.zsolve("w", self.w, dt_z, theta)
-        plan.apply_bc(self.u, self.v, self.w)
+        """z-solves and projection with the ghosts they need and leave; returns
+        the buffer holding phi: self.p, or for SL steps with the 'inc' option
+        a separate phi buffer (self.p then ends as the full pressure
+        p^{n+1})."""
         if sl and self.sl_bdf2_pressure == "inc":
             if self._phi is None:
                 self._phi = torch.zeros_like(self.p)
@@ -275,7 +264,7 @@ class SLChannelFlow:
             if self.p is self._P_curr or self.p is self._P_prev:
                 self.p = torch.empty_like(self.p)  # keep the 'inc' history intact
             phi = self.p
-        plan.project_step(self.u, self.v, self.w, rhs_scale, dt_proj, phi)
+        self.plan.implicit_project(self.u, self.v, self.w, dt_z, theta, rhs_scale, dt_proj, phi)
         return phi
 
     def _step_sl_bdf1_bootstrap(self, dt):
@@ -287,9 +276,9 @@ class SLChannelFlow:
             self.u_nm1.copy_(self.u)
             self.v_nm1.copy_(self.v)
             self.w_nm1.copy_(self.w)
-        self._nclamp.zero_()
+        nclamp = torch.zeros(1, dtype=torch.int64, device=self.device)
         us, vs, ws = self._star
-        self.plan.bdf1_predict(self.u, self.v, self.w, dt, us, vs, ws, self._nclamp)
+        self.plan.bdf1_predict(self.u, self.v, self.w, dt, us, vs, ws, nclamp)
         # adopt the predictor buffers; the old field buffers become scratch
         self._star = [self.u, self.v, self.w]
         self.u, self.v, self.w = us, vs, ws
@@ -302,7 +291,7 @@ class SLChannelFlow:
                 self._P_curr.copy_(phi)
             self._P_prev = None
             self.p = self._P_curr
-        self.sl.n_clamped_last = self._nclamp[0].clone()
+        self.sl.n_clamped_last = nclamp[0]
         self._dt_prev_step = dt
         return self._apply_bulk_forcing(dt)
 
@@ -318,10 +307,10 @@ class SLChannelFlow:
             out = self._step_sl_bdf1_bootstrap(dt)
         else:
             self._ensure_star()
-            self._nclamp.zero_()
+            nclamp = torch.zeros(1, dtype=torch.int64, device=self.device)
             us, vs, ws = self._star
             self.plan.bdf2_predict(self.u, self.v, self.w, self.u_nm1, self.v_nm1, self.w_nm1,
-                                   dt, us, vs, ws, self._nclamp)
+                                   dt, us, vs, ws, nclamp)
             dt_eff = (2.0 / 3.0) * dt
             p_ext = self._pressure_extrapolation()
             if p_ext is not None:
@@ -335,7 +324,7 @@ class SLChannelFlow:
             phi = self._implicit_and_project(dt_eff, dt_eff, dt_eff)
             if self.sl_bdf2_pressure == "inc":
                 self._pressure_update(p_ext, phi)
-            self.sl.n_clamped_last = self._nclamp[0].clone()
+            self.sl.n_clamped_last = nclamp[0]
             self._dt_prev_step = dt
             out = self._apply_bulk_forcing(dt)
         self.current_step += 1
