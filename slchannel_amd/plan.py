@@ -317,6 +317,19 @@ class HipPlan:
                                             *[_ptr(t) for t in r], *rp, float(dt),
                                             self._stream()), "slc_ab2_update")
 
+    def imex_advance(self, u, v, w, new, r, r_prev, dt):
+        """imex_rhs and ab2_update in one pass: r and the updated fields `new`
+        (interiors only; slc_imex_advance)."""
+        self._uvw(u, v, w)
+        self._uvw(*new, "_new")
+        self._uvw(*r, "_rhs")
+        if r_prev is not None:
+            self._uvw(*r_prev, "_prev")
+        rp = [_ptr(t) for t in r_prev] if r_prev is not None else [_ptr(None)] * 3
+        _lib.check(self._lib.slc_imex_advance(self._h, _ptr(u), _ptr(v), _ptr(w),
+                                              *[_ptr(t) for t in new], *[_ptr(t) for t in r], *rp,
+                                              float(dt), self._stream()), "slc_imex_advance")
+
     def set_viscosity(self, nu):
         """slc_set_viscosity: the plan's nu (z-solve factors rebuilt at next use)."""
         _lib.check(self._lib.slc_set_viscosity(self._h, float(nu)), "slc_set_viscosity")

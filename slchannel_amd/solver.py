@@ -377,9 +377,11 @@ class SLChannelFlow:
         if self._imex_cur is None:
             self._imex_cur = [torch.empty(s[c], dtype=torch.float64, device=self.device)
                               for c in "uvw"]
-        self.plan.imex_rhs(self.u, self.v, self.w, *self._imex_cur)
-        prev = self._imex_prev
-        self.plan.ab2_update(self.u, self.v, self.w, self._imex_cur, prev, dt)
+        self._ensure_star()
+        prev, new = self._imex_prev, self._star
+        self.plan.imex_advance(self.u, self.v, self.w, new, self._imex_cur, prev, dt)
+        self._star = [self.u, self.v, self.w]
+        self.u, self.v, self.w = new
         # the current rhs becomes the previous one (buffers swapped, no copy)
         self._imex_prev, self._imex_cur = self._imex_cur, prev
         self._implicit_and_project(dt, dt, dt, theta=0.5, sl=False)
