@@ -121,6 +121,12 @@ __host__ __device__ inline void ens_tile_shape(int s, int& ti, int& tj, int& tk)
     tk = s == 1 ? 32 : 16;
 }
 
+// Columns per work unit of the register z-solve: four wavefronts walk them.
+#ifndef SLC_ENS_ZCOLS
+#define SLC_ENS_ZCOLS 32
+#endif
+constexpr unsigned kEnsZCols = SLC_ENS_ZCOLS;
+
 // launchers: `grid` is the persistent grid size (workgroups); the SL tile
 // launcher runs one workgroup per unit and ignores it
 hipError_t run_ens_bc3(const EnsLaunch& L, unsigned grid, hipStream_t s);
@@ -132,8 +138,9 @@ void run_ens_tile_d4(const EnsMember* mem, const EnsTiles& t, int pass, int shap
 void run_ens_tile_d6(const EnsMember* mem, const EnsTiles& t, int pass, int shape, hipStream_t s);
 void run_ens_tile_f4(const EnsMember* mem, const EnsTiles& t, int pass, int shape, hipStream_t s);
 void run_ens_tile_f6(const EnsMember* mem, const EnsTiles& t, int pass, int shape, hipStream_t s);
+// max_ch: 2, 4 or 8 where no member's columns hold more unknowns per lane, else 0
 hipError_t run_ens_zsolve(const EnsLaunch& L, int comp, size_t lds_bytes, unsigned grid,
-                          bool short_cols, hipStream_t s);
+                          int max_ch, hipStream_t s);
 hipError_t run_ens_div_planes(const EnsLaunch& L, unsigned grid, hipStream_t s);
 hipError_t run_ens_thomas(const EnsLaunch& L, unsigned grid, hipStream_t s);
 hipError_t run_ens_project(const EnsLaunch& L, unsigned grid, hipStream_t s);

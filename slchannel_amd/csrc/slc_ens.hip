@@ -116,7 +116,7 @@ struct slc_ens {
     unsigned totals[EK_COUNT] = {};
     size_t zs_lds[3] = {0, 0, 0};
     bool big = false;  // a member needs the tile kernels' 64-bit addressing (tile shape 0 only)
-    bool zs_short[3] = {false, false, false};  // every member: <= 2 unknowns per lane
+    int zs_max[3] = {0, 0, 0};  // run_ens_zsolve's max_ch
     // rocFFT
     rocfft_execution_info info = nullptr;
     void* fft_work = nullptr;
@@ -311,7 +311,7 @@ int rebuild(slc_ens* e) {
     std::vector<int> umap[3];
     for (int k = 0; k < 3; ++k) {
         e->zs_lds[k] = 0;
-        e->zs_short[k] = true;
+        e->zs_max[k] = 2;
     }
     e->big = false;
     for (const Member* m : e->members) e->big = e->big || big_index(m->plan->g);
@@ -353,8 +353,9 @@ int rebuild(slc_ens* e) {
         M.npart = bulk_partials_needed(pl->g);
         for (int k = 0; k < 3; ++k) {
             M.zch[k] = zsolve_scan_ch(k, m->nz);
-            M.zcols[k] = M.zch[k] > 0 ? kZScanCols * zscan_k(M.zch[k]) : zsolve_cols(k, m->nz);
-            e->zs_short[k] = e->zs_short[k] && (M.zch[k] == 1 || M.zch[k] == 2);
+            M.zcols[k] = M.zch[k] > 0 ? (int)kEnsZCols : zsolve_cols(k, m->nz);
+            if (M.zch[k] == 0 || M.zch[k] > 8) e->zs_max[k] = 0;
+            else if (e->zs_max[k] != 0) e->zs_max[k] = std::max(e->zs_max[k], M.zch[k]);
         }
         for (int k = 0; k < 3; ++k) M.nghost[k] = ghost_count(k, m->nx, m->ny, m->nz);
         // work units
@@ -489,7 +490,7 @@ int enqueue_step(slc_ens* e) {
     // projection and the bulk shift write them with the interior
     for (int c = 0; c < 3; ++c)
         HIP_OK(run_ens_zsolve(launch(e, EK_ZS0 + c), c, e->zs_lds[c], pgrid(e, EK_ZS0 + c),
-                              e->zs_short[c], s));
+                              e->zs_max[c], s));
     HIP_OK(run_ens_div_planes(launch(e, EK_PLANE), pgrid(e, EK_PLANE), s));
     if (int rc = fft_all(e, true)) return rc;
     HIP_OK(run_ens_thomas(launch(e, EK_THOMAS), pgrid(e, EK_THOMAS), s));
@@ -968,7 +969,7 @@ static int autotune_sweeps(slc_ens* e, int reps, hipEvent_t t0, hipEvent_t t1,
             HIP_OK(run_ens_ustar(launch(e, EK_ELEM), pgrid(e, EK_ELEM), s));
             for (int c = 0; c < 3; ++c)
                 HIP_OK(run_ens_zsolve(launch(e, EK_ZS0 + c), c, e->zs_lds[c],
-                                      pgrid(e, EK_ZS0 + c), e->zs_short[c], s));
+                                      pgrid(e, EK_ZS0 + c), e->zs_max[c], s));
             HIP_OK(run_ens_div_planes(launch(e, EK_PLANE), pgrid(e, EK_PLANE), s));
             HIP_OK(run_ens_thomas(launch(e, EK_THOMAS), pgrid(e, EK_THOMAS), s));
             return SLC_OK;

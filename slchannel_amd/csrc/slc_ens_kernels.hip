@@ -98,8 +98,12 @@ hipError_t run_ens_tile(const EnsMember* mem, const EnsTiles& t, int pass, int o
 // implicit z-diffusion (theta = 1) of the predictor, BDF1 or BDF2 factor
 // ---------------------------------------------------------------------------
 
-template <int C>
-__global__ __launch_bounds__(256) void ens_zsolve_kernel(ENS_PARAMS) {
+// One kernel per longest column of the ensemble, so that its registers (and
+// the wavefronts that they leave) are those of the columns it solves: at most
+// 2 unknowns per lane, at most 4 or 8, or any (MAXCH 0: the LDS path as well).
+template <int C, int MAXCH>
+__global__ __launch_bounds__(256, MAXCH == 2 ? 5 : MAXCH == 4 ? 4 : MAXCH == 8 ? 2 : 1) void ens_zsolve_kernel(
+    ENS_PARAMS) {
     extern __shared__ double lds[];
     __shared__ long cbase[kZColsMax];
     ens_for(start, nmem, total, [&](int m, unsigned u) {
@@ -107,11 +111,11 @@ __global__ __launch_bounds__(256) void ens_zsolve_kernel(ENS_PARAMS) {
         const int st = *M.state;
         const int nz = M.g.nz;
         const double* tab = M.ztab + (ens_bdf2(st) ? 9 : 0) * (long)(nz + 2) + C * 3L * (nz + 2);
-        if (M.zch[C] > 0) {
-            const long ncols = (long)M.g.nx * M.g.ny;
-            const long col0 = ((long)u * kZScanCols + (threadIdx.x >> 6)) * zscan_k(M.zch[C]);
-            if (col0 < ncols)
-                zsolve_scan_any<C>(M.g, M.fld[ens_c(st)][C], tab, col0, ncols, M.zch[C]);
+        if (MAXCH > 0 || M.zch[C] > 0) {
+            const unsigned col0 = u * kEnsZCols, ncols = (unsigned)(M.g.nx * M.g.ny);
+            zsolve_run_any<C, (MAXCH > 0 ? MAXCH : kZScanMaxCh)>(
+                M.g, M.fld[ens_c(st)][C], tab, col0 + (threadIdx.x >> 6), kZScanCols,
+                min(col0 + kEnsZCols, ncols), M.zch[C]);
         } else {
             zsolve_body<C>(M.g, M.fld[ens_c(st)][C], tab, 0.0, M.dzc, M.dzf, M.zcols[C], u, lds,
                            cbase);
@@ -119,47 +123,25 @@ __global__ __launch_bounds__(256) void ens_zsolve_kernel(ENS_PARAMS) {
     });
 }
 
-// The same for ensembles whose every member's columns hold at most 2
-// unknowns per lane: only those variants are compiled in, so the kernel is
-// built for more waves per SIMD than the general one (which the longest
-// variants and the LDS column path hold at 125 VGPRs, four waves).
-#ifndef SLC_ENS_ZS_SHORT_WAVES
-#define SLC_ENS_ZS_SHORT_WAVES 6
-#endif
 template <int C>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SLC_ENS_ZS_SHORT_WAVES)))
-void ens_zsolve_short_kernel(ENS_PARAMS) {
-    static_assert(zscan_k(1) == zscan_k(2), "one column count for both short variants");
-    ens_for(start, nmem, total, [&](int m, unsigned u) {
-        const EnsMember& M = mem[m];
-        const int st = *M.state;
-        const int nz = M.g.nz;
-        const double* tab = M.ztab + (ens_bdf2(st) ? 9 : 0) * (long)(nz + 2) + C * 3L * (nz + 2);
-        const long ncols = (long)M.g.nx * M.g.ny;
-        const long col0 = ((long)u * kZScanCols + (threadIdx.x >> 6)) * zscan_k(1);
-        double* F = M.fld[ens_c(st)][C];
-        if (col0 < ncols) {
-            if (M.zch[C] == 1) zsolve_scan_cols<C, 1, zscan_k(1)>(M.g, F, tab, col0, ncols);
-            else zsolve_scan_cols<C, 2, zscan_k(2)>(M.g, F, tab, col0, ncols);
-        }
-    });
+void launch_ens_zsolve(const EnsLaunch& L, size_t lds_bytes, unsigned grid, int max_ch,
+                       hipStream_t s) {
+#define SLC_ENS_ZS(MAXCH)                                                                    \
+    hipLaunchKernelGGL((ens_zsolve_kernel<C, MAXCH>), dim3(grid), dim3(256), lds_bytes, s,   \
+                       ENS_ARGS(L))
+    if (max_ch == 2) SLC_ENS_ZS(2);
+    else if (max_ch == 4) SLC_ENS_ZS(4);
+    else if (max_ch == 8) SLC_ENS_ZS(8);
+    else SLC_ENS_ZS(0);
+#undef SLC_ENS_ZS
 }
 
 hipError_t run_ens_zsolve(const EnsLaunch& L, int comp, size_t lds_bytes, unsigned grid,
-                          bool short_cols, hipStream_t s) {
+                          int max_ch, hipStream_t s) {
     if (L.total == 0) return hipSuccess;
-#define SLC_ENS_ZS(K, CV) \
-    hipLaunchKernelGGL((K<CV>), dim3(grid), dim3(256), lds_bytes, s, ENS_ARGS(L))
-    if (short_cols) {
-        if (comp == 0) SLC_ENS_ZS(ens_zsolve_short_kernel, 0);
-        else if (comp == 1) SLC_ENS_ZS(ens_zsolve_short_kernel, 1);
-        else SLC_ENS_ZS(ens_zsolve_short_kernel, 2);
-    } else {
-        if (comp == 0) SLC_ENS_ZS(ens_zsolve_kernel, 0);
-        else if (comp == 1) SLC_ENS_ZS(ens_zsolve_kernel, 1);
-        else SLC_ENS_ZS(ens_zsolve_kernel, 2);
-    }
-#undef SLC_ENS_ZS
+    if (comp == 0) launch_ens_zsolve<0>(L, lds_bytes, grid, max_ch, s);
+    else if (comp == 1) launch_ens_zsolve<1>(L, lds_bytes, grid, max_ch, s);
+    else launch_ens_zsolve<2>(L, lds_bytes, grid, max_ch, s);
     return hipGetLastError();
 }
 

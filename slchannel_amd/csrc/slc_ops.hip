@@ -140,11 +140,6 @@ __global__ __launch_bounds__(256) void zsolve_kernel(Grid g, double* __restrict_
     zsolve_body<C>(g, F, tab, beta, dz_c, dz_f, kZCols, blockIdx.x, lds, cbase);
 }
 
-// columns per wavefront of the single-run z-solve (compile-time sweep knob)
-#ifndef SLC_ZSCAN_K
-#define SLC_ZSCAN_K 1
-#endif
-constexpr int kZScanK = SLC_ZSCAN_K;
 // Columns of 8 or more unknowns per lane move through LDS (coalesced), the
 // shorter ones straight to the lanes.  Measured: 1024x1024x512 (8 per lane)
 // 4.1 -> 2.8 ms per component; 256^3 (4 per lane) 0.0825 -> 0.0845 ms.
@@ -152,43 +147,80 @@ constexpr int kZScanK = SLC_ZSCAN_K;
 #define SLC_ZSCAN_LDS_MIN_CH 8
 #endif
 
-template <int C, int CH, int K>
-__global__ __launch_bounds__(256) void zsolve_scan_kernel(Grid g, double* __restrict__ F,
-                                                          const double* __restrict__ tab,
-                                                          double beta,
-                                                          const double* __restrict__ dz_c,
-                                                          const double* __restrict__ dz_f) {
-    constexpr bool X = CH >= SLC_ZSCAN_LDS_MIN_CH;
-    __shared__ double xl[kZScanCols][X ? zscan_lds<CH>(K) : 1];
-    const long ncols = (long)g.nx * g.ny;
-    const long col0 = ((long)blockIdx.x * kZScanCols + (threadIdx.x >> 6)) * K;
-    if (col0 < ncols)
-        zsolve_scan_cols<C, CH, K>(g, F, tab, col0, ncols, beta, dz_c, dz_f,
-                                   X ? xl[threadIdx.x >> 6] : nullptr);
+// The components' column solves in one launch: nb[c] blocks of component c
+// walk its columns with a stride of all its wavefronts.
+struct ZSolve3 {
+    double* f[3];
+    const double* tab[3];
+    const double* dz_c;
+    const double* dz_f;
+    double beta;
+    unsigned nb[3];
+};
+
+// Wavefronts per SIMD that the columns' registers leave.
+constexpr int zwaves(int ch, bool expl) {
+    return ch <= 1 ? (expl ? 5 : 8) : ch <= 2 ? (expl ? 4 : 6) : ch <= 4 ? (expl ? 3 : 4)
+           : ch <= 8 ? 2 : 1;
 }
 
-template <int C>
-void launch_zsolve_scan(const Grid& g, double* f, const double* tab, int ch, double beta,
-                        const double* dz_c, const double* dz_f, hipStream_t s) {
-    const long ncols = (long)g.nx * g.ny;
-    // one column per wavefront (a single small grid needs the workgroups: four
-    // short columns per wavefront, as the ensemble solves them, measured
-    // 14.8 -> 17.3 us at 96x64x128); 16 unknowns per lane: two would not fit
-    // the registers
-    const long K = ch <= 8 ? kZScanK : 1;
-    const long per = (long)kZScanCols * K;
-    const dim3 grid((unsigned)((ncols + per - 1) / per)), blk(256);
-#define SLC_ZSCAN(CHV)                                                                        \
-    hipLaunchKernelGGL((zsolve_scan_kernel<C, CHV, (CHV <= 8 ? kZScanK : 1)>), grid, blk, 0, s, \
-                       g, f, tab, beta, dz_c, dz_f)
-    switch (ch) {
-        case 1: SLC_ZSCAN(1); break;
-        case 2: SLC_ZSCAN(2); break;
-        case 4: SLC_ZSCAN(4); break;
-        case 8: SLC_ZSCAN(8); break;
-        default: SLC_ZSCAN(16); break;
+template <int CHU, int CHW, bool EXPL>
+__global__ __launch_bounds__(256, zwaves(CHU, EXPL)) void zsolve3_kernel(Grid g, ZSolve3 a) {
+    constexpr bool XU = CHU >= SLC_ZSCAN_LDS_MIN_CH, XW = CHW >= SLC_ZSCAN_LDS_MIN_CH;
+    __shared__ double xl[kZScanCols][XU ? zscan_lds<CHU>() : 1];
+    unsigned b = blockIdx.x;
+    const int c = b < a.nb[0] ? 0 : b < a.nb[0] + a.nb[1] ? 1 : 2;
+    if (c > 0) b -= a.nb[0];
+    if (c > 1) b -= a.nb[1];
+    const unsigned ncols = (unsigned)(g.nx * g.ny);
+    const unsigned wave = threadIdx.x >> 6;
+    const unsigned col = b * kZScanCols + wave, stride = a.nb[c] * kZScanCols;
+    double* xu = XU ? xl[wave] : nullptr;
+    double* xw = XW ? xl[wave] : nullptr;
+    if (c == 0)
+        zsolve_run<0, CHU, EXPL>(g, a.f[0], a.tab[0], col, stride, ncols, a.beta, a.dz_c, a.dz_f, xu);
+    else if (c == 1)
+        zsolve_run<1, CHU, EXPL>(g, a.f[1], a.tab[1], col, stride, ncols, a.beta, a.dz_c, a.dz_f, xu);
+    else
+        zsolve_run<2, CHW, EXPL>(g, a.f[2], a.tab[2], col, stride, ncols, a.beta, a.dz_c, a.dz_f, xw);
+}
+
+// Arguments of `comps` components in one launch: a block per 4 columns, and
+// where those are more than the chip holds at once, as many as it holds.
+constexpr int kCUs = 256;
+static ZSolve3 zsolve3(const Grid& g, double beta, const double* dz_c, const double* dz_f,
+                       int comps) {
+    ZSolve3 a{};
+    a.dz_c = dz_c;
+    a.dz_f = dz_f;
+    a.beta = beta;
+    const long ncols = (long)g.nx * g.ny, most =
+        kCUs * zwaves(zsolve_scan_ch(0, g.nz), beta != 0.0) / comps;
+    for (int c = 0; c < 3; ++c)
+        a.nb[c] = (unsigned)std::min<long>((ncols + kZScanCols - 1) / kZScanCols, most);
+    return a;
+}
+
+static hipError_t launch_zsolve3(const Grid& g, const ZSolve3& a, hipStream_t s) {
+    const int cu = zsolve_scan_ch(0, g.nz), cw = zsolve_scan_ch(2, g.nz);
+    const dim3 grid(a.nb[0] + a.nb[1] + a.nb[2]), blk(256);
+#define SLC_ZS3(CU, CW)                                                              \
+    if (a.beta != 0.0)                                                               \
+        hipLaunchKernelGGL((zsolve3_kernel<CU, CW, true>), grid, blk, 0, s, g, a);   \
+    else                                                                             \
+        hipLaunchKernelGGL((zsolve3_kernel<CU, CW, false>), grid, blk, 0, s, g, a)
+    // w's columns are one unknown shorter: a class below where u's just
+    // spill over
+    switch (cu) {
+        case 1: SLC_ZS3(1, 1); break;
+        case 2: if (cw == 2) { SLC_ZS3(2, 2); } else { SLC_ZS3(2, 1); } break;
+        case 4: if (cw == 4) { SLC_ZS3(4, 4); } else { SLC_ZS3(4, 2); } break;
+        case 8: if (cw == 8) { SLC_ZS3(8, 8); } else { SLC_ZS3(8, 4); } break;
+        case 16: if (cw == 16) { SLC_ZS3(16, 16); } else { SLC_ZS3(16, 8); } break;
+        default: SLC_ZS3(16, 16);  // w alone: u's columns are too long
     }
-#undef SLC_ZSCAN
+#undef SLC_ZS3
+    return hipGetLastError();
 }
 
 hipError_t run_zsolve(const Grid& g, int comp, double* f, double dt, double theta,
@@ -200,10 +232,11 @@ hipError_t run_zsolve(const Grid& g, int comp, double* f, double dt, double thet
     double beta = theta < 1.0 ? (1.0 - theta) * dt * g.nu : 0.0;
     const int ch = zsolve_scan_ch(comp, g.nz);
     if (ch > 0) {
-        if (comp == 0) launch_zsolve_scan<0>(g, f, tab, ch, beta, dz_c, dz_f, s);
-        else if (comp == 1) launch_zsolve_scan<1>(g, f, tab, ch, beta, dz_c, dz_f, s);
-        else launch_zsolve_scan<2>(g, f, tab, ch, beta, dz_c, dz_f, s);
-        return hipGetLastError();
+        ZSolve3 a = zsolve3(g, beta, dz_c, dz_f, 1);
+        a.f[comp] = f;
+        a.tab[comp] = tab;
+        for (int c = 0; c < 3; ++c) a.nb[c] = c == comp ? a.nb[c] : 0u;
+        return launch_zsolve3(g, a, s);
     }
     long ncols = (long)g.nx * g.ny;
     const int cols = zsolve_cols(comp, g.nz);
@@ -222,51 +255,18 @@ hipError_t run_zsolve(const Grid& g, int comp, double* f, double dt, double thet
     return hipGetLastError();
 }
 
-// The three components' solves in one launch (blocks of u, then v, then w): CHW
-// unknowns per lane for w's columns, which are one shorter.  Small grids leave
-// a component's launch mostly latency (3 x 5.5 -> 10.7 us at 64^3); large ones
-// lose two tails (3 x 82 -> 226 us at 256^3, 3.6 TB/s).
-struct ZSolve3 {
-    double* f[3];
-    const double* tab[3];
-    const double* dz_c;
-    const double* dz_f;
-    double beta;
-    unsigned nb;  // blocks per component
-};
-
-template <int CHU, int CHW>
-__global__ __launch_bounds__(256) void zsolve3_kernel(Grid g, ZSolve3 a) {
-    constexpr bool X = CHU >= SLC_ZSCAN_LDS_MIN_CH;
-    __shared__ double xl[kZScanCols][X ? zscan_lds<CHU>() : 1];
-    unsigned b = blockIdx.x;
-    const int c = b < a.nb ? 0 : b < 2 * a.nb ? 1 : 2;
-    b -= (unsigned)c * a.nb;
-    const long ncols = (long)g.nx * g.ny;
-    const long col = (long)b * kZScanCols + (threadIdx.x >> 6);
-    if (col >= ncols) return;
-    double* x = X ? xl[threadIdx.x >> 6] : nullptr;
-    double* xw = CHW >= SLC_ZSCAN_LDS_MIN_CH ? x : nullptr;
-    if (c == 0)
-        zsolve_scan_cols<0, CHU, 1>(g, a.f[0], a.tab[0], col, ncols, a.beta, a.dz_c, a.dz_f, x);
-    else if (c == 1)
-        zsolve_scan_cols<1, CHU, 1>(g, a.f[1], a.tab[1], col, ncols, a.beta, a.dz_c, a.dz_f, x);
-    else
-        zsolve_scan_cols<2, CHW, 1>(g, a.f[2], a.tab[2], col, ncols, a.beta, a.dz_c, a.dz_f, xw);
-}
-
+// The three components' solves, in one launch where the columns fit the lanes.
 hipError_t run_zsolve3(const Grid& g, double* const f[3], double dt, double theta,
                        const double* dz_c, const double* dz_f, double* const tab[3],
                        const bool refactor[3], hipStream_t s) {
-    const int cu = zsolve_scan_ch(0, g.nz), cw = zsolve_scan_ch(2, g.nz);
-    if (cu == 0 || cw == 0) {
+    if (zsolve_scan_ch(0, g.nz) == 0 || zsolve_scan_ch(2, g.nz) == 0) {
         for (int c = 0; c < 3; ++c) {
             hipError_t e = run_zsolve(g, c, f[c], dt, theta, dz_c, dz_f, tab[c], refactor[c], s);
             if (e != hipSuccess) return e;
         }
         return hipSuccess;
     }
-    ZSolve3 a;
+    ZSolve3 a = zsolve3(g, theta < 1.0 ? (1.0 - theta) * dt * g.nu : 0.0, dz_c, dz_f, 3);
     for (int c = 0; c < 3; ++c) {
         if (refactor[c])
             hipLaunchKernelGGL(zfactor_kernel, dim3(1), dim3(64), 0, s, g, c, dt, theta, dz_c, dz_f,
@@ -274,21 +274,7 @@ hipError_t run_zsolve3(const Grid& g, double* const f[3], double dt, double thet
         a.f[c] = f[c];
         a.tab[c] = tab[c];
     }
-    a.dz_c = dz_c;
-    a.dz_f = dz_f;
-    a.beta = theta < 1.0 ? (1.0 - theta) * dt * g.nu : 0.0;
-    a.nb = (unsigned)(((long)g.nx * g.ny + kZScanCols - 1) / kZScanCols);
-    const dim3 grid(3 * a.nb), blk(256);
-#define SLC_ZS3(CU, CW) hipLaunchKernelGGL((zsolve3_kernel<CU, CW>), grid, blk, 0, s, g, a)
-    switch (cu) {
-        case 1: SLC_ZS3(1, 1); break;
-        case 2: if (cw == 2) SLC_ZS3(2, 2); else SLC_ZS3(2, 1); break;
-        case 4: if (cw == 4) SLC_ZS3(4, 4); else SLC_ZS3(4, 2); break;
-        case 8: if (cw == 8) SLC_ZS3(8, 8); else SLC_ZS3(8, 4); break;
-        default: if (cw == 16) SLC_ZS3(16, 16); else SLC_ZS3(16, 8);
-    }
-#undef SLC_ZS3
-    return hipGetLastError();
+    return launch_zsolve3(g, a, s);
 }
 
 // ---------------------------------------------------------------------------

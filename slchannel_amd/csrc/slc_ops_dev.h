@@ -11,6 +11,8 @@
 // within one channel) instead of reading blockIdx.
 #pragma once
 
+#include <type_traits>
+
 #include "slc_internal.h"
 
 namespace slc {
@@ -268,7 +270,7 @@ __device__ inline void zsolve_body(const Grid& g, double* __restrict__ F,
     }
 }
 
-// z-solve of the theta-method, one column per wavefront.  Lane
+// z-solve of the theta-method, a column at a time per wavefront.  Lane
 // l holds unknowns [l CH, (l+1) CH) in registers.  Forward and back
 // substitution of the shared factorisation are first-order linear
 // recurrences: each lane runs its stretch as an affine map of the value
@@ -284,22 +286,51 @@ constexpr int kZScanCols = 4;  // columns (wavefronts) per 256-thread workgroup
 
 // unknowns per lane (power of two), 0 when the column is too long for the
 // register path (n > 64 kZScanMaxCh)
-// Columns per wavefront of the ensemble's register z-solve: short columns
-// (at most 2 unknowns per lane, 128 levels) are solved four to a wavefront,
-// so that a wavefront has more than one or two 512-byte rows of loads in
-// flight (48 members of 64x48x64 .. 192x128x128: 712 -> 555 us per
-// component).  The single-run z-solve keeps one column per wavefront.
-#ifndef SLC_ZSCAN_SHORT_K
-#define SLC_ZSCAN_SHORT_K 4
-#endif
-__host__ __device__ constexpr int zscan_k(int ch) { return ch <= 2 ? SLC_ZSCAN_SHORT_K : 1; }
-
 __host__ __device__ inline int zsolve_scan_ch(int comp, int nz) {
     const int n = comp == 2 ? nz - 1 : nz;
     int ch = 1;
     while (ch * 64 < n) ch *= 2;
     return ch <= kZScanMaxCh ? ch : 0;
 }
+
+// The level distances of a lane's unknowns, with their reciprocals as pairs
+// (quotient) on lanes of up to 4: a wavefront's columns share them.
+// Correctly rounded either way; 12 general divisions a column made the
+// theta < 1 solve of 256x192x192 60 us where theta = 1 takes 31 (now 45; 256^3
+// 98 -> 61).  Longer columns' pairs would not fit the registers.
+template <int C, int CH>
+struct ZDist {
+    static constexpr bool kPairs = CH <= 4;
+    double d[CH + 1], m[CH];  // below and above the unknowns, around them
+    double dh[kPairs ? CH + 1 : 1], dl[kPairs ? CH + 1 : 1];
+    double mh[kPairs ? CH : 1], ml[kPairs ? CH : 1];
+
+    __device__ ZDist(int j0, int n, const double* __restrict__ dz_c,
+                     const double* __restrict__ dz_f) {
+#pragma unroll
+        for (int i = 0; i <= CH; ++i) {
+            const int j = j0 + i < n ? j0 + i : n;
+            d[i] = C < 2 ? dz_c[j] : dz_f[j];
+            if (kPairs) {
+                dh[i] = 1.0 / d[i];
+                dl[i] = fma(-d[i], dh[i], 1.0) * dh[i];
+            }
+            if (i == CH) break;
+            const int jm = j0 + i < n ? j0 + i : n - 1;
+            m[i] = C < 2 ? dz_f[jm] : dz_c[jm + 1];
+            if (kPairs) {
+                mh[i] = 1.0 / m[i];
+                ml[i] = fma(-m[i], mh[i], 1.0) * mh[i];
+            }
+        }
+    }
+    __device__ double by_d(double x, int i) const {
+        return kPairs ? quotient(x, d[i], dh[i], dl[i]) : x / d[i];
+    }
+    __device__ double by_m(double x, int i) const {
+        return kPairs ? quotient(x, m[i], mh[i], ml[i]) : x / m[i];
+    }
+};
 
 // Explicit part of the theta-method right-hand side, x_j + beta Dzz x_j, on
 // the lane's unknowns (the formulas and operation order of zsolve_body, from
@@ -309,8 +340,7 @@ __host__ __device__ inline int zsolve_scan_ch(int comp, int nz) {
 // face.  Neighbours across lanes come by shuffles (all lanes take part).
 template <int C, int CH>
 __device__ inline void zsolve_explicit(const Grid& g, double* p, int j0, int n, double beta,
-                                       const double* __restrict__ dz_c,
-                                       const double* __restrict__ dz_f, double s0) {
+                                       const ZDist<C, CH>& z, double s0) {
     double ext[CH + 3];  // unknowns j0-2 .. j0+CH
     ext[1] = __shfl_up(p[CH - 1], 1);
     ext[0] = CH >= 2 ? __shfl_up(p[CH >= 2 ? CH - 2 : 0], 1) : __shfl_up(p[0], 2);
@@ -321,30 +351,28 @@ __device__ inline void zsolve_explicit(const Grid& g, double* p, int j0, int n, 
     for (int i = 0; i < CH; ++i) {
         const int j = j0 + i;
         if (j >= n) continue;
-        double d2;
+        // (x / dzr - y / dzl) / dzc, the walls' cases by x and y
+        double x, y, at;
         if (C < 2) {
             const double lo = ext[i + 1], mid = ext[i + 2], hi = ext[i + 3];
-            const double dzl = dz_c[j], dzr = dz_c[j + 1], dzc = dz_f[j];
-            if (j == 0) {
-                d2 = ((hi - mid) / dzr - 2.0 * mid / dzl) / dzc;
-            } else if (j == n - 1) {
-                if (g.top_neumann) d2 = (-(mid - lo) / dzl) / dzc;
-                else d2 = (-2.0 * mid / dzr - (mid - lo) / dzl) / dzc;
-            } else {
-                d2 = ((hi - mid) / dzr - (mid - lo) / dzl) / dzc;
-            }
-            p[i] = mid + beta * d2;
+            x = hi - mid;
+            y = mid - lo;
+            if (j == 0) y = 2.0 * mid;
+            else if (j == n - 1) x = g.top_neumann ? -0.0 : -2.0 * mid;
+            at = mid;
         } else {
             // centred on face j (value b), stored to face j + 1 (value c)
             const double c = ext[i + 2];
             const double b = (j == 0) ? s0 : ext[i + 1];
             const double a = (j == 1) ? s0 : ext[i];
-            const double dzl = dz_f[j], dzr = dz_f[j + 1], dzc = dz_c[j + 1];
-            if (j == 0) d2 = ((c - b) / dzr - b / dzl) / dzc;
-            else if (j == n - 1) d2 = (-b / dzr - (b - a) / dzl) / dzc;
-            else d2 = ((c - b) / dzr - (b - a) / dzl) / dzc;
-            p[i] = c + beta * d2;
+            x = c - b;
+            y = b - a;
+            if (j == 0) y = b;
+            else if (j == n - 1) x = -b;
+            at = c;
         }
+        const double d2 = z.by_m(z.by_d(x, i + 1) - z.by_d(y, i), i);
+        p[i] = at + beta * d2;
     }
 }
 
@@ -356,191 +384,218 @@ __device__ inline void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// LDS doubles per column of the transposed z-solve (zsolve_scan_cols): one
+// LDS doubles per column of the transposed z-solve (zsolve_run): one
 // pad after every CH unknowns, so that lane-contiguous reads of CH values
 // spread over the banks.
 template <int CH>
-__host__ __device__ constexpr int zscan_lds(int K = 1) {
-    return 64 * (CH + 1) * K;
+__host__ __device__ constexpr int zscan_lds() {
+    return 64 * (CH + 1);
 }
 
-// K columns col0 .. col0 + K - 1 (those below ncols) per wavefront: the
-// loads of all K are issued before any is solved (more bytes in flight per
-// wavefront; the factor tables are shared), then each column is solved
-// exactly as a column alone.  With xlds (zscan_lds<CH>(K) doubles of the
-// wavefront's own LDS) the column moves between HBM and the registers
-// through LDS: wavefront-contiguous loads and stores (each load instruction
-// touches 512 consecutive bytes) instead of each lane reading its CH
-// consecutive unknowns (an instruction touches every cache line of the
-// column).  Same unknowns in the same registers, so the same results.
-template <int C, int CH, int K>
-__device__ inline void zsolve_scan_cols(const Grid& g, double* __restrict__ F,
-                                        const double* __restrict__ tab, long col0, long ncols,
-                                        double beta = 0.0,
-                                        const double* __restrict__ dz_c = nullptr,
-                                        const double* __restrict__ dz_f = nullptr,
-                                        double* __restrict__ xlds = nullptr) {
+// The lane's part of the factorisation and of both scans' multipliers: the
+// same for every column, so a wavefront that solves several keeps it in
+// registers.  a = 0 at unknown 0 and c = 0 at unknown n - 1 end the
+// recurrences there.
+template <int CH>
+struct ZFactor {
+    double a[CH], r[CH], c[CH];  // the three tables
+    double q[CH], t[CH];         // the affine maps' factors
+    double Q[6], T[6];           // their products before each scan step
+};
+
+template <int CH>
+__device__ inline void zfactor_load(ZFactor<CH>& z, const double* __restrict__ tab, int n,
+                                    int lane) {
+    const int j0 = lane * CH;
+    double qr = 1.0, tr = 1.0;
+#pragma unroll
+    for (int i = 0; i < CH; ++i) {
+        const int j = j0 + i, jl = j < n ? j : n - 1;
+        z.a[i] = j == 0 ? 0.0 : tab[jl];
+        z.c[i] = j == n - 1 ? 0.0 : tab[n + jl];
+        z.r[i] = tab[2 * n + jl];
+        if (j < n) qr = j == 0 ? 0.0 : -(z.a[i] * qr) * z.r[i];
+        z.q[i] = qr;
+    }
+#pragma unroll
+    for (int i = CH - 1; i >= 0; --i) {
+        const int j = j0 + i;
+        if (j < n) tr = j == n - 1 ? 0.0 : -(z.c[i] * tr);
+        z.t[i] = tr;
+    }
+#pragma unroll
+    for (int s = 0; s < 6; ++s) {
+        const int off = 1 << s;
+        z.Q[s] = qr;
+        z.T[s] = tr;
+        const double Qp = __shfl_up(qr, off), Tn = __shfl_down(tr, off);
+        if (lane >= off) qr = qr * Qp;
+        if (lane + off < 64) tr = tr * Tn;
+    }
+}
+
+struct ZNoDist {
+    __device__ ZNoDist(int, int, const double*, const double*) {}
+};
+
+// The columns col, col + stride, .. below end, one at a time, the next one's
+// loads ahead of the solve.  EXPL: theta < 1.  With X (zscan_lds<CH> doubles
+// of the wavefront's own LDS) a column moves between HBM and the registers
+// through LDS in wavefront-contiguous pieces (each load instruction touches
+// 512 consecutive bytes) instead of each lane reading its CH consecutive
+// unknowns (an instruction touches every cache line of the column).
+// The factorisation's part done once for many columns halves the arithmetic
+// and the shuffles of a column and leaves its own bytes as its only loads.
+// One column per wavefront and all of it per column: 52 us a component at
+// 256x192x192, 88 at 256^3, 707 at 512^3, 578 at 256x256x1000 (2.9, 3.1,
+// 3.0, 1.8 TB/s); so 31, 61, 427 and 226 us (4.8, 4.4, 5.0, 4.6 TB/s).
+template <int C, int CH, bool EXPL>
+__device__ inline void zsolve_run(const Grid& g, double* __restrict__ F,
+                                  const double* __restrict__ tab, unsigned col, unsigned stride,
+                                  unsigned end, double beta = 0.0,
+                                  const double* __restrict__ dz_c = nullptr,
+                                  const double* __restrict__ dz_f = nullptr,
+                                  double* __restrict__ X = nullptr) {
+    typedef double Two __attribute__((ext_vector_type(2), aligned(8)));
     const int lane = threadIdx.x & 63;
     const int n = (C == 2) ? g.nz - 1 : g.nz;
-    const double* A = tab;
-    const double* CP = tab + n;
-    const double* INV = tab + 2 * n;
     const int j0 = lane * CH;
-    double* Fc[K];
-    bool ok[K];
-    double p[K][CH], q[K][CH];
+    const unsigned ny = (unsigned)g.ny;
+    unsigned I = col / ny, J = col % ny;
+    const unsigned dI = stride / ny, dJ = stride % ny;
+    auto column = [&] {
+        return F + ((long)(I + 1) * Comp<C>::SY(g) + (J + 1)) * Comp<C>::SZ(g) + 1;
+    };
+    // raw: through LDS the wavefront's coalesced pieces of the column, else
+    // the lane's own unknowns (and the entry above the last one)
+    auto load = [&](const double* Fc, double* raw) {
+        if (X) {
 #pragma unroll
-    for (int kc = 0; kc < K; ++kc) {
-        const long col = col0 + kc;
-        ok[kc] = col < ncols;
-        const unsigned ug = (unsigned)(ok[kc] ? col : col0);
-        const int I = 1 + (int)(ug / (unsigned)g.ny), J = 1 + (int)(ug % (unsigned)g.ny);
-        Fc[kc] = F + ((long)I * Comp<C>::SY(g) + J) * Comp<C>::SZ(g) + 1;
-        if (xlds) {
-            double* X = xlds + kc * zscan_lds<CH>();
+            for (int m = 0; m < CH; ++m) raw[m] = 64 * m + lane <= n ? Fc[64 * m + lane] : 0.0;
+        } else if (CH > 1 && j0 + CH - 1 <= n) {
+#pragma unroll
+            for (int i = 0; i < CH / 2; ++i) {
+                const Two d = *reinterpret_cast<const Two*>(Fc + j0 + 2 * i);
+                raw[2 * i] = d.x;
+                raw[2 * i + 1] = d.y;
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < CH; ++i) raw[i] = j0 + i <= n ? Fc[j0 + i] : 0.0;
+        }
+    };
+    if (col >= end) return;
+    double next[CH];
+    double* Fn = column();
+    load(Fn, next);
+    double sn = EXPL ? Fn[-1] : 0.0;
+    ZFactor<CH> z;
+    zfactor_load(z, tab, n, lane);
+    const std::conditional_t<EXPL, ZDist<C, CH>, ZNoDist> dist(j0, n, dz_c, dz_f);
+#pragma unroll 1
+    while (true) {
+        double p[CH];
+        double* Fc = Fn;
+        const double s0 = sn;
+        if (X) {
 #pragma unroll
             for (int m = 0; m < CH; ++m) {
                 const int e = 64 * m + lane;
-                X[e + e / CH] = (ok[kc] && e <= n) ? Fc[kc][e] : 0.0;
+                X[e + e / CH] = next[m];
+            }
+            wave_sync();
+#pragma unroll
+            for (int i = 0; i < CH; ++i) p[i] = X[lane * (CH + 1) + i];
+            wave_sync();
+        } else {
+#pragma unroll
+            for (int i = 0; i < CH; ++i) p[i] = next[i];
+        }
+        const bool more = col + stride < end;
+        if (more) {
+            col += stride;
+            J += dJ;
+            I += dI;
+            if (J >= ny) {
+                J -= ny;
+                ++I;
+            }
+            Fn = column();
+            load(Fn, next);
+            if (EXPL) sn = Fn[-1];
+        }
+        if constexpr (EXPL) zsolve_explicit<C, CH>(g, p, j0, n, beta, dist, s0);
+        double v = 0.0;
+#pragma unroll
+        for (int i = 0; i < CH; ++i) {
+            if (j0 + i < n) v = (p[i] - z.a[i] * v) * z.r[i];
+            p[i] = v;
+        }
+#pragma unroll
+        for (int s = 0; s < 6; ++s) {
+            const double Pp = __shfl_up(v, 1 << s);
+            if (lane >= 1 << s) v = v + z.Q[s] * Pp;
+        }
+        double y = __shfl_up(v, 1);
+        if (lane == 0) y = 0.0;
+        v = 0.0;
+#pragma unroll
+        for (int i = CH - 1; i >= 0; --i) {
+            if (j0 + i < n) v = (p[i] + z.q[i] * y) - z.c[i] * v;
+            p[i] = v;
+        }
+#pragma unroll
+        for (int s = 0; s < 6; ++s) {
+            const double Rn = __shfl_down(v, 1 << s);
+            if (lane + (1 << s) < 64) v = v + z.T[s] * Rn;
+        }
+        double x = __shfl_down(v, 1);
+        if (lane == 63) x = 0.0;
+#pragma unroll
+        for (int i = 0; i < CH; ++i) p[i] = p[i] + z.t[i] * x;
+        if (X) {
+#pragma unroll
+            for (int i = 0; i < CH; ++i) X[lane * (CH + 1) + i] = p[i];
+            wave_sync();
+#pragma unroll
+            for (int m = 0; m < CH; ++m) {
+                const int e = 64 * m + lane;
+                if (e < n) Fc[e] = X[e + e / CH];
+            }
+            wave_sync();
+        } else if (CH > 1 && j0 + CH <= n) {
+#pragma unroll
+            for (int i = 0; i < CH / 2; ++i) {
+                Two d;
+                d.x = p[2 * i];
+                d.y = p[2 * i + 1];
+                *reinterpret_cast<Two*>(Fc + j0 + 2 * i) = d;
             }
         } else {
 #pragma unroll
             for (int i = 0; i < CH; ++i)
-                p[kc][i] = (ok[kc] && j0 + i <= n) ? Fc[kc][j0 + i] : 0.0;
+                if (j0 + i < n) Fc[j0 + i] = p[i];
         }
-    }
-    if (xlds) {
-        wave_sync();
-#pragma unroll
-        for (int kc = 0; kc < K; ++kc)
-#pragma unroll
-            for (int i = 0; i < CH; ++i) p[kc][i] = xlds[kc * zscan_lds<CH>() + lane * (CH + 1) + i];
-        wave_sync();
-    }
-    if (beta != 0.0) {
-#pragma unroll
-        for (int kc = 0; kc < K; ++kc)
-            zsolve_explicit<C, CH>(g, p[kc], j0, n, beta, dz_c, dz_f, ok[kc] ? Fc[kc][-1] : 0.0);
-    }
-    // forward: dp_j = p_j + q_j y with y = dp_{j0-1}
-    double P[K], Q[K];
-#pragma unroll
-    for (int kc = 0; kc < K; ++kc) {
-        double pr = 0.0, qr = 1.0;
-#pragma unroll
-        for (int i = 0; i < CH; ++i) {
-            const int j = j0 + i;
-            if (j < n) {
-                if (j == 0) {
-                    pr = p[kc][i] * INV[0];
-                    qr = 0.0;
-                } else {
-                    const double a = A[j], r = INV[j];
-                    pr = (p[kc][i] - a * pr) * r;
-                    qr = -(a * qr) * r;
-                }
-            }
-            p[kc][i] = pr;
-            q[kc][i] = qr;
-        }
-        P[kc] = pr;
-        Q[kc] = qr;
-    }
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-#pragma unroll
-        for (int kc = 0; kc < K; ++kc) {
-            const double Pp = __shfl_up(P[kc], off), Qp = __shfl_up(Q[kc], off);
-            if (lane >= off) {
-                P[kc] = P[kc] + Q[kc] * Pp;
-                Q[kc] = Q[kc] * Qp;
-            }
-        }
-    }
-#pragma unroll
-    for (int kc = 0; kc < K; ++kc) {
-        double y = __shfl_up(P[kc], 1);
-        if (lane == 0) y = 0.0;
-#pragma unroll
-        for (int i = 0; i < CH; ++i) p[kc][i] = p[kc][i] + q[kc][i] * y;
-    }
-    // backward: x_j = r_j + t_j z with z = x_{j0+CH}
-    double R[K], T[K];
-#pragma unroll
-    for (int kc = 0; kc < K; ++kc) {
-        double rr = 0.0, tr = 1.0;
-#pragma unroll
-        for (int i = CH - 1; i >= 0; --i) {
-            const int j = j0 + i;
-            if (j < n) {
-                if (j == n - 1) {
-                    rr = p[kc][i];
-                    tr = 0.0;
-                } else {
-                    const double c = CP[j];
-                    rr = p[kc][i] - c * rr;
-                    tr = -(c * tr);
-                }
-            }
-            p[kc][i] = rr;
-            q[kc][i] = tr;
-        }
-        R[kc] = rr;
-        T[kc] = tr;
-    }
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-#pragma unroll
-        for (int kc = 0; kc < K; ++kc) {
-            const double Rn = __shfl_down(R[kc], off), Tn = __shfl_down(T[kc], off);
-            if (lane + off < 64) {
-                R[kc] = R[kc] + T[kc] * Rn;
-                T[kc] = T[kc] * Tn;
-            }
-        }
-    }
-#pragma unroll
-    for (int kc = 0; kc < K; ++kc) {
-        double z = __shfl_down(R[kc], 1);
-        if (lane == 63) z = 0.0;
-        if (xlds) {
-            double* X = xlds + kc * zscan_lds<CH>();
-#pragma unroll
-            for (int i = 0; i < CH; ++i) X[lane * (CH + 1) + i] = p[kc][i] + q[kc][i] * z;
-            continue;
-        }
-        if (!ok[kc]) continue;
-#pragma unroll
-        for (int i = 0; i < CH; ++i)
-            if (j0 + i < n) Fc[kc][j0 + i] = p[kc][i] + q[kc][i] * z;
-    }
-    if (xlds) {
-        wave_sync();
-#pragma unroll
-        for (int kc = 0; kc < K; ++kc) {
-            if (!ok[kc]) continue;
-            const double* X = xlds + kc * zscan_lds<CH>();
-#pragma unroll
-            for (int m = 0; m < CH; ++m) {
-                const int e = 64 * m + lane;
-                if (e < n) Fc[kc][e] = X[e + e / CH];
-            }
-        }
+        if (!more) break;
     }
 }
 
-// Runtime CH dispatch (ch from zsolve_scan_ch), theta = 1: the zscan_k(ch)
-// columns col0 .. of one wavefront (those below ncols).
-template <int C>
-__device__ inline void zsolve_scan_any(const Grid& g, double* __restrict__ F,
-                                       const double* __restrict__ tab, long col0, long ncols,
-                                       int ch) {
+// Runtime dispatch of ch (from zsolve_scan_ch, at most MAXCH), theta = 1.
+template <int C, int MAXCH>
+__device__ inline void zsolve_run_any(const Grid& g, double* __restrict__ F,
+                                      const double* __restrict__ tab, unsigned col,
+                                      unsigned stride, unsigned end, int ch) {
     switch (ch) {
-        case 1: zsolve_scan_cols<C, 1, zscan_k(1)>(g, F, tab, col0, ncols); break;
-        case 2: zsolve_scan_cols<C, 2, zscan_k(2)>(g, F, tab, col0, ncols); break;
-        case 4: zsolve_scan_cols<C, 4, zscan_k(4)>(g, F, tab, col0, ncols); break;
-        case 8: zsolve_scan_cols<C, 8, zscan_k(8)>(g, F, tab, col0, ncols); break;
-        default: zsolve_scan_cols<C, 16, zscan_k(16)>(g, F, tab, col0, ncols); break;
+        case 1: zsolve_run<C, 1, false>(g, F, tab, col, stride, end); break;
+        case 2: zsolve_run<C, 2, false>(g, F, tab, col, stride, end); break;
+        case 4:
+            if constexpr (MAXCH >= 4) zsolve_run<C, 4, false>(g, F, tab, col, stride, end);
+            break;
+        case 8:
+            if constexpr (MAXCH >= 8) zsolve_run<C, 8, false>(g, F, tab, col, stride, end);
+            break;
+        default:
+            if constexpr (MAXCH >= 16) zsolve_run<C, 16, false>(g, F, tab, col, stride, end);
     }
 }
 
