@@ -454,9 +454,9 @@ int slc_departure(slc_plan* p, int comp, const double* um, const double* vm, con
     if (layout != 0 && layout != 1) return fail(SLC_EINVAL, "layout must be 0 or 1");
     if (!um || !vm || !wm || !xd || !yd || !zd) return fail(SLC_EINVAL, "null array");
     DeviceGuard dg(p->device);
-    TrajVel V{{um, vm, wm}, {nullptr, nullptr, nullptr}};
+    const double* const a[3] = {um, vm, wm};
     Timed t(p, kLabel[comp][5], stream);
-    HIP_OK(run_departure(p->g, comp, V, layout, dt, xd, yd, zd,
+    HIP_OK(run_departure(p->g, comp, p->at[comp], a, layout, dt, xd, yd, zd,
                          reinterpret_cast<unsigned long long*>(nclamp), S(stream)));
     return SLC_OK;
 }

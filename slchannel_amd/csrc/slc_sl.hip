@@ -20,6 +20,7 @@
 // 64-bit atomic per block.
 #include "slc_device.h"
 #include "slc_internal.h"
+#include "slc_tile.h"
 
 namespace slc {
 
@@ -35,11 +36,11 @@ __device__ inline void block_count(unsigned long long* counter, int mine) {
     if (threadIdx.x == 0 && s_cnt) atomicAdd(counter, (unsigned long long)s_cnt);
 }
 
-// TV: TrajVel (ghost-shaped trajectory fields) or TrajNodes (packed node
-// buffers).  With nclamp the stored z is clamped into [z_lo, z_hi] and the
+// Tricubic trajectories (the trilinear ones: feet_kernel).  TV: TrajA
+// (ghost-shaped trajectory fields) or TrajNodes (packed node buffers).  With nclamp the stored z is clamped into [z_lo, z_hi] and the
 // clamped feet are counted (TritonSL.departure, semilag_triton.py:262-269);
 // without it z is stored unclamped (departure_coords, semilag.py:534-552).
-template <int C, int T, typename TV>
+template <int C, typename TV>
 __global__ __launch_bounds__(kBlock) void departure_kernel(Grid g, TV V, double dt,
                                                            double* __restrict__ xd,
                                                            double* __restrict__ yd,
@@ -53,7 +54,7 @@ __global__ __launch_bounds__(kBlock) void departure_kernel(Grid g, TV V, double 
         int I, J, K;
         arrival<C>(g, n, xa, ya, za, I, J, K);
         double x, y, z;
-        foot<T, TV>(g, V, xa, ya, za, 0.5 * dt, x, y, z);
+        foot<4, TV>(g, V, xa, ya, za, 0.5 * dt, x, y, z);
         if (nclamp) {
             clamped = (z < g.z_lo || z > g.z_hi) ? 1 : 0;
             z = clampd(z, g.z_lo, g.z_hi);
@@ -61,6 +62,39 @@ __global__ __launch_bounds__(kBlock) void departure_kernel(Grid g, TV V, double 
         xd[n] = x;
         yd[n] = y;
         zd[n] = z;
+    }
+    if (nclamp) block_count(nclamp, clamped);
+}
+
+// The same with trilinear trajectories, sampled as the step kernels do
+// (sample3: one round of loads a sample, 32-bit addresses): the same doubles.
+// A wavefront's points run along z, so its corner loads are contiguous.
+// 161x128x97 (2 M points): 78-87 -> 47-51 us a component.
+template <int C, bool BIG, typename TV>
+__global__ __launch_bounds__(kBlock) void feet_kernel(Grid g, ArrivalTabs A, TV V, double dt,
+                                                      double* __restrict__ xd,
+                                                      double* __restrict__ yd,
+                                                      double* __restrict__ zd, unsigned N,
+                                                      unsigned long long* nclamp) {
+    const unsigned n = (unsigned)xcd_block(gridDim.x) * kBlock + threadIdx.x;
+    int clamped = 0;
+    if (n < N) {
+        const unsigned nzi = (unsigned)Comp<C>::NZI(g), col = n / nzi;
+        const int k = (int)(n - col * nzi);
+        const int i = (int)(col / (unsigned)g.ny), j = (int)(col - (unsigned)i * (unsigned)g.ny);
+        double xa, ya, za, x, y, z, u0, v0, w0;
+        arrival_at<C>(g, i, j, k, xa, ya, za);
+        const int csel = A.csel[k], c = csel >> 1;
+        sample3_at<BIG>(g, V, over_dx(g, xa), over_dy(g, ya), clampd(za, g.z_lo, g.z_hi), c,
+                        c + (csel & 1), u0, v0, w0);
+        trace_foot<C, BIG>(g, V, xa, ya, za, k + 1, u0, v0, w0, 0.5 * dt, x, y, z);
+        if (nclamp) {
+            clamped = (z < g.z_lo || z > g.z_hi) ? 1 : 0;
+            z = clampd(z, g.z_lo, g.z_hi);
+        }
+        *elem<BIG>(xd, n) = x;
+        *elem<BIG>(yd, n) = y;
+        *elem<BIG>(zd, n) = z;
     }
     if (nclamp) block_count(nclamp, clamped);
 }
@@ -302,32 +336,37 @@ static inline dim3 grid_for(long N) { return dim3((unsigned)((N + kBlock - 1) / 
     }
 
 template <int C, typename TV>
-static void launch_departure_tv(const Grid& g, const TV& V, double dt, double* xd, double* yd,
-                                double* zd, unsigned long long* ncl, hipStream_t s) {
+static void launch_departure_tv(const Grid& g, const ArrivalTabs& A, const TV& V, double dt,
+                                double* xd, double* yd, double* zd, unsigned long long* ncl,
+                                hipStream_t s) {
     long N = n_arrival(g, C);
     if (N <= 0) return;
     if (g.traj_order == 4)
-        hipLaunchKernelGGL((departure_kernel<C, 4, TV>), grid_for(N), dim3(kBlock), 0, s, g, V,
-                           dt, xd, yd, zd, N, ncl);
+        hipLaunchKernelGGL((departure_kernel<C, TV>), grid_for(N), dim3(kBlock), 0, s, g, V, dt, xd,
+                           yd, zd, N, ncl);
+    else if (big_index(g))
+        hipLaunchKernelGGL((feet_kernel<C, true, TV>), grid_for(N), dim3(kBlock), 0, s, g, A, V, dt,
+                           xd, yd, zd, (unsigned)N, ncl);
     else
-        hipLaunchKernelGGL((departure_kernel<C, 2, TV>), grid_for(N), dim3(kBlock), 0, s, g, V,
-                           dt, xd, yd, zd, N, ncl);
+        hipLaunchKernelGGL((feet_kernel<C, false, TV>), grid_for(N), dim3(kBlock), 0, s, g, A, V,
+                           dt, xd, yd, zd, (unsigned)N, ncl);
 }
 
 template <int C>
-static void launch_departure(const Grid& g, const TrajVel& V, int layout, double dt, double* xd,
-                             double* yd, double* zd, unsigned long long* ncl, hipStream_t s) {
+static void launch_departure(const Grid& g, const ArrivalTabs& A, const double* const a[3],
+                             int layout, double dt, double* xd, double* yd, double* zd,
+                             unsigned long long* ncl, hipStream_t s) {
     if (layout == 1)
-        launch_departure_tv<C, TrajNodes>(g, TrajNodes{{V.a[0], V.a[1], V.a[2]}}, dt, xd, yd, zd,
-                                          ncl, s);
+        launch_departure_tv<C, TrajNodes>(g, A, TrajNodes{{a[0], a[1], a[2]}}, dt, xd, yd, zd, ncl,
+                                          s);
     else
-        launch_departure_tv<C, TrajVel>(g, V, dt, xd, yd, zd, ncl, s);
+        launch_departure_tv<C, TrajA>(g, A, TrajA{{a[0], a[1], a[2]}}, dt, xd, yd, zd, ncl, s);
 }
 
-hipError_t run_departure(const Grid& g, int comp, const TrajVel& V, int layout, double dt,
-                         double* xd, double* yd, double* zd, unsigned long long* ncl,
-                         hipStream_t s) {
-    SLC_DISPATCH_C(comp, launch_departure, g, V, layout, dt, xd, yd, zd, ncl, s);
+hipError_t run_departure(const Grid& g, int comp, const ArrivalTabs& A, const double* const a[3],
+                         int layout, double dt, double* xd, double* yd, double* zd,
+                         unsigned long long* ncl, hipStream_t s) {
+    SLC_DISPATCH_C(comp, launch_departure, g, A, a, layout, dt, xd, yd, zd, ncl, s);
     return hipGetLastError();
 }
 

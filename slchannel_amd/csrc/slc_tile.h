@@ -210,12 +210,14 @@ __device__ inline XYCells xy_cells(const Grid& g, double xdx, double ydy) {
 // The eight corner values of component C's trilinear cell: (i, j) columns,
 // levels k0, k0 + 1.  Without BIG the indices and strides are below 2^24
 // (big_index), so the products are full-rate 24-bit ones (a 32-bit product
-// takes four times as long).
-template <int C, bool BIG>
+// takes four times as long).  PACKED: a (nx, ny, levels) node buffer.
+template <int C, bool BIG, bool PACKED>
 __device__ inline void cell_cols(const Grid& g, const double* F, const Cell& x, const Cell& y,
                                  int k0, Pair (&v)[2][2]) {
-    const unsigned SZ = (unsigned)Comp<C>::SZ(g), PS = (unsigned)Comp<C>::SY(g) * SZ;
-    const double* base = F + ((size_t)Comp<C>::ox * PS + (size_t)Comp<C>::oy * SZ);
+    const unsigned SZ = (unsigned)Comp<C>::SZ(g);
+    const unsigned PS = (unsigned)(PACKED ? g.ny : Comp<C>::SY(g)) * SZ;
+    const double* base =
+        PACKED ? F : F + ((size_t)Comp<C>::ox * PS + (size_t)Comp<C>::oy * SZ);
     auto mul = [](int a, unsigned b) { return BIG ? (unsigned)a * b : __umul24((unsigned)a, b); };
     const unsigned x0 = mul(x.i0, PS), x1 = mul(x.i1, PS);
     const unsigned y0 = mul(y.i0, SZ) + (unsigned)k0, y1 = mul(y.i1, SZ) + (unsigned)k0;
@@ -247,18 +249,18 @@ __device__ inline double cell_sum(const Cell& x, const Cell& y, const double (&w
 // Trajectory samples of the three U* components at (xdx, ydy) = (x/dx, y/dy)
 // and the clamped z, whose face interval c and centre node interval m are
 // known (semilag.py:512-528 recomputes them per component with identical
-// results).
-template <bool BIG>
-__device__ inline void sample3_at(const Grid& g, const TrajA& V, double xdx, double ydy,
+// results).  TV: TrajA or TrajNodes.
+template <bool BIG, typename TV>
+__device__ inline void sample3_at(const Grid& g, const TV& V, double xdx, double ydy,
                                   double zc, int c, int m, double& us, double& vs, double& ws) {
     const XYCells q = xy_cells(g, xdx, ydy);
     const Pair nf = pair_at<false>(g.z_f, (unsigned)c), nc = pair_at<false>(g.z_c, (unsigned)m);
     const Pair pc = pair_at<false>(g.dinv_c2, 2u * (unsigned)m);
     const Pair pf = pair_at<false>(g.dinv_f2, 2u * (unsigned)c);
     Pair uv[2][2], vv[2][2], wv[2][2];
-    cell_cols<0, BIG>(g, V.a[0], q.xf, q.yc, m, uv);
-    cell_cols<1, BIG>(g, V.a[1], q.xc, q.yf, m, vv);
-    cell_cols<2, BIG>(g, V.a[2], q.xc, q.yc, c, wv);
+    cell_cols<0, BIG, TV::packed>(g, V.a[0], q.xf, q.yc, m, uv);
+    cell_cols<1, BIG, TV::packed>(g, V.a[1], q.xc, q.yf, m, vv);
+    cell_cols<2, BIG, TV::packed>(g, V.a[2], q.xc, q.yc, c, wv);
     const double wzc[2] = {(zc - nc.b) * pc.a, (zc - nc.a) * pc.b};
     const double wzf[2] = {(zc - nf.b) * pf.a, (zc - nf.a) * pf.b};
     us = cell_sum(q.xf, q.yc, wzc, uv);
@@ -283,8 +285,8 @@ __device__ inline void sample3_at(const Grid& g, const TrajA& V, double xdx, dou
 // production grids) c and m are located as face_cell_fast does and the values
 // read again.  Either way the sums are the same operations on the same
 // values as with a located interval.
-template <int C, bool BIG>
-__device__ inline void sample3(const Grid& g, const TrajA& V, double x, double y, double z,
+template <int C, bool BIG, typename TV>
+__device__ inline void sample3(const Grid& g, const TV& V, double x, double y, double z,
                                double za, int K, double& us, double& vs, double& ws) {
     const double zc = clampd(z, g.z_lo, g.z_hi);
     const XYCells q = xy_cells(g, over_dx(g, x), over_dy(g, y));
@@ -300,9 +302,9 @@ __device__ inline void sample3(const Grid& g, const TrajA& V, double x, double y
         const Pair pc = pair_at<false>(g.dinv_c2, 2u * (unsigned)m);
         const Pair pf = pair_at<false>(g.dinv_f2, 2u * (unsigned)c);
         Pair uv[2][2], vv[2][2], wv[2][2];
-        cell_cols<0, BIG>(g, V.a[0], q.xf, q.yc, m, uv);
-        cell_cols<1, BIG>(g, V.a[1], q.xc, q.yf, m, vv);
-        cell_cols<2, BIG>(g, V.a[2], q.xc, q.yc, c, wv);
+        cell_cols<0, BIG, TV::packed>(g, V.a[0], q.xf, q.yc, m, uv);
+        cell_cols<1, BIG, TV::packed>(g, V.a[1], q.xc, q.yf, m, vv);
+        cell_cols<2, BIG, TV::packed>(g, V.a[2], q.xc, q.yc, c, wv);
         const double split = m > c ? nc.a : nc.b;  // z_c[c + 1]
         if (located || (face_estimate_holds(g, c, zc, nf.a, nf.b) && (zc >= split) == (m > c))) {
             const double wzc[2] = {(zc - nc.b) * pc.a, (zc - nc.a) * pc.b};
@@ -735,15 +737,15 @@ __device__ inline void box_add(SBox& l, const FootSt& f) {
 
 // Iterated midpoint (semilag.py:534-552) from the arrival point with its
 // shared first sample (u0, v0, w0); returns the unclamped foot.
-template <int C, bool BIG>
-__device__ inline void trace_foot(const Grid& g, const TrajA& V, double xa, double ya,
+template <int C, bool BIG, typename TV>
+__device__ inline void trace_foot(const Grid& g, const TV& V, double xa, double ya,
                                   double za, int K, double u0, double v0, double w0, double h,
                                   double& x, double& y, double& z) {
     double xm = xa - h * u0, ym = ya - h * v0;
     double zm = clampd(za - h * w0, g.z_lo, g.z_hi);
     for (int it = 1; it < g.n_iters; ++it) {
         double us, vs, ws;
-        sample3<C, BIG>(g, V, xm, ym, zm, za, K, us, vs, ws);
+        sample3<C, BIG, TV>(g, V, xm, ym, zm, za, K, us, vs, ws);
         xm = xa - h * us;
         ym = ya - h * vs;
         zm = clampd(za - h * ws, g.z_lo, g.z_hi);
