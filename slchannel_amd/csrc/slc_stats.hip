@@ -1,24 +1,32 @@
 // slc_stats.hip -- on-device turbulence statistics (include/slc_stats.h).
 //
 // One snapshot of TurbulenceStats.accumulate_statistics
-// (slchannel/turbstats.py:156-361) as five small launches plus, with
-// spectra planes, three more:
+// (slchannel/turbstats.py:156-361) as four launches plus, with spectra
+// planes, two more:
 //
-//   pass 1   plane sums of the cell-centred u, v, w and of the u / v nodes
-//            and w faces, per z level, as column-chunk partials;
-//   reduce   partials -> plane means (fixed order);
-//   pass 2   sums of squared node / face fluctuations about those means and
-//            of the cell-centred u'w' product;
-//   reduce   partials -> per-snapshot moments;
-//   update   running sums += this snapshot's profiles (w'w' faces averaged
+//   shift    a provisional mean of u, v and w per z level, from 64 columns;
+//   pass     sums of the cell-centred u and v, of the u / v nodes and w
+//            faces and of their squares, and of the cell-centred u w, all of
+//            values less the provisional means, per z level, as column-chunk
+//            partials, and the planes of the spectra pairs into a contiguous
+//            batch;
+//   reduce   partials -> plane averages (fixed order);
+//   final    means and central moments of the averages (the squares' average
+//            less the square of the average of the same shifted values),
+//            running sums += this snapshot's profiles (w'w' faces averaged
 //            to centres, turbstats.py:229-231);
-//   planes   fluctuation planes of the spectra pairs into a contiguous batch;
 //   rocFFT   batched real-forward 2-D transforms (torch.fft.rfft2 layout);
 //   fold     auto / cross spectra, both walls averaged, folded onto
 //            kx > 0, ky > 0, added to the running sums
 //            (turbstats.py:256-351).
 //
-// Layout of the passes: a workgroup is 64 z lanes x 4 column groups.  The z
+// One read of the fields in place of two (a pass of means, then one of
+// fluctuations about them; 86 + 82 us at 256^3, each at the rate of memory).
+// The shift keeps the precision: the shifted values are of the size of the
+// fluctuations, and what the last subtraction loses is the square of the
+// provisional mean's error, a fraction of the variance.
+//
+// Layout of the pass: a workgroup is 64 z lanes x 4 column groups.  The z
 // lanes make every load a coalesced 512-byte row segment; each thread walks
 // an x-run of 16 cells for 4 y-rows, carrying the previous u face in a
 // register so the cell-centred u costs one load.  Partials go to
@@ -40,23 +48,66 @@ constexpr int kLanes = 64;  // z lanes per workgroup
 constexpr int kSub = 4;     // column groups per workgroup
 constexpr int kIB = 16;     // x cells per thread run
 constexpr int kJB = 16;     // y rows per workgroup (kJB / kSub per thread)
-constexpr int kNQ1 = 6;     // pass-1 sums: ucc, vcc, wcc, u node, v node, w face
-constexpr int kNQ2 = 4;     // pass-2 sums: u'u' node, v'v' node, w'w' face, u'w' centre
+constexpr int kSide = 8;    // shift: kSide x kSide columns
+// sums of shifted values: u, v at centres; u node and square; v node and
+// square; w face and square; u w at centres
+enum { kUc = 0, kVc, kUn, kUU, kVn, kVV, kWf, kWW, kUW, kNQ };
 
 struct Dims {
     int nx, ny, nz, nbx, nby;
 };
 
+// shift[c * (nz + 1) + k]: the average of component c at level k (w: face k)
+// over kSide x kSide columns spread over the plane.
+constexpr int kRSub = 16;
+
+__global__ __launch_bounds__(kLanes * kRSub) void stats_shift_kernel(
+    Dims d, const double* __restrict__ u, const double* __restrict__ v,
+    const double* __restrict__ w, double* __restrict__ shift) {
+    __shared__ double red[3][kRSub][kLanes];
+    const int lane = threadIdx.x % kLanes, sub = threadIdx.x / kLanes;
+    const int k = blockIdx.x * kLanes + lane, nz = d.nz;
+    constexpr int kPer = kSide * kSide / kRSub;
+    double s[3] = {0.0, 0.0, 0.0};
+    if (k <= nz) {
+#pragma unroll
+        for (int t = 0; t < kPer; ++t) {
+            const int c = sub * kPer + t;
+            const size_t I = (size_t)((long)(c / kSide) * d.nx / kSide) + 1;
+            const size_t J = (size_t)((long)(c % kSide) * d.ny / kSide) + 1;
+            if (k < nz) {
+                s[0] += u[(I * (d.ny + 2) + J) * (nz + 2) + k + 1];
+                s[1] += v[(I * (d.ny + 1) + J) * (nz + 2) + k + 1];
+            }
+            s[2] += w[(I * (d.ny + 2) + J) * (nz + 1) + k];
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < 3; ++q) red[q][sub][lane] = s[q];
+    __syncthreads();
+    if (sub < 3 && k <= nz) {
+        double t = red[sub][0][lane];
+        for (int g = 1; g < kRSub; ++g) t += red[sub][g][lane];
+        shift[sub * (nz + 1) + k] = t * (1.0 / (kSide * kSide));
+    }
+}
+
 // Plane sums over one workgroup's columns for z lane k (0..nz-1); lane
-// nz-1 also sums the top w face (index nz), which it loads anyway.  mean:
-// pass-1 means, (6, nz + 1).
-template <int PASS>
+// nz-1 also sums the top w face (index nz), which it loads anyway.
+//
+// Lanes at a level of a spectra pair also write its planes, batch index
+// 6 * pair + c: c = 0, 1, 2 bottom u node, v node, cell-centred w; 3, 4, 5
+// the same at the top with w negated (turbstats.py:256-276).  Planes are
+// (nx, ny), y fastest, of the shifted values: what those lack to the
+// fluctuations is a constant, which only the mean mode sees, and no spectrum
+// holds it (kx > 0, ky > 0).  Read back from the fields, a level at a time,
+// the planes of 4 pairs cost 37 us at 256^3 (a cache line per value).
 __global__ __launch_bounds__(kLanes * kSub) void stats_pass_kernel(
     Dims d, const double* __restrict__ u, const double* __restrict__ v,
-    const double* __restrict__ w, const double* __restrict__ mean, double* __restrict__ part) {
-    constexpr int NQ = PASS == 1 ? kNQ1 : kNQ2;
-    __shared__ double red[kSub][NQ][kLanes];
-    __shared__ double red_top[kSub];
+    const double* __restrict__ w, const double* __restrict__ shift, double* __restrict__ part,
+    const int* __restrict__ kp, int nsides, double* __restrict__ planes) {
+    __shared__ double red[kSub][kNQ][kLanes];
+    __shared__ double red_top[2][kSub];
     const int lane = threadIdx.x % kLanes, sub = threadIdx.x / kLanes;
     const int k = blockIdx.x * kLanes + lane;
     const int nx = d.nx, ny = d.ny, nz = d.nz, nzf = nz + 1;
@@ -64,80 +115,86 @@ __global__ __launch_bounds__(kLanes * kSub) void stats_pass_kernel(
     const int j0 = blockIdx.z * kJB, j1 = min(ny, j0 + kJB);
     const size_t su = (size_t)(ny + 2) * (nz + 2), sv = (size_t)(ny + 1) * (nz + 2),
                  sw = (size_t)(ny + 2) * (nz + 1);
-    double s[NQ];
+    double s[kNQ];
 #pragma unroll
-    for (int q = 0; q < NQ; ++q) s[q] = 0.0;
-    double top = 0.0;  // lane nz-1: sums of the top face
-    double mun = 0.0, mvn = 0.0, mwf = 0.0, mU = 0.0, mW = 0.0, mwt = 0.0;
-    if (PASS == 2 && k < nz) {
-        mwf = mean[5 * nzf + k];
-        mU = mean[0 * nzf + k];
-        mW = mean[2 * nzf + k];
-        mun = mean[3 * nzf + k];
-        mvn = mean[4 * nzf + k];
-        if (k == nz - 1) mwt = mean[5 * nzf + nz];
+    for (int q = 0; q < kNQ; ++q) s[q] = 0.0;
+    double top = 0.0, top2 = 0.0;  // lane nz-1: sums of the top face
+    double pu = 0.0, pv = 0.0, pw = 0.0, pt = 0.0;
+    if (k < nz) {
+        pu = shift[k];
+        pv = shift[nzf + k];
+        pw = shift[2 * nzf + k];
+        pt = shift[2 * nzf + k + 1];
     }
+    // sides whose plane is this level: bits of the first 64
+    unsigned long long sides = 0ull;
+    for (int q = 0; q < min(nsides, 64); ++q)
+        if (kp[q] - 1 == k) sides |= 1ull << q;
+    const size_t plane = (size_t)nx * ny;
     for (int j = j0 + sub; j < j1; j += kSub) {
         // u[i0, j+1, k+1], v[i0+1, j, k+1], w[i0+1, j+1, k]
         const double* ur = u + ((size_t)i0 * (ny + 2) + (j + 1)) * (nz + 2) + (k + 1);
         const double* vr = v + ((size_t)(i0 + 1) * (ny + 1) + j) * (nz + 2) + (k + 1);
         const double* wr = w + ((size_t)(i0 + 1) * (ny + 2) + (j + 1)) * (nz + 1) + k;
         if (k < nz) {
-            double up = ur[0];
+            double up = ur[0] - pu;
             for (int i = i0; i < i1; ++i) {
                 const size_t o = (size_t)(i - i0);
-                const double un = ur[(o + 1) * su];
-                const double v0 = vr[o * sv], v1 = vr[o * sv + (nz + 2)];
-                const double w0 = wr[o * sw], w1 = wr[o * sw + 1];
+                const double un = ur[(o + 1) * su] - pu;
+                const double v0 = vr[o * sv] - pv, v1 = vr[o * sv + (nz + 2)] - pv;
+                const double w0 = wr[o * sw] - pw, w1 = wr[o * sw + 1] - pt;
                 const double ucc = 0.5 * (up + un);
-                const double wcc = 0.5 * (w0 + w1);
-                if (PASS == 1) {
-                    s[0] += ucc;
-                    s[1] += 0.5 * (v0 + v1);
-                    s[2] += wcc;
-                    s[3] += un;
-                    s[4] += v1;
-                    s[5] += w0;
-                } else {
-                    const double du = un - mun, dv = v1 - mvn, dw = w0 - mwf;
-                    s[0] += du * du;
-                    s[1] += dv * dv;
-                    s[2] += dw * dw;
-                    s[3] += (ucc - mU) * (wcc - mW);
-                }
+                s[kUc] += ucc;
+                s[kVc] += 0.5 * (v0 + v1);
+                s[kUn] += un;
+                s[kUU] += un * un;
+                s[kVn] += v1;
+                s[kVV] += v1 * v1;
+                s[kWf] += w0;
+                s[kWW] += w0 * w0;
+                s[kUW] += ucc * (0.5 * (w0 + w1));
                 if (k == nz - 1) {
-                    if (PASS == 1) {
-                        top += w1;
-                    } else {
-                        const double dt = w1 - mwt;
-                        top += dt * dt;
-                    }
+                    top += w1;
+                    top2 += w1 * w1;
                 }
+                auto put = [&](int side) {
+                    double* o3 = planes + (size_t)side * 3 * plane + ((size_t)i * ny + j);
+                    o3[0] = un;
+                    o3[plane] = v1;
+                    o3[2 * plane] = (side & 1) ? -(0.5 * (w0 + w1)) : 0.5 * (w0 + w1);
+                };
+                for (unsigned long long m = sides; m; m &= m - 1) put(__ffsll(m) - 1);
+                for (int q = 64; q < nsides; ++q)
+                    if (kp[q] - 1 == k) put(q);
                 up = un;
             }
         }
     }
 #pragma unroll
-    for (int q = 0; q < NQ; ++q) red[sub][q][lane] = s[q];
-    if (k == nz - 1) red_top[sub] = top;
+    for (int q = 0; q < kNQ; ++q) red[sub][q][lane] = s[q];
+    if (k == nz - 1) {
+        red_top[0][sub] = top;
+        red_top[1][sub] = top2;
+    }
     __syncthreads();
     if (sub == 0 && k < nz) {
         const size_t chunk = (size_t)blockIdx.z * d.nbx + blockIdx.y;
 #pragma unroll
-        for (int q = 0; q < NQ; ++q) {
+        for (int q = 0; q < kNQ; ++q) {
             double r = red[0][q][lane];
 #pragma unroll
             for (int t = 1; t < kSub; ++t) r += red[t][q][lane];
-            part[(chunk * NQ + q) * nzf + k] = r;
+            part[(chunk * kNQ + q) * nzf + k] = r;
         }
         if (k == nz - 1) {
-            double r = red_top[0];
-            for (int t = 1; t < kSub; ++t) r += red_top[t];
-            // the top face is quantity 5 (w face) in pass 1, 2 (w'w' face) in
-            // pass 2; the other quantities have no entry there (zero)
-            constexpr int QT = PASS == 1 ? 5 : 2;
+            // the other quantities have no entry at the top face (zero)
 #pragma unroll
-            for (int q = 0; q < NQ; ++q) part[(chunk * NQ + q) * nzf + nz] = q == QT ? r : 0.0;
+            for (int q = 0; q < kNQ; ++q) {
+                double r = 0.0;
+                if (q == kWf || q == kWW)
+                    for (int t = 0; t < kSub; ++t) r += red_top[q == kWW][t];
+                part[(chunk * kNQ + q) * nzf + nz] = r;
+            }
         }
     }
 }
@@ -145,17 +202,15 @@ __global__ __launch_bounds__(kLanes * kSub) void stats_pass_kernel(
 // Sums the partials of quantity q = blockIdx.y at lane k in chunk order
 // (column group t of kRSub takes chunks t, t + kRSub, ...; groups combined in
 // order) and divides by the plane size: out[q * (nz + 1) + k].
-constexpr int kRSub = 16;
-
 __global__ __launch_bounds__(kLanes * kRSub) void stats_reduce_kernel(
-    const double* __restrict__ part, int nchunks, int NQ, int nz, double plane,
+    const double* __restrict__ part, int nchunks, int nz, double plane,
     double* __restrict__ out) {
     __shared__ double red[kRSub][kLanes];
     const int lane = threadIdx.x % kLanes, sub = threadIdx.x / kLanes;
     const int k = blockIdx.x * kLanes + lane, q = blockIdx.y, nzf = nz + 1;
     double r = 0.0;
     if (k <= nz)
-        for (int c = sub; c < nchunks; c += kRSub) r += part[((size_t)c * NQ + q) * nzf + k];
+        for (int c = sub; c < nchunks; c += kRSub) r += part[((size_t)c * kNQ + q) * nzf + k];
     red[sub][lane] = r;
     __syncthreads();
     if (sub == 0 && k <= nz) {
@@ -165,18 +220,29 @@ __global__ __launch_bounds__(kLanes * kRSub) void stats_reduce_kernel(
     }
 }
 
-// Running sums += this snapshot (turbstats.py:177, 195-200, 239-242).
-__global__ __launch_bounds__(256) void stats_update_kernel(int nz, const double* __restrict__ mean,
-                                                            const double* __restrict__ mom,
-                                                            double* __restrict__ prof) {
+// Means and central moments from the shifted averages; running sums += this
+// snapshot (turbstats.py:177, 195-200, 239-242).
+__global__ __launch_bounds__(256) void stats_final_kernel(int nz, const double* __restrict__ avg,
+                                                           const double* __restrict__ shift,
+                                                           double* __restrict__ prof) {
     const int nzf = nz + 1;
+    // a variance of rounding size may come out below zero
+    auto var = [&](int sq, int av, int k) {
+        const double m = avg[av * nzf + k], x = avg[sq * nzf + k] - m * m;
+        return x < 0.0 ? 0.0 : x;
+    };
     for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < nz; k += gridDim.x * blockDim.x) {
-        const double U = mean[0 * nzf + k], V = mean[1 * nzf + k], W = mean[2 * nzf + k];
+        const double pu = shift[k], pv = shift[nzf + k];
+        const double pw = shift[2 * nzf + k], pt = shift[2 * nzf + k + 1];
+        const double dU = avg[kUc * nzf + k];
+        const double dw = avg[kWf * nzf + k], dt = avg[kWf * nzf + k + 1];
+        const double U = pu + dU, V = pv + avg[kVc * nzf + k];
+        const double W = 0.5 * ((pw + dw) + (pt + dt));
         prof[0 * nz + k] += U;
-        prof[1 * nz + k] += mom[0 * nzf + k];
-        prof[2 * nz + k] += mom[1 * nzf + k];
-        prof[3 * nz + k] += 0.5 * (mom[2 * nzf + k] + mom[2 * nzf + k + 1]);
-        prof[4 * nz + k] += mom[3 * nzf + k];
+        prof[1 * nz + k] += var(kUU, kUn, k);
+        prof[2 * nz + k] += var(kVV, kVn, k);
+        prof[3 * nz + k] += 0.5 * (var(kWW, kWf, k) + var(kWW, kWf, k + 1));
+        prof[4 * nz + k] += avg[kUW * nzf + k] - dU * (0.5 * (dw + dt));
         prof[5 * nz + k] += V;
         prof[6 * nz + k] += W;
         prof[7 * nz + k] += U * U;
@@ -184,34 +250,6 @@ __global__ __launch_bounds__(256) void stats_update_kernel(int nz, const double*
         prof[9 * nz + k] += W * W;
         prof[10 * nz + k] += U * W;
     }
-}
-
-// Fluctuation planes of the spectra pairs, batch index 6 * pair + c:
-// c = 0, 1, 2 bottom u node, v node, cell-centred w; 3, 4, 5 the same at
-// the top with w negated (turbstats.py:256-276).  Planes are (nx, ny), y
-// fastest.
-__global__ __launch_bounds__(256) void stats_planes_kernel(
-    Dims d, const double* __restrict__ u, const double* __restrict__ v,
-    const double* __restrict__ w, const double* __restrict__ mean, const int* __restrict__ kp,
-    double* __restrict__ planes) {
-    const int nx = d.nx, ny = d.ny, nz = d.nz, nzf = nz + 1;
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= nx * ny) return;
-    const int i = t / ny, j = t % ny;
-    const int b = blockIdx.y, pair = b / 6, c = b % 6;
-    const int k = kp[2 * pair + (c < 3 ? 0 : 1)];  // 1..nz
-    const int kk = k - 1;
-    double val;
-    if (c % 3 == 0) {
-        val = u[((size_t)(i + 1) * (ny + 2) + (j + 1)) * (nz + 2) + k] - mean[3 * nzf + kk];
-    } else if (c % 3 == 1) {
-        val = v[((size_t)(i + 1) * (ny + 1) + (j + 1)) * (nz + 2) + k] - mean[4 * nzf + kk];
-    } else {
-        const double* wc = w + ((size_t)(i + 1) * (ny + 2) + (j + 1)) * (nz + 1);
-        val = 0.5 * (wc[kk] + wc[kk + 1]) - mean[2 * nzf + kk];
-        if (c == 5) val = -val;
-    }
-    planes[(size_t)b * nx * ny + t] = val;
 }
 
 __device__ inline double auto_spec(double2 f, double norm) {
@@ -253,9 +291,9 @@ struct slc_stats {
     int device = 0;
     Dims d{};
     int nzc = 0, nzr = 0, nchunks = 0, nplanes = 0;
-    double* part = nullptr;    // nchunks x 6 x (nz + 1)
-    double* mean = nullptr;    // 6 x (nz + 1)
-    double* mom = nullptr;     // 4 x (nz + 1)
+    double* part = nullptr;    // nchunks x kNQ x (nz + 1)
+    double* shift = nullptr;   // 3 x (nz + 1)
+    double* avg = nullptr;     // kNQ x (nz + 1)
     int* kp = nullptr;         // 2 x nplanes (k_bot, k_top)
     double* planes = nullptr;  // 6 nplanes x nx x ny
     double2* fhat = nullptr;   // 6 nplanes x nx x (ny/2 + 1)
@@ -322,12 +360,11 @@ int slc_stats_create(int device, int nx, int ny, int nz, int nplanes, const int*
     const size_t nzf = (size_t)nz + 1;
     void* p = nullptr;
     int rc;
-    if ((rc = stats_alloc(st, sizeof(double) * st->nchunks * kNQ1 * nzf, &p))) goto bad;
+    if ((rc = stats_alloc(st, sizeof(double) * st->nchunks * kNQ * nzf, &p))) goto bad;
     st->part = (double*)p;
-    if ((rc = stats_alloc(st, sizeof(double) * kNQ1 * nzf, &p))) goto bad;
-    st->mean = (double*)p;
-    if ((rc = stats_alloc(st, sizeof(double) * kNQ2 * nzf, &p))) goto bad;
-    st->mom = (double*)p;
+    if ((rc = stats_alloc(st, sizeof(double) * (3 + kNQ) * nzf, &p))) goto bad;
+    st->shift = (double*)p;
+    st->avg = st->shift + 3 * nzf;
     if (nplanes > 0) {
         std::vector<int> kp(2 * (size_t)nplanes);
         for (int i = 0; i < nplanes; ++i) {
@@ -391,23 +428,17 @@ int slc_stats_accumulate(slc_stats* st, const double* u, const double* v, const 
     const Dims d = st->d;
     const dim3 grid(st->nzc, d.nbx, d.nby), blk(kLanes * kSub);
     const double plane = (double)d.nx * (double)d.ny;
-    hipLaunchKernelGGL(stats_pass_kernel<1>, grid, blk, 0, s, d, u, v, w, st->mean, st->part);
+    hipLaunchKernelGGL(stats_shift_kernel, dim3(st->nzr), dim3(kLanes * kRSub), 0, s, d, u, v, w,
+                       st->shift);
     HIP_OK(hipGetLastError());
-    hipLaunchKernelGGL(stats_reduce_kernel, dim3(st->nzr, kNQ1), dim3(kLanes * kRSub), 0, s,
-                       st->part, st->nchunks,
-                       kNQ1, d.nz, plane, st->mean);
-    hipLaunchKernelGGL(stats_pass_kernel<2>, grid, blk, 0, s, d, u, v, w, st->mean, st->part);
-    hipLaunchKernelGGL(stats_reduce_kernel, dim3(st->nzr, kNQ2), dim3(kLanes * kRSub), 0, s,
-                       st->part, st->nchunks,
-                       kNQ2, d.nz, plane, st->mom);
-    hipLaunchKernelGGL(stats_update_kernel, dim3((d.nz + 255) / 256), dim3(256), 0, s, d.nz,
-                       st->mean, st->mom, prof);
+    hipLaunchKernelGGL(stats_pass_kernel, grid, blk, 0, s, d, u, v, w, st->shift, st->part,
+                       st->kp, 2 * st->nplanes, st->planes);
+    hipLaunchKernelGGL(stats_reduce_kernel, dim3(st->nzr, kNQ), dim3(kLanes * kRSub), 0, s,
+                       st->part, st->nchunks, d.nz, plane, st->avg);
+    hipLaunchKernelGGL(stats_final_kernel, dim3((d.nz + 255) / 256), dim3(256), 0, s, d.nz,
+                       st->avg, st->shift, prof);
     HIP_OK(hipGetLastError());
     if (st->nplanes == 0) return SLC_OK;
-    const int npts = d.nx * d.ny;
-    hipLaunchKernelGGL(stats_planes_kernel, dim3((npts + 255) / 256, 6 * st->nplanes), dim3(256),
-                       0, s, d, u, v, w, st->mean, st->kp, st->planes);
-    HIP_OK(hipGetLastError());
     FFT_OK(rocfft_execution_info_set_stream(st->info, s));
     void* in[1] = {st->planes};
     void* outp[1] = {st->fhat};
