@@ -330,8 +330,8 @@ def stats_bench(args):
     """On-device turbulence statistics (TurbulenceStats.accumulate_statistics,
     include/slc_stats.h) at n^3 with the primary z+ = 15 plane pair and three
     extra spectra planes (z+ = 5, 30, 100): snapshots per second, fields
-    resident in HBM.  Algorithmic bytes per snapshot: the two plane passes
-    read u, v, w once each (2 x 24 B per grid point)."""
+    resident in HBM.  Algorithmic bytes per snapshot: u, v, w read once
+    (24 B per grid point)."""
     import numpy as np
     import torch
 
@@ -364,7 +364,7 @@ def stats_bench(args):
     ms = e0.elapsed_time(e1) / args.steps
     nfield = ((n + 1) * (n + 2) * (nz + 2) + (n + 2) * (n + 1) * (nz + 2) +
               (n + 2) * (n + 2) * (nz + 1))
-    bytes_snap = 2.0 * 8.0 * nfield
+    bytes_snap = 8.0 * nfield
     achieved = bytes_snap / (ms * 1e-3) / 1e9
     cpu = None
     if not args.no_cpu_baseline:
@@ -394,8 +394,8 @@ def stats_bench(args):
         "data": "synthetic (seeded random fields)",
         "config": {"workload": f"TurbulenceStats.accumulate_statistics {n}x{n}x{nz}, "
                                "4 spectra plane pairs", "nx": n, "ny": n, "nz": nz},
-        "roofline": {"bound": "hbm", "kernel": "slc_stats_accumulate (two plane passes, "
-                                               "reduces, spectra)",
+        "roofline": {"bound": "hbm", "kernel": "slc_stats_accumulate (one pass over the fields, "
+                                               "reduce, spectra)",
                      "achieved": round(achieved, 1), "peak": PEAK_HBM_GBPS, "unit": "GB/s",
                      "frac": round(achieved / PEAK_HBM_GBPS, 4), "traffic": None,
                      "bytes_per_launch": bytes_snap, "avg_ms": round(ms, 4)},
