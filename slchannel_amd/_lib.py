@@ -18,8 +18,8 @@ EXPORTS = (
     "slc_version", "slc_last_error", "slc_plan_create", "slc_plan_destroy",
     "slc_plan_workspace_bytes", "slc_apply_bc", "slc_departure", "slc_gather",
     "slc_stencil", "slc_locate_z", "slc_advect", "slc_bdf1_predict", "slc_bdf2_predict",
-    "slc_zsolve", "slc_divergence", "slc_poisson", "slc_project", "slc_project_step", "slc_implicit_project",
-    "slc_pressure_combine",
+    "slc_zsolve", "slc_divergence", "slc_poisson", "slc_project", "slc_project_step",
+    "slc_implicit_project", "slc_pressure_combine",
     "slc_bulk_velocity", "slc_bulk_force", "slc_bulk_force_noalloc", "slc_diagnostics",
     "slc_init_solenoidal", "slc_init_solenoidal_work", "slc_interp_trilinear",
     "slc_imex_rhs",

@@ -3,7 +3,8 @@
 A grid of more columns than the chip holds wavefronts has each of them walk
 several, with the factorisation, the scans' products and the level distances'
 reciprocals formed once.  The columns of a small grid, one to a wavefront, must
-come out as the same doubles, at every number of unknowns per lane.
+come out as the same doubles, at every number of unknowns per lane (1025: w
+alone fits the lanes).
 """
 
 import pytest
@@ -17,7 +18,8 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("theta", [1.0, 0.5])
 @pytest.mark.parametrize("nz,top", [(5, "dirichlet"), (64, "neumann"), (65, "dirichlet"),
                                     (100, "neumann"), (200, "dirichlet"), (257, "dirichlet"),
-                                    (300, "neumann"), (520, "dirichlet")])
+                                    (300, "neumann"), (520, "dirichlet"),
+                                    (1025, "dirichlet")])
 def test_walked_columns_match_single_columns(check, theta, nz, top):
     big = make_plan(_random_case(130, 90, nz, 4, "symmetric", seed=1), nu=1e-2, top=top)
     small = make_plan(_random_case(13, 9, nz, 4, "symmetric", seed=1), nu=1e-2, top=top)
