@@ -111,6 +111,12 @@ struct EnsTiles {
     bool big;            // a member needs 64-bit addressing (big_index)
 };
 
+// z-solve units and persistent workgroups of the three components.
+struct EnsColumns {
+    const unsigned* start[3];
+    unsigned n[3], grid[3];
+};
+
 // SL tile shapes the ensemble kernels are compiled for (autotuned):
 //   0: 4 x 4 x 16, 24 KB LDS   1: 4 x 4 x 32, 40 KB LDS   2: 2 x 8 x 16, 24 KB LDS
 //   (TI x TJ x TK arrival points per 256-thread workgroup)
@@ -139,7 +145,7 @@ void run_ens_tile_d6(const EnsMember* mem, const EnsTiles& t, int pass, int shap
 void run_ens_tile_f4(const EnsMember* mem, const EnsTiles& t, int pass, int shape, hipStream_t s);
 void run_ens_tile_f6(const EnsMember* mem, const EnsTiles& t, int pass, int shape, hipStream_t s);
 // max_ch: 2, 4 or 8 where no member's columns hold more unknowns per lane, else 0
-hipError_t run_ens_zsolve(const EnsLaunch& L, int comp, size_t lds_bytes, unsigned grid,
+hipError_t run_ens_zsolve(const EnsMember* mem, int nmem, const EnsColumns& z, size_t lds_bytes,
                           int max_ch, hipStream_t s);
 hipError_t run_ens_div_planes(const EnsLaunch& L, unsigned grid, hipStream_t s);
 hipError_t run_ens_thomas(const EnsLaunch& L, unsigned grid, hipStream_t s);

@@ -114,9 +114,9 @@ struct slc_ens {
     size_t d_umap_cap[3] = {0, 0, 0};
     std::vector<unsigned> h_start;
     unsigned totals[EK_COUNT] = {};
-    size_t zs_lds[3] = {0, 0, 0};
+    size_t zs_lds = 0;
     bool big = false;  // a member needs the tile kernels' 64-bit addressing (tile shape 0 only)
-    int zs_max[3] = {0, 0, 0};  // run_ens_zsolve's max_ch
+    int zs_max = 0;  // run_ens_zsolve's max_ch
     // rocFFT
     rocfft_execution_info info = nullptr;
     void* fft_work = nullptr;
@@ -309,10 +309,8 @@ int rebuild(slc_ens* e) {
     std::vector<EnsMember> tab(n);
     e->h_start.assign((size_t)EK_COUNT * (n + 1), 0u);
     std::vector<int> umap[3];
-    for (int k = 0; k < 3; ++k) {
-        e->zs_lds[k] = 0;
-        e->zs_max[k] = 2;
-    }
+    e->zs_lds = 0;
+    e->zs_max = 2;
     e->big = false;
     for (const Member* m : e->members) e->big = e->big || big_index(m->plan->g);
     for (int i = 0; i < n; ++i) {
@@ -354,8 +352,8 @@ int rebuild(slc_ens* e) {
         for (int k = 0; k < 3; ++k) {
             M.zch[k] = zsolve_scan_ch(k, m->nz);
             M.zcols[k] = M.zch[k] > 0 ? (int)kEnsZCols : zsolve_cols(k, m->nz);
-            if (M.zch[k] == 0 || M.zch[k] > 8) e->zs_max[k] = 0;
-            else if (e->zs_max[k] != 0) e->zs_max[k] = std::max(e->zs_max[k], M.zch[k]);
+            if (M.zch[k] == 0 || M.zch[k] > 8) e->zs_max = 0;
+            else if (e->zs_max != 0) e->zs_max = std::max(e->zs_max, M.zch[k]);
         }
         for (int k = 0; k < 3; ++k) M.nghost[k] = ghost_count(k, m->nx, m->ny, m->nz);
         // work units
@@ -369,8 +367,8 @@ int rebuild(slc_ens* e) {
             const long ncols = (long)m->nx * m->ny;
             units[EK_ZS0 + k] = (unsigned)((ncols + M.zcols[k] - 1) / M.zcols[k]);
             if (M.zch[k] == 0)
-                e->zs_lds[k] = std::max(e->zs_lds[k], (size_t)M.zcols[k] *
-                                                          zsolve_ld(k, m->nz) * sizeof(double));
+                e->zs_lds = std::max(
+                    e->zs_lds, (size_t)M.zcols[k] * zsolve_ld(k, m->nz) * sizeof(double));
         }
         units[EK_PLANE] = (unsigned)plane_tiles(m->nx, m->ny, m->nz);
         units[EK_THOMAS] = spike_ok(m->nz)
@@ -454,6 +452,17 @@ unsigned pgrid(const slc_ens* e, int kind) {
     return t < cap ? t : cap;
 }
 
+hipError_t run_zsolves(slc_ens* e) {
+    const int n = (int)e->members.size();
+    EnsColumns z;
+    for (int c = 0; c < 3; ++c) {
+        z.start[c] = e->d_start + (size_t)(EK_ZS0 + c) * (n + 1);
+        z.n[c] = e->totals[EK_ZS0 + c];
+        z.grid[c] = pgrid(e, EK_ZS0 + c);
+    }
+    return run_ens_zsolve(e->d_mem, n, z, e->zs_lds, e->zs_max, e->es);
+}
+
 int fft_all(slc_ens* e, bool forward) {
     FFT_OK(rocfft_execution_info_set_stream(e->info, e->es));
     for (SizeClass& c : e->classes) {
@@ -488,9 +497,7 @@ int enqueue_step(slc_ens* e) {
     if (int rc = sl_passes(e)) return rc;
     // nothing up to the divergence reads the predictor's ghosts; the
     // projection and the bulk shift write them with the interior
-    for (int c = 0; c < 3; ++c)
-        HIP_OK(run_ens_zsolve(launch(e, EK_ZS0 + c), c, e->zs_lds[c], pgrid(e, EK_ZS0 + c),
-                              e->zs_max[c], s));
+    HIP_OK(run_zsolves(e));
     HIP_OK(run_ens_div_planes(launch(e, EK_PLANE), pgrid(e, EK_PLANE), s));
     if (int rc = fft_all(e, true)) return rc;
     HIP_OK(run_ens_thomas(launch(e, EK_THOMAS), pgrid(e, EK_THOMAS), s));
@@ -967,9 +974,7 @@ static int autotune_sweeps(slc_ens* e, int reps, hipEvent_t t0, hipEvent_t t1,
             hipStream_t s = e->es;
             HIP_OK(run_ens_bc3(launch(e, EK_BC3), pgrid(e, EK_BC3), s));
             HIP_OK(run_ens_ustar(launch(e, EK_ELEM), pgrid(e, EK_ELEM), s));
-            for (int c = 0; c < 3; ++c)
-                HIP_OK(run_ens_zsolve(launch(e, EK_ZS0 + c), c, e->zs_lds[c],
-                                      pgrid(e, EK_ZS0 + c), e->zs_max[c], s));
+            HIP_OK(run_zsolves(e));
             HIP_OK(run_ens_div_planes(launch(e, EK_PLANE), pgrid(e, EK_PLANE), s));
             HIP_OK(run_ens_thomas(launch(e, EK_THOMAS), pgrid(e, EK_THOMAS), s));
             return SLC_OK;

@@ -6,9 +6,9 @@
 
 namespace slc {
 
-__device__ inline void ens_span(unsigned total, unsigned& beg, unsigned& end) {
-    const unsigned G = gridDim.x;
-    const unsigned lb = (unsigned)xcd_block(G);
+__device__ inline void ens_span(unsigned total, unsigned blk, unsigned G, unsigned& beg,
+                                unsigned& end) {
+    const unsigned lb = (unsigned)xcd_block(blk, G);
     const unsigned per = total / G, rem = total % G;
     beg = lb * per + (lb < rem ? lb : rem);
     end = beg + per + (lb < rem ? 1u : 0u);
@@ -25,13 +25,13 @@ __device__ inline int ens_find(const unsigned* start, int nmem, unsigned u) {
     return lo;
 }
 
-// f(member index, unit index within the member) for every unit of this
-// workgroup's chunk; a barrier separates consecutive units (LDS reuse).
+// f(member index, unit index within the member) for every unit of the chunk
+// of workgroup blk of G; a barrier separates consecutive units (LDS reuse).
 template <typename Fn>
 __device__ inline void ens_for(const unsigned* __restrict__ start, int nmem, unsigned total,
-                               Fn&& f) {
+                               unsigned blk, unsigned G, Fn&& f) {
     unsigned beg, end;
-    ens_span(total, beg, end);
+    ens_span(total, blk, G, beg, end);
     if (beg >= end) return;
     int m = ens_find(start, nmem, beg);
     for (unsigned u = beg; u < end; ++u) {
@@ -39,6 +39,12 @@ __device__ inline void ens_for(const unsigned* __restrict__ start, int nmem, uns
         if (u != beg) __syncthreads();
         f(m, u - start[m]);
     }
+}
+
+template <typename Fn>
+__device__ inline void ens_for(const unsigned* __restrict__ start, int nmem, unsigned total,
+                               Fn&& f) {
+    ens_for(start, nmem, total, blockIdx.x, gridDim.x, f);
 }
 
 // Kernel parameters of a batched launch.  The member table is read through

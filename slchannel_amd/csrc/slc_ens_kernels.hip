@@ -101,12 +101,12 @@ hipError_t run_ens_tile(const EnsMember* mem, const EnsTiles& t, int pass, int o
 // One kernel per longest column of the ensemble, so that its registers (and
 // the wavefronts that they leave) are those of the columns it solves: at most
 // 2 unknowns per lane, at most 4 or 8, or any (MAXCH 0: the LDS path as well).
+// The three components in one launch (workgroups of u, then v, then w): a
+// component's columns of small members are one generation of workgroups.
 template <int C, int MAXCH>
-__global__ __launch_bounds__(256, MAXCH == 2 ? 5 : MAXCH == 4 ? 4 : MAXCH == 8 ? 2 : 1) void ens_zsolve_kernel(
-    ENS_PARAMS) {
-    extern __shared__ double lds[];
-    __shared__ long cbase[kZColsMax];
-    ens_for(start, nmem, total, [&](int m, unsigned u) {
+__device__ inline void ens_zsolve_units(const EnsMember* __restrict__ mem, const EnsColumns& z,
+                                        int nmem, unsigned blk, double* lds, long* cbase) {
+    ens_for(z.start[C], nmem, z.n[C], blk, z.grid[C], [&](int m, unsigned u) {
         const EnsMember& M = mem[m];
         const int st = *M.state;
         const int nz = M.g.nz;
@@ -123,25 +123,31 @@ __global__ __launch_bounds__(256, MAXCH == 2 ? 5 : MAXCH == 4 ? 4 : MAXCH == 8 ?
     });
 }
 
-template <int C>
-void launch_ens_zsolve(const EnsLaunch& L, size_t lds_bytes, unsigned grid, int max_ch,
-                       hipStream_t s) {
-#define SLC_ENS_ZS(MAXCH)                                                                    \
-    hipLaunchKernelGGL((ens_zsolve_kernel<C, MAXCH>), dim3(grid), dim3(256), lds_bytes, s,   \
-                       ENS_ARGS(L))
+template <int MAXCH>
+__global__ __launch_bounds__(256, MAXCH == 2 ? 5 : MAXCH == 4 ? 4 : MAXCH == 8 ? 2 : 1)
+void ens_zsolve_kernel(const EnsMember* __restrict__ mem, EnsColumns z, int nmem) {
+    extern __shared__ double lds[];
+    __shared__ long cbase[kZColsMax];
+    const unsigned b = blockIdx.x;
+    if (b < z.grid[0])
+        ens_zsolve_units<0, MAXCH>(mem, z, nmem, b, lds, cbase);
+    else if (b < z.grid[0] + z.grid[1])
+        ens_zsolve_units<1, MAXCH>(mem, z, nmem, b - z.grid[0], lds, cbase);
+    else
+        ens_zsolve_units<2, MAXCH>(mem, z, nmem, b - z.grid[0] - z.grid[1], lds, cbase);
+}
+
+hipError_t run_ens_zsolve(const EnsMember* mem, int nmem, const EnsColumns& z, size_t lds_bytes,
+                          int max_ch, hipStream_t s) {
+    if (z.n[0] + z.n[1] + z.n[2] == 0) return hipSuccess;
+    const dim3 grid(z.grid[0] + z.grid[1] + z.grid[2]);
+#define SLC_ENS_ZS(MAXCH) \
+    hipLaunchKernelGGL(ens_zsolve_kernel<MAXCH>, grid, dim3(256), lds_bytes, s, mem, z, nmem)
     if (max_ch == 2) SLC_ENS_ZS(2);
     else if (max_ch == 4) SLC_ENS_ZS(4);
     else if (max_ch == 8) SLC_ENS_ZS(8);
     else SLC_ENS_ZS(0);
 #undef SLC_ENS_ZS
-}
-
-hipError_t run_ens_zsolve(const EnsLaunch& L, int comp, size_t lds_bytes, unsigned grid,
-                          int max_ch, hipStream_t s) {
-    if (L.total == 0) return hipSuccess;
-    if (comp == 0) launch_ens_zsolve<0>(L, lds_bytes, grid, max_ch, s);
-    else if (comp == 1) launch_ens_zsolve<1>(L, lds_bytes, grid, max_ch, s);
-    else launch_ens_zsolve<2>(L, lds_bytes, grid, max_ch, s);
     return hipGetLastError();
 }
 
