@@ -28,8 +28,8 @@
 //
 // Layout of the pass: a workgroup is 64 z lanes x 4 column groups.  The z
 // lanes make every load a coalesced 512-byte row segment; each thread walks
-// an x-run of 16 cells for 4 y-rows, carrying the previous u face in a
-// register so the cell-centred u costs one load.  Partials go to
+// an x-run of 16 cells for 4 y-rows (shorter on small grids), carrying the
+// previous u face in a register so the cell-centred u costs one load.  Partials go to
 // part[(chunk * NQ + q) * (nz + 1) + k] and are summed in chunk order by the
 // reduce kernel, so the result does not depend on scheduling.
 #include <rocfft/rocfft.h>
@@ -46,15 +46,16 @@ namespace {
 
 constexpr int kLanes = 64;  // z lanes per workgroup
 constexpr int kSub = 4;     // column groups per workgroup
-constexpr int kIB = 16;     // x cells per thread run
-constexpr int kJB = 16;     // y rows per workgroup (kJB / kSub per thread)
+constexpr int kRun = 16;    // most x cells of a thread's run, and y rows of a workgroup
 constexpr int kSide = 8;    // shift: kSide x kSide columns
 // sums of shifted values: u, v at centres; u node and square; v node and
 // square; w face and square; u w at centres
 enum { kUc = 0, kVc, kUn, kUU, kVn, kVV, kWf, kWW, kUW, kNQ };
 
+// ib x cells per thread run, jb y rows per workgroup (jb / kSub per thread);
+// nbx x nby chunks of columns
 struct Dims {
-    int nx, ny, nz, nbx, nby;
+    int nx, ny, nz, ib, jb, nbx, nby;
 };
 
 // shift[c * (nz + 1) + k]: the average of component c at level k (w: face k)
@@ -111,8 +112,8 @@ __global__ __launch_bounds__(kLanes * kSub) void stats_pass_kernel(
     const int lane = threadIdx.x % kLanes, sub = threadIdx.x / kLanes;
     const int k = blockIdx.x * kLanes + lane;
     const int nx = d.nx, ny = d.ny, nz = d.nz, nzf = nz + 1;
-    const int i0 = blockIdx.y * kIB, i1 = min(nx, i0 + kIB);
-    const int j0 = blockIdx.z * kJB, j1 = min(ny, j0 + kJB);
+    const int i0 = blockIdx.y * d.ib, i1 = min(nx, i0 + d.ib);
+    const int j0 = blockIdx.z * d.jb, j1 = min(ny, j0 + d.jb);
     const size_t su = (size_t)(ny + 2) * (nz + 2), sv = (size_t)(ny + 1) * (nz + 2),
                  sw = (size_t)(ny + 2) * (nz + 1);
     double s[kNQ];
@@ -352,8 +353,17 @@ int slc_stats_create(int device, int nx, int ny, int nz, int nplanes, const int*
     DeviceGuard dg(device);
     slc_stats* st = new slc_stats();
     st->device = device;
-    st->d = Dims{nx, ny, nz, (nx + kIB - 1) / kIB, (ny + kJB - 1) / kJB};
     st->nzc = (nz + kLanes - 1) / kLanes;        // pass workgroups along z
+    // 16 x 16 columns a workgroup; smaller chunks while the workgroups do not
+    // fill the chip, since a thread's walk is a chain of loads (30x20x40:
+    // 53 us a snapshot with 16 x 16, 30 with 4 x 4; 128^3: 49)
+    int ib = kRun, jb = kRun;
+    auto cover = [](int n, int m) { return (n + m - 1) / m; };
+    while (jb > kSub && (long)st->nzc * cover(nx, ib) * cover(ny, jb) < 512) {
+        jb /= 2;
+        ib /= 2;
+    }
+    st->d = Dims{nx, ny, nz, ib, jb, cover(nx, ib), cover(ny, jb)};
     st->nzr = (nz + 1 + kLanes - 1) / kLanes;    // reduce workgroups along z (faces)
     st->nchunks = st->d.nbx * st->d.nby;
     st->nplanes = nplanes;
