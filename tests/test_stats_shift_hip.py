@@ -1,6 +1,6 @@
 """Statistics about a provisional mean: fields with means far above their
-fluctuations, levels that are exactly uniform, and more spectra planes than the
-pass marks per level in one word.
+fluctuations, levels that are exactly uniform, more spectra planes than the
+pass marks per level in one word, and a grid large enough for the longest runs.
 
 Moments come from one pass over values less a provisional mean of 64 columns, so
 nothing of the size of the mean may be left in their error; a uniform level's
@@ -20,7 +20,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("shape,mean,extra", [
     ((24, 20, 33), (50.0, -20.0, 3.0), 2), ((5, 3, 66), (50.0, 0.0, 0.0), 2),
-    ((18, 14, 40), (1.0, 0.05, 0.0), 34)])
+    ((18, 14, 40), (1.0, 0.05, 0.0), 34), ((140, 100, 700), (1.0, 0.05, 0.0), 1)])
 def test_shifted_moments_match_oracle(check, shape, mean, extra):
     nx, ny, nz = shape
     ts, _ = _stats(nx, ny, nz, planes=[2.0 + 4.0 * q for q in range(extra)])
