@@ -373,7 +373,11 @@ struct BoxPlan {
 // y, and in x too when a plane holds an odd number of rows; a wrapped box
 // keeps the turns where the period is even.  A piece may reach one or two
 // elements out of its row, into a neighbouring row of the field (the first
-// and last rows of a field are ghost rows, never staged).
+// and last rows of a field are ghost rows, never staged).  A row's pieces are
+// one load of a wavefront: rows of more than kPairRow doubles go in 4-byte
+// pieces, unshifted.
+constexpr int kPairRow = 128;
+
 template <typename T, int C, int P>
 __device__ inline BoxPlan plan_box(const Grid& g, const T* S, const SBox& b, int cap_bytes) {
     BoxPlan r{BOX_NONE, b.xmin, b.ymin, b.kmin, 0, 1, 1, 1, 0, 0, 0, 0, 0};
@@ -412,6 +416,10 @@ __device__ inline BoxPlan plan_box(const Grid& g, const T* S, const SBox& b, int
         r.LD = kLZ;
         r.ns = r.BX;
         return r;
+    }
+    if (ld > kPairRow) {  // no pieces, so no row shifted
+        r.pairs = r.ax = r.ay = r.c = 0;
+        ld = ez;
     }
     // past eight slabs the box holds about as many values as the stencils do
     if (ey * ld > cap || ex * ey * ld > 8 * cap) return r;
@@ -553,7 +561,7 @@ template <typename T, int C, bool BIG>
 __device__ inline void stage_slab(const Grid& g, const T* __restrict__ S, const BoxPlan& b,
                                   int s0, int n, T* __restrict__ lds) {
     if constexpr (sizeof(T) == 8) {
-        if (b.pairs && b.LD <= 128) {
+        if (b.pairs) {
             // lane / NP and 64 / NP by a float reciprocal: the operands are small
             // integers, and half a unit keeps the quotient off the integers
             const int tid = phase_tid(), lane = tid & 63, NP = b.LD >> 1;
