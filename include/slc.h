@@ -221,6 +221,16 @@ int slc_imex_advance(slc_plan* plan, const double* u, const double* v, const dou
                      const double* ru_prev, const double* rv_prev, const double* rw_prev,
                      double dt, void* stream);
 
+/* One IMEX step but for the bulk constraint, u, v, w updated in place:
+ * slc_imex_advance into the plan's workspace, then the z-solves over dt with
+ * theta in (0, 1) and the projection with (dt, dt, p) of
+ * slc_implicit_project.  The fields come with their ghosts filled (the rhs reads them) and leave so; of
+ * ru, rv, rw the interiors are written.  Needs nz >= 3.
+ * Replaces solver.py:1062-1120. */
+int slc_imex_step(slc_plan* plan, double* u, double* v, double* w, double* ru, double* rv,
+                  double* rw, const double* ru_prev, const double* rv_prev, const double* rw_prev,
+                  double dt, double theta, double* p, void* stream);
+
 /* Run-loop diagnostics of the current fields, written to out (5 device
  * doubles, no host synchronisation): [0] max|div| (compute_divergence,
  * utils.py:166-180), [1] u_tau (compute_u_tau, utils.py:116-146), [2] the

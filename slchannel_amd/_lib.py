@@ -23,7 +23,7 @@ EXPORTS = (
     "slc_bulk_velocity", "slc_bulk_force", "slc_bulk_force_noalloc", "slc_diagnostics",
     "slc_init_solenoidal", "slc_init_solenoidal_work", "slc_interp_trilinear",
     "slc_imex_rhs",
-    "slc_ab2_update", "slc_imex_advance", "slc_set_option", "slc_set_viscosity",
+    "slc_ab2_update", "slc_imex_advance", "slc_imex_step", "slc_set_option", "slc_set_viscosity",
     "slc_profile_enable", "slc_profile_report",
     "slc_ens_create", "slc_ens_destroy", "slc_ens_member_bytes", "slc_ens_add",
     "slc_ens_remove", "slc_ens_count", "slc_ens_bytes", "slc_ens_trim_pool",
@@ -95,6 +95,7 @@ def load():
         "slc_interp_trilinear": ([i, vp, i, i, i, vp, vp, i, vp, vp, i, vp, vp, i, vp, vp], i),
         "slc_imex_rhs": ([vp, vp, vp, vp, vp, vp, vp, vp], i),
         "slc_imex_advance": ([vp] * 13 + [d, vp], i),
+        "slc_imex_step": ([vp] * 10 + [d, d, vp, vp], i),
         "slc_ab2_update": ([vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, d, vp], i),
         "slc_set_option": ([vp, i, i], i),
         "slc_set_viscosity": ([vp, d], i),

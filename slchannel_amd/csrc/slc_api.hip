@@ -656,7 +656,7 @@ int slc_zsolve(slc_plan* p, int comp, double* field, double dt, double theta, vo
     DeviceGuard dg(p->device);
     const bool refactor = zrefactor(p, comp, dt, theta);
     Timed t(p, kZLabel[comp], stream);
-    HIP_OK(run_zsolve(p->g, comp, field, dt, theta, p->d_dzc, p->d_dzf,
+    HIP_OK(run_zsolve(p->g, comp, field, field, dt, theta, p->d_dzc, p->d_dzf,
                       p->ztab + (size_t)comp * 3 * (p->nz + 2), refactor, S(stream)));
     return SLC_OK;
 }
@@ -732,13 +732,21 @@ int slc_implicit_project(slc_plan* p, double* u, double* v, double* w, double dt
     if (!(theta > 0.0 && theta <= 1.0)) return fail(SLC_EINVAL, "theta must be in (0, 1]");
     if (p->nz < 3) return fail(SLC_EINVAL, "w z-solve needs nz >= 3");
     DeviceGuard dg(p->device);
+    double* const F[3] = {u, v, w};
+    return implicit_project(p, F, F, dt_z, theta, rhs_scale, dt_proj, pr, stream);
+}
+
+}  // extern "C"
+
+int slc::implicit_project(slc_plan* p, double* const src[3], double* const F[3], double dt_z,
+                          double theta, double rhs_scale, double dt_proj, double* pr,
+                          void* stream) {
     // ghosts enter the z-solves only in the explicit part of a theta < 1
     // right-hand side
     if (theta != 1.0) {
         Timed t(p, "ghost_fill_uvw", stream);
-        HIP_OK(run_bc(p->g, u, v, w, S(stream)));
+        HIP_OK(run_bc(p->g, src[0], src[1], src[2], S(stream)));
     }
-    double* const F[3] = {u, v, w};
     double* tab[3];
     bool refactor[3];
     for (int c = 0; c < 3; ++c) {
@@ -748,14 +756,17 @@ int slc_implicit_project(slc_plan* p, double* u, double* v, double* w, double dt
     if (p->prof) {
         for (int c = 0; c < 3; ++c) {
             Timed t(p, kZLabel[c], stream);
-            HIP_OK(run_zsolve(p->g, c, F[c], dt_z, theta, p->d_dzc, p->d_dzf, tab[c], refactor[c],
-                              S(stream)));
+            HIP_OK(run_zsolve(p->g, c, src[c], F[c], dt_z, theta, p->d_dzc, p->d_dzf, tab[c],
+                              refactor[c], S(stream)));
         }
     } else {
-        HIP_OK(run_zsolve3(p->g, F, dt_z, theta, p->d_dzc, p->d_dzf, tab, refactor, S(stream)));
+        HIP_OK(run_zsolve3(p->g, src, F, dt_z, theta, p->d_dzc, p->d_dzf, tab, refactor,
+                           S(stream)));
     }
-    return projection(p, u, v, w, rhs_scale, dt_proj, pr, true, stream);
+    return projection(p, F[0], F[1], F[2], rhs_scale, dt_proj, pr, true, stream);
 }
+
+extern "C" {
 
 int slc_bulk_velocity(slc_plan* p, const double* u, double* out, void* stream) {
     if (int rc = check_plan(p)) return rc;

@@ -117,8 +117,8 @@ __device__ inline void ens_zsolve_units(const EnsMember* __restrict__ mem, const
                 M.g, M.fld[ens_c(st)][C], tab, col0 + (threadIdx.x >> 6), kZScanCols,
                 min(col0 + kEnsZCols, ncols), M.zch[C]);
         } else {
-            zsolve_body<C>(M.g, M.fld[ens_c(st)][C], tab, 0.0, M.dzc, M.dzf, M.zcols[C], u, lds,
-                           cbase);
+            double* f = M.fld[ens_c(st)][C];
+            zsolve_body<C>(M.g, f, f, tab, 0.0, M.dzc, M.dzf, M.zcols[C], u, lds, cbase);
         }
     });
 }

@@ -1,5 +1,6 @@
 // slc_imex.hip -- the Eulerian IMEX explicit terms (slc_imex_rhs,
-// slc_ab2_update, slc_imex_advance).
+// slc_ab2_update, slc_imex_advance) and the step's part up to the projection
+// (slc_imex_step).
 //
 // compute_momentum_rhs_fused_imex (operators.py:639-835; the Triton kernel of
 // eulerian_triton.py:31-193 computes the same): divergence-form advection on
@@ -263,6 +264,23 @@ extern "C" int slc_imex_advance(slc_plan* p, const double* u, const double* v, c
     const Ab2 ab{{un, vn, wn}, {(double*)ru_prev, (double*)rv_prev, (double*)rw_prev}, dt};
     HIP_OK(run_imex<true>(p, u, v, w, Rhs3{ru, rv, rw}, ab, static_cast<hipStream_t>(stream)));
     return SLC_OK;
+}
+
+extern "C" int slc_imex_step(slc_plan* p, double* u, double* v, double* w, double* ru, double* rv,
+                             double* rw, const double* ru_prev, const double* rv_prev,
+                             const double* rw_prev, double dt, double theta, double* pr,
+                             void* stream) {
+    if (!p) return fail(SLC_EINVAL, "null plan");
+    if (!(theta > 0.0 && theta < 1.0)) return fail(SLC_EINVAL, "theta must be in (0, 1)");
+    if (p->nz < 3) return fail(SLC_EINVAL, "w z-solve needs nz >= 3");
+    // the advanced fields wait in the plan's U* arrays for the z-solves, which
+    // write u, v and w: as many bytes as solves in place, no copy
+    if (int rc = slc_imex_advance(p, u, v, w, p->us[0], p->us[1], p->us[2], ru, rv, rw, ru_prev,
+                                  rv_prev, rw_prev, dt, stream))
+        return rc;
+    DeviceGuard dg(p->device);
+    double* const f[3] = {u, v, w};
+    return implicit_project(p, p->us, f, dt, theta, dt, dt, pr, stream);
 }
 
 extern "C" int slc_ab2_update(slc_plan* p, double* u, double* v, double* w, const double* ru,

@@ -95,13 +95,14 @@ hipError_t run_fill_f64(double* p, long n, double v, hipStream_t s);
 hipError_t run_bc(const Grid& g, double* u, double* v, double* w, hipStream_t s);
 hipError_t run_zfactor(const Grid& g, int comp, double dt, double theta, const double* dz_c,
                        const double* dz_f, double* tab, hipStream_t s);
-hipError_t run_zsolve(const Grid& g, int comp, double* f, double dt, double theta,
-                      const double* dz_c, const double* dz_f, double* tab, bool refactor,
-                      hipStream_t s);
+// src to f: the same array, or another one where theta < 1
+hipError_t run_zsolve(const Grid& g, int comp, const double* src, double* f, double dt,
+                      double theta, const double* dz_c, const double* dz_f, double* tab,
+                      bool refactor, hipStream_t s);
 // the three components' z-solves (tab, refactor: per component) in one launch
-hipError_t run_zsolve3(const Grid& g, double* const f[3], double dt, double theta,
-                       const double* dz_c, const double* dz_f, double* const tab[3],
-                       const bool refactor[3], hipStream_t s);
+hipError_t run_zsolve3(const Grid& g, const double* const src[3], double* const f[3], double dt,
+                       double theta, const double* dz_c, const double* dz_f,
+                       double* const tab[3], const bool refactor[3], hipStream_t s);
 // wrap: read no ghost entry (the fields' ghosts need not be filled)
 hipError_t run_div_planes(const Grid& g, const double* u, const double* v, const double* w,
                           const double* dz_f, double scale, double* planes, bool wrap,

@@ -130,14 +130,14 @@ hipError_t run_zfactor(const Grid& g, int comp, double dt, double theta, const d
 }
 
 template <int C>
-__global__ __launch_bounds__(256) void zsolve_kernel(Grid g, double* __restrict__ F,
+__global__ __launch_bounds__(256) void zsolve_kernel(Grid g, const double* S, double* F,
                                                      const double* __restrict__ tab, double beta,
                                                      const double* __restrict__ dz_c,
                                                      const double* __restrict__ dz_f,
                                                      int kZCols) {
     extern __shared__ double lds[];
     __shared__ long cbase[kZColsMax];
-    zsolve_body<C>(g, F, tab, beta, dz_c, dz_f, kZCols, blockIdx.x, lds, cbase);
+    zsolve_body<C>(g, S, F, tab, beta, dz_c, dz_f, kZCols, blockIdx.x, lds, cbase);
 }
 
 // Columns of 8 or more unknowns per lane move through LDS (coalesced), the
@@ -150,6 +150,7 @@ __global__ __launch_bounds__(256) void zsolve_kernel(Grid g, double* __restrict_
 // The components' column solves in one launch: nb[c] blocks of component c
 // walk its columns with a stride of all its wavefronts.
 struct ZSolve3 {
+    const double* s[3];
     double* f[3];
     const double* tab[3];
     const double* dz_c;
@@ -178,11 +179,14 @@ __global__ __launch_bounds__(256, zwaves(CHU, EXPL)) void zsolve3_kernel(Grid g,
     double* xu = XU ? xl[wave] : nullptr;
     double* xw = XW ? xl[wave] : nullptr;
     if (c == 0)
-        zsolve_run<0, CHU, EXPL>(g, a.f[0], a.tab[0], col, stride, ncols, a.beta, a.dz_c, a.dz_f, xu);
+        zsolve_run<0, CHU, EXPL>(g, a.s[0], a.f[0], a.tab[0], col, stride, ncols, a.beta,
+                                  a.dz_c, a.dz_f, xu);
     else if (c == 1)
-        zsolve_run<1, CHU, EXPL>(g, a.f[1], a.tab[1], col, stride, ncols, a.beta, a.dz_c, a.dz_f, xu);
+        zsolve_run<1, CHU, EXPL>(g, a.s[1], a.f[1], a.tab[1], col, stride, ncols, a.beta,
+                                  a.dz_c, a.dz_f, xu);
     else
-        zsolve_run<2, CHW, EXPL>(g, a.f[2], a.tab[2], col, stride, ncols, a.beta, a.dz_c, a.dz_f, xw);
+        zsolve_run<2, CHW, EXPL>(g, a.s[2], a.f[2], a.tab[2], col, stride, ncols, a.beta,
+                                  a.dz_c, a.dz_f, xw);
 }
 
 // Arguments of `comps` components in one launch: a block per 4 columns, and
@@ -204,8 +208,10 @@ static ZSolve3 zsolve3(const Grid& g, double beta, const double* dz_c, const dou
 static hipError_t launch_zsolve3(const Grid& g, const ZSolve3& a, hipStream_t s) {
     const int cu = zsolve_scan_ch(0, g.nz), cw = zsolve_scan_ch(2, g.nz);
     const dim3 grid(a.nb[0] + a.nb[1] + a.nb[2]), blk(256);
+    bool expl = a.beta != 0.0;
+    for (int c = 0; c < 3; ++c) expl = expl || a.s[c] != a.f[c];
 #define SLC_ZS3(CU, CW)                                                              \
-    if (a.beta != 0.0)                                                               \
+    if (expl)                                                                        \
         hipLaunchKernelGGL((zsolve3_kernel<CU, CW, true>), grid, blk, 0, s, g, a);   \
     else                                                                             \
         hipLaunchKernelGGL((zsolve3_kernel<CU, CW, false>), grid, blk, 0, s, g, a)
@@ -223,8 +229,8 @@ static hipError_t launch_zsolve3(const Grid& g, const ZSolve3& a, hipStream_t s)
     return hipGetLastError();
 }
 
-hipError_t run_zsolve(const Grid& g, int comp, double* f, double dt, double theta,
-                      const double* dz_c, const double* dz_f, double* tab, bool refactor,
+hipError_t run_zsolve(const Grid& g, int comp, const double* src, double* f, double dt,
+                      double theta, const double* dz_c, const double* dz_f, double* tab, bool refactor,
                       hipStream_t s) {
     if (refactor)
         hipLaunchKernelGGL(zfactor_kernel, dim3(1), dim3(64), 0, s, g, comp, dt, theta, dz_c,
@@ -233,6 +239,7 @@ hipError_t run_zsolve(const Grid& g, int comp, double* f, double dt, double thet
     const int ch = zsolve_scan_ch(comp, g.nz);
     if (ch > 0) {
         ZSolve3 a = zsolve3(g, beta, dz_c, dz_f, 1);
+        a.s[comp] = src;
         a.f[comp] = f;
         a.tab[comp] = tab;
         for (int c = 0; c < 3; ++c) a.nb[c] = c == comp ? a.nb[c] : 0u;
@@ -244,24 +251,25 @@ hipError_t run_zsolve(const Grid& g, int comp, double* f, double dt, double thet
     dim3 grid((unsigned)((ncols + cols - 1) / cols));
     size_t shm = (size_t)cols * zsolve_ld(comp, g.nz) * sizeof(double);
     if (comp == 0)
-        hipLaunchKernelGGL(zsolve_kernel<0>, grid, dim3(256), shm, s, g, f, tab, beta, dz_c, dz_f,
-                           cols);
+        hipLaunchKernelGGL(zsolve_kernel<0>, grid, dim3(256), shm, s, g, src, f, tab, beta, dz_c,
+                           dz_f, cols);
     else if (comp == 1)
-        hipLaunchKernelGGL(zsolve_kernel<1>, grid, dim3(256), shm, s, g, f, tab, beta, dz_c, dz_f,
-                           cols);
+        hipLaunchKernelGGL(zsolve_kernel<1>, grid, dim3(256), shm, s, g, src, f, tab, beta, dz_c,
+                           dz_f, cols);
     else
-        hipLaunchKernelGGL(zsolve_kernel<2>, grid, dim3(256), shm, s, g, f, tab, beta, dz_c, dz_f,
-                           cols);
+        hipLaunchKernelGGL(zsolve_kernel<2>, grid, dim3(256), shm, s, g, src, f, tab, beta, dz_c,
+                           dz_f, cols);
     return hipGetLastError();
 }
 
 // The three components' solves, in one launch where the columns fit the lanes.
-hipError_t run_zsolve3(const Grid& g, double* const f[3], double dt, double theta,
-                       const double* dz_c, const double* dz_f, double* const tab[3],
-                       const bool refactor[3], hipStream_t s) {
+hipError_t run_zsolve3(const Grid& g, const double* const src[3], double* const f[3], double dt,
+                       double theta, const double* dz_c, const double* dz_f,
+                       double* const tab[3], const bool refactor[3], hipStream_t s) {
     if (zsolve_scan_ch(0, g.nz) == 0 || zsolve_scan_ch(2, g.nz) == 0) {
         for (int c = 0; c < 3; ++c) {
-            hipError_t e = run_zsolve(g, c, f[c], dt, theta, dz_c, dz_f, tab[c], refactor[c], s);
+            hipError_t e =
+                run_zsolve(g, c, src[c], f[c], dt, theta, dz_c, dz_f, tab[c], refactor[c], s);
             if (e != hipSuccess) return e;
         }
         return hipSuccess;
@@ -271,6 +279,7 @@ hipError_t run_zsolve3(const Grid& g, double* const f[3], double dt, double thet
         if (refactor[c])
             hipLaunchKernelGGL(zfactor_kernel, dim3(1), dim3(64), 0, s, g, c, dt, theta, dz_c, dz_f,
                                tab[c]);
+        a.s[c] = src[c];
         a.f[c] = f[c];
         a.tab[c] = tab[c];
     }

@@ -170,11 +170,11 @@ __host__ __device__ inline int zsolve_cols(int comp, int nz) {
     return cols > kZColsMax ? kZColsMax : cols;
 }
 
-// Column block cb (kZCols columns) of component C.  lds: kZCols * ld doubles;
-// cbase: kZColsMax longs.  Ends with a barrier-free write-back; the caller
-// synchronises before reusing lds.
+// Column block cb (kZCols columns) of component C, of S into F (the same array
+// or another).  lds: kZCols * ld doubles; cbase: kZColsMax longs.  Ends with a
+// barrier-free write-back; the caller synchronises before reusing lds.
 template <int C>
-__device__ inline void zsolve_body(const Grid& g, double* __restrict__ F,
+__device__ inline void zsolve_body(const Grid& g, const double* S, double* F,
                                    const double* __restrict__ tab, double beta,
                                    const double* __restrict__ dz_c,
                                    const double* __restrict__ dz_f, int kZCols, long cb,
@@ -203,7 +203,7 @@ __device__ inline void zsolve_body(const Grid& g, double* __restrict__ F,
     for (int e = tid; e < kZCols * SZ; e += blockDim.x) {
         const int c = e / SZ, k = e - (e / SZ) * SZ;
         const long a = cbase[c];
-        if (a >= 0) lds[c * ld + k] = F[a + k];
+        if (a >= 0) lds[c * ld + k] = S[a + k];
     }
     __syncthreads();
 
@@ -438,8 +438,10 @@ struct ZNoDist {
     __device__ ZNoDist(int, int, const double*, const double*) {}
 };
 
-// The columns col, col + stride, .. below end, one at a time, the next one's
-// loads ahead of the solve.  EXPL: theta < 1.  With X (zscan_lds<CH> doubles
+// The columns col, col + stride, .. below end of F, one at a time, the next
+// one's loads ahead of the solve.  EXPL: theta < 1, and the columns come from S
+// (F or another array; without EXPL S is not read: a second address spilled
+// the eight waves of one unknown per lane).  With X (zscan_lds<CH> doubles
 // of the wavefront's own LDS) a column moves between HBM and the registers
 // through LDS in wavefront-contiguous pieces (each load instruction touches
 // 512 consecutive bytes) instead of each lane reading its CH consecutive
@@ -450,7 +452,7 @@ struct ZNoDist {
 // 256x192x192, 88 at 256^3, 707 at 512^3, 578 at 256x256x1000 (2.9, 3.1,
 // 3.0, 1.8 TB/s); so 31, 61, 427 and 226 us (4.8, 4.4, 5.0, 4.6 TB/s).
 template <int C, int CH, bool EXPL>
-__device__ inline void zsolve_run(const Grid& g, double* __restrict__ F,
+__device__ inline void zsolve_run(const Grid& g, const double* S, double* F,
                                   const double* __restrict__ tab, unsigned col, unsigned stride,
                                   unsigned end, double beta = 0.0,
                                   const double* __restrict__ dz_c = nullptr,
@@ -464,8 +466,9 @@ __device__ inline void zsolve_run(const Grid& g, double* __restrict__ F,
     unsigned I = col / ny, J = col % ny;
     const unsigned dI = stride / ny, dJ = stride % ny;
     auto column = [&] {
-        return F + ((long)(I + 1) * Comp<C>::SY(g) + (J + 1)) * Comp<C>::SZ(g) + 1;
+        return F + (((long)(I + 1) * Comp<C>::SY(g) + (J + 1)) * Comp<C>::SZ(g) + 1);
     };
+    auto source = [&](const double* Fc) { return EXPL ? S + (Fc - F) : Fc; };
     // raw: through LDS the wavefront's coalesced pieces of the column, else
     // the lane's own unknowns (and the entry above the last one)
     auto load = [&](const double* Fc, double* raw) {
@@ -487,8 +490,8 @@ __device__ inline void zsolve_run(const Grid& g, double* __restrict__ F,
     if (col >= end) return;
     double next[CH];
     double* Fn = column();
-    load(Fn, next);
-    double sn = EXPL ? Fn[-1] : 0.0;
+    load(source(Fn), next);
+    double sn = EXPL ? source(Fn)[-1] : 0.0;
     ZFactor<CH> z;
     zfactor_load(z, tab, n, lane);
     const std::conditional_t<EXPL, ZDist<C, CH>, ZNoDist> dist(j0, n, dz_c, dz_f);
@@ -521,8 +524,8 @@ __device__ inline void zsolve_run(const Grid& g, double* __restrict__ F,
                 ++I;
             }
             Fn = column();
-            load(Fn, next);
-            if (EXPL) sn = Fn[-1];
+            load(source(Fn), next);
+            if (EXPL) sn = source(Fn)[-1];
         }
         if constexpr (EXPL) zsolve_explicit<C, CH>(g, p, j0, n, beta, dist, s0);
         double v = 0.0;
@@ -582,20 +585,20 @@ __device__ inline void zsolve_run(const Grid& g, double* __restrict__ F,
 
 // Runtime dispatch of ch (from zsolve_scan_ch, at most MAXCH), theta = 1.
 template <int C, int MAXCH>
-__device__ inline void zsolve_run_any(const Grid& g, double* __restrict__ F,
+__device__ inline void zsolve_run_any(const Grid& g, double* F,
                                       const double* __restrict__ tab, unsigned col,
                                       unsigned stride, unsigned end, int ch) {
     switch (ch) {
-        case 1: zsolve_run<C, 1, false>(g, F, tab, col, stride, end); break;
-        case 2: zsolve_run<C, 2, false>(g, F, tab, col, stride, end); break;
+        case 1: zsolve_run<C, 1, false>(g, F, F, tab, col, stride, end); break;
+        case 2: zsolve_run<C, 2, false>(g, F, F, tab, col, stride, end); break;
         case 4:
-            if constexpr (MAXCH >= 4) zsolve_run<C, 4, false>(g, F, tab, col, stride, end);
+            if constexpr (MAXCH >= 4) zsolve_run<C, 4, false>(g, F, F, tab, col, stride, end);
             break;
         case 8:
-            if constexpr (MAXCH >= 8) zsolve_run<C, 8, false>(g, F, tab, col, stride, end);
+            if constexpr (MAXCH >= 8) zsolve_run<C, 8, false>(g, F, F, tab, col, stride, end);
             break;
         default:
-            if constexpr (MAXCH >= 16) zsolve_run<C, 16, false>(g, F, tab, col, stride, end);
+            if constexpr (MAXCH >= 16) zsolve_run<C, 16, false>(g, F, F, tab, col, stride, end);
     }
 }
 

@@ -330,6 +330,20 @@ class HipPlan:
                                               *[_ptr(t) for t in new], *[_ptr(t) for t in r], *rp,
                                               float(dt), self._stream()), "slc_imex_advance")
 
+    def imex_step(self, u, v, w, r, r_prev, dt, theta, p=None):
+        """One IMEX step of u, v, w in place, up to the projection, and its
+        rhs r (interiors only; slc_imex_step)."""
+        self._uvw(u, v, w)
+        self._uvw(*r, "_rhs")
+        if r_prev is not None:
+            self._uvw(*r_prev, "_prev")
+        if p is not None:
+            self._chk(p, self.shapes["p"], "p")
+        rp = [_ptr(t) for t in r_prev] if r_prev is not None else [_ptr(None)] * 3
+        _lib.check(self._lib.slc_imex_step(self._h, _ptr(u), _ptr(v), _ptr(w),
+                                           *[_ptr(t) for t in r], *rp, float(dt), float(theta),
+                                           _ptr(p), self._stream()), "slc_imex_step")
+
     def set_viscosity(self, nu):
         """slc_set_viscosity: the plan's nu (z-solve factors rebuilt at next use)."""
         _lib.check(self._lib.slc_set_viscosity(self._h, float(nu)), "slc_set_viscosity")

@@ -251,20 +251,24 @@ class SLChannelFlow:
         self.forcing = self._bulk[1]
         return self._bulk[2], self.forcing
 
-    def _implicit_and_project(self, dt_z, rhs_scale, dt_proj, theta=1.0, sl=True):
+    def _own_p(self):
+        """A pressure array apart from the 'inc' history."""
+        if self.p is self._P_curr or self.p is self._P_prev:
+            self.p = torch.empty_like(self.p)
+
+    def _implicit_and_project(self, dt_z, rhs_scale, dt_proj):
         """z-solves and projection with the ghosts they need and leave; returns
         the buffer holding phi: self.p, or for SL steps with the 'inc' option
         a separate phi buffer (self.p then ends as the full pressure
         p^{n+1})."""
-        if sl and self.sl_bdf2_pressure == "inc":
+        if self.sl_bdf2_pressure == "inc":
             if self._phi is None:
                 self._phi = torch.zeros_like(self.p)
             phi = self._phi
         else:
-            if self.p is self._P_curr or self.p is self._P_prev:
-                self.p = torch.empty_like(self.p)  # keep the 'inc' history intact
+            self._own_p()
             phi = self.p
-        self.plan.implicit_project(self.u, self.v, self.w, dt_z, theta, rhs_scale, dt_proj, phi)
+        self.plan.implicit_project(self.u, self.v, self.w, dt_z, 1.0, rhs_scale, dt_proj, phi)
         return phi
 
     def _step_sl_bdf1_bootstrap(self, dt):
@@ -369,22 +373,20 @@ class SLChannelFlow:
     def step_imex(self, dt):
         """solver.py:1055-1127: AB2 explicit advection + xy-diffusion (forward
         Euler while there is no previous rhs), Crank-Nicolson z-diffusion,
-        projection with dt, bulk shift.  Returns (u_bulk, forcing) as 0-D
-        device tensors."""
+        projection with dt, bulk shift.  u, v, w are updated in their own
+        tensors.  Returns (u_bulk, forcing) as 0-D device tensors."""
         dt = float(dt)
         self.apply_bc_uvw()
         s = self.shapes
         if self._imex_cur is None:
-            self._imex_cur = [torch.empty(s[c], dtype=torch.float64, device=self.device)
+            # zero off the interiors, which is all that a step writes
+            self._imex_cur = [torch.zeros(s[c], dtype=torch.float64, device=self.device)
                               for c in "uvw"]
-        self._ensure_star()
-        prev, new = self._imex_prev, self._star
-        self.plan.imex_advance(self.u, self.v, self.w, new, self._imex_cur, prev, dt)
-        self._star = [self.u, self.v, self.w]
-        self.u, self.v, self.w = new
+        prev = self._imex_prev
+        self._own_p()
+        self.plan.imex_step(self.u, self.v, self.w, self._imex_cur, prev, dt, 0.5, self.p)
         # the current rhs becomes the previous one (buffers swapped, no copy)
         self._imex_prev, self._imex_cur = self._imex_cur, prev
-        self._implicit_and_project(dt, dt, dt, theta=0.5, sl=False)
         out = self._apply_bulk_forcing(dt)
         self.current_step += 1
         self.time += dt
