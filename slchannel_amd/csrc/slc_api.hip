@@ -638,13 +638,18 @@ int slc_bdf2_predict(slc_plan* p, const double* u, const double* v, const double
 }
 
 // The factorisation of a component's z-solve depends only on (dt, theta):
-// whether the plan's is for others, which it then counts as rebuilt.
+// whether the plan's is for others.  It counts as none from then on until the
+// solve that rebuilds it has been launched (zbuilt).
 static bool zrefactor(slc_plan* p, int comp, double dt, double theta) {
-    const bool same = p->zvalid[comp] && p->zkey[comp][0] == dt && p->zkey[comp][1] == theta;
+    p->zvalid[comp] =
+        p->zvalid[comp] && p->zkey[comp][0] == dt && p->zkey[comp][1] == theta;
+    return !p->zvalid[comp];
+}
+
+static void zbuilt(slc_plan* p, int comp, double dt, double theta) {
     p->zvalid[comp] = true;
     p->zkey[comp][0] = dt;
     p->zkey[comp][1] = theta;
-    return !same;
 }
 
 int slc_zsolve(slc_plan* p, int comp, double* field, double dt, double theta, void* stream) {
@@ -658,6 +663,7 @@ int slc_zsolve(slc_plan* p, int comp, double* field, double dt, double theta, vo
     Timed t(p, kZLabel[comp], stream);
     HIP_OK(run_zsolve(p->g, comp, field, field, dt, theta, p->d_dzc, p->d_dzf,
                       p->ztab + (size_t)comp * 3 * (p->nz + 2), refactor, S(stream)));
+    zbuilt(p, comp, dt, theta);
     return SLC_OK;
 }
 
@@ -730,13 +736,22 @@ int slc_implicit_project(slc_plan* p, double* u, double* v, double* w, double dt
     if (int rc = check_plan(p)) return rc;
     if (!u || !v || !w) return fail(SLC_EINVAL, "null array");
     if (!(theta > 0.0 && theta <= 1.0)) return fail(SLC_EINVAL, "theta must be in (0, 1]");
-    if (p->nz < 3) return fail(SLC_EINVAL, "w z-solve needs nz >= 3");
+    if (int rc = check_zsolves(p)) return rc;
     DeviceGuard dg(p->device);
     double* const F[3] = {u, v, w};
     return implicit_project(p, F, F, dt_z, theta, rhs_scale, dt_proj, pr, stream);
 }
 
 }  // extern "C"
+
+int slc::check_zsolves(const slc_plan* p) {
+    if (p->nz < 3) return fail(SLC_EINVAL, "w z-solve needs nz >= 3");
+    for (int c = 0; c < 3; ++c)
+        if (!zsolve_fits(c, p->nz))
+            return fail(SLC_EINVAL, "nz=%d: a column of %c does not fit the z-solve's LDS", p->nz,
+                        "uvw"[c]);
+    return SLC_OK;
+}
 
 int slc::implicit_project(slc_plan* p, double* const src[3], double* const F[3], double dt_z,
                           double theta, double rhs_scale, double dt_proj, double* pr,
@@ -763,6 +778,7 @@ int slc::implicit_project(slc_plan* p, double* const src[3], double* const F[3],
         HIP_OK(run_zsolve3(p->g, src, F, dt_z, theta, p->d_dzc, p->d_dzf, tab, refactor,
                            S(stream)));
     }
+    for (int c = 0; c < 3; ++c) zbuilt(p, c, dt_z, theta);
     return projection(p, F[0], F[1], F[2], rhs_scale, dt_proj, pr, true, stream);
 }
 

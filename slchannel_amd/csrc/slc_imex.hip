@@ -272,7 +272,7 @@ extern "C" int slc_imex_step(slc_plan* p, double* u, double* v, double* w, doubl
                              void* stream) {
     if (!p) return fail(SLC_EINVAL, "null plan");
     if (!(theta > 0.0 && theta < 1.0)) return fail(SLC_EINVAL, "theta must be in (0, 1)");
-    if (p->nz < 3) return fail(SLC_EINVAL, "w z-solve needs nz >= 3");
+    if (int rc = check_zsolves(p)) return rc;
     // the advanced fields wait in the plan's U* arrays for the z-solves, which
     // write u, v and w: as many bytes as solves in place, no copy
     if (int rc = slc_imex_advance(p, u, v, w, p->us[0], p->us[1], p->us[2], ru, rv, rw, ru_prev,

@@ -95,6 +95,8 @@ hipError_t run_fill_f64(double* p, long n, double v, hipStream_t s);
 hipError_t run_bc(const Grid& g, double* u, double* v, double* w, hipStream_t s);
 hipError_t run_zfactor(const Grid& g, int comp, double dt, double theta, const double* dz_c,
                        const double* dz_f, double* tab, hipStream_t s);
+// Whether run_zsolve takes a column of component comp (nz up to about 6000).
+bool zsolve_fits(int comp, int nz);
 // src to f: the same array, or another one where theta < 1
 hipError_t run_zsolve(const Grid& g, int comp, const double* src, double* f, double dt,
                       double theta, const double* dz_c, const double* dz_f, double* tab,

@@ -229,9 +229,13 @@ static hipError_t launch_zsolve3(const Grid& g, const ZSolve3& a, hipStream_t s)
     return hipGetLastError();
 }
 
+bool zsolve_fits(int comp, int nz) {
+    return zsolve_scan_ch(comp, nz) > 0 || zsolve_cols(comp, nz) > 0;
+}
+
 hipError_t run_zsolve(const Grid& g, int comp, const double* src, double* f, double dt,
-                      double theta, const double* dz_c, const double* dz_f, double* tab, bool refactor,
-                      hipStream_t s) {
+                      double theta, const double* dz_c, const double* dz_f, double* tab,
+                      bool refactor, hipStream_t s) {
     if (refactor)
         hipLaunchKernelGGL(zfactor_kernel, dim3(1), dim3(64), 0, s, g, comp, dt, theta, dz_c,
                            dz_f, tab);

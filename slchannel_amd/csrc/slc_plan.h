@@ -104,6 +104,10 @@ constexpr int kDiagMaxBlocks = 2048;
 // rocFFT plans (members of an ensemble share per-size-class ones).
 int plan_create(const slc_grid_desc* d, int device, bool spectral, slc_plan** out);
 
+// Whether implicit_project can solve this plan's columns (SLC_OK), asked before
+// anything is launched.
+int check_zsolves(const slc_plan* p);
+
 // slc_implicit_project of the fields src into f: the same arrays, or with
 // theta < 1 others (src's ghosts are filled then).
 int implicit_project(slc_plan* p, double* const src[3], double* const f[3], double dt_z,
