@@ -311,16 +311,12 @@ int slc::plan_create(const slc_grid_desc* d, int device, bool spectral, slc_plan
         }
         for (int c = 0; c < 3; ++c) {
             const int nzi = c == 2 ? nz - 1 : nz;
-            void *a = nullptr, *b = nullptr, *q = nullptr;
-            if ((rc = dev_alloc(p, sizeof(double) * nx, &a)) ||
-                (rc = dev_alloc(p, sizeof(double) * ny, &b)) ||
-                (rc = dev_alloc(p, sizeof(int) * (nzi > 0 ? nzi : 1), &q))) {
+            if ((rc = dev_alloc(p, sizeof(int) * (nzi > 0 ? nzi : 1), &ptr))) {
                 slc_plan_destroy(p);
                 return rc;
             }
-            p->at[c] = ArrivalTabs{(const double*)a, (const double*)b, (const int*)q};
-            hipError_t e = run_arrival_tabs(g, c, (double*)a, (double*)b, (int*)q,
-                                            p->init_stream);
+            p->at[c] = ArrivalTabs{(const int*)ptr};
+            hipError_t e = run_arrival_tabs(g, c, (int*)ptr, p->init_stream);
             if (e == hipSuccess) e = hipStreamSynchronize(p->init_stream);
             if (e != hipSuccess) {
                 slc_plan_destroy(p);

@@ -532,7 +532,7 @@ int64_t member_bytes(int nx, int ny, int nz, int order, int storage) {
     b += spectral_bytes(nx, ny, nz);
     // tables: z (2 P + 4 columns of nz+2), arrival, Poisson, z-solve factors,
     // bulk and diagnostics partials
-    b += 8L * (nz + 2) * (2 * order + 8 + 19) + 8L * (nx + ny) * 4 + 4L * 3 * nz +
+    b += 8L * (nz + 2) * (2 * order + 8 + 19) + 8L * (nx + ny) + 4L * 3 * nz +
          8L * bulk_scratch(bulk_blocks(nx, ny, nz)) + 8L * 5 * kDiagMaxBlocks + 4096;
     return b;
 }

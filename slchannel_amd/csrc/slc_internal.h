@@ -43,11 +43,9 @@ hipError_t run_bdf2(const Grid& g, int comp, int pass, const TrajVel& V, const d
                     const double* Fm, double dt, double* out, unsigned long long* ncl,
                     hipStream_t s);
 
-// Per-component arrival tables: x/dx (nx), y/dy (ny), and per arrival z
-// (nzi) 2 * its face cell + (z >= the cell's centre split).
+// Per-component arrival table: per arrival z (nzi) 2 * its face cell + (z >=
+// the cell's centre split).
 struct ArrivalTabs {
-    const double* xdx;
-    const double* ydy;
     const int* csel;
 };
 
@@ -81,8 +79,7 @@ long step_tiles(const Grid& g, int comp);
 // Tiles of a component up to which the three components share a launch: where
 // two launches and tails (15-20 us) outweigh the merged kernel's 2-3%.
 constexpr long kMergeTiles = 8192;
-hipError_t run_arrival_tabs(const Grid& g, int comp, double* xdx, double* ydy, int* cell,
-                            hipStream_t s);
+hipError_t run_arrival_tabs(const Grid& g, int comp, int* cell, hipStream_t s);
 hipError_t run_ustar(const Grid& g, double* const o[3], const double* const a[3],
                      const double* const b[3], float* const fa[3], float* const fb[3],
                      hipStream_t s);

@@ -131,40 +131,26 @@ static int device_cus() {
     return n;
 }
 
-// Arrival tables of component C: x/dx, y/dy of the arrival columns and the
-// face cell and centre split of each arrival z (2 c + split), evaluated with
-// the very functions the trajectory sampling uses (so looked-up values are
-// the computed ones).
+// Arrival table of component C: the face cell and centre split of each arrival
+// z (2 c + split), evaluated with the very functions the trajectory sampling
+// uses (so looked-up values are the computed ones).
 template <int C>
-__global__ void arrival_tabs_kernel(Grid g, double* xdx, double* ydy, int* cell) {
+__global__ void arrival_tabs_kernel(Grid g, int* cell) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    const int nzi = Comp<C>::NZI(g);
+    if (t >= Comp<C>::NZI(g)) return;
     double xa, ya, za;
     int I, J, K;
-    if (t < g.nx) {
-        arrival<C>(g, (long)t * g.ny * nzi, xa, ya, za, I, J, K);
-        xdx[t] = xa / g.dx;
-    }
-    if (t < g.ny) {
-        arrival<C>(g, (long)t * nzi, xa, ya, za, I, J, K);
-        ydy[t] = ya / g.dy;
-    }
-    if (t < nzi) {
-        arrival<C>(g, (long)t, xa, ya, za, I, J, K);
-        const double zc = clampd(za, g.z_lo, g.z_hi);
-        const int c = face_cell(g, zc);
-        cell[t] = 2 * c + (zc >= g.z_c[c + 1] ? 1 : 0);
-    }
+    arrival<C>(g, (long)t, xa, ya, za, I, J, K);
+    const double zc = clampd(za, g.z_lo, g.z_hi);
+    const int c = face_cell(g, zc);
+    cell[t] = 2 * c + (zc >= g.z_c[c + 1] ? 1 : 0);
 }
 
-hipError_t run_arrival_tabs(const Grid& g, int comp, double* xdx, double* ydy, int* cell,
-                            hipStream_t s) {
-    int n = g.nx > g.ny ? g.nx : g.ny;
-    n = n > g.nz ? n : g.nz;
-    dim3 grid((n + 255) / 256);
-    if (comp == 0) hipLaunchKernelGGL(arrival_tabs_kernel<0>, grid, dim3(256), 0, s, g, xdx, ydy, cell);
-    else if (comp == 1) hipLaunchKernelGGL(arrival_tabs_kernel<1>, grid, dim3(256), 0, s, g, xdx, ydy, cell);
-    else hipLaunchKernelGGL(arrival_tabs_kernel<2>, grid, dim3(256), 0, s, g, xdx, ydy, cell);
+hipError_t run_arrival_tabs(const Grid& g, int comp, int* cell, hipStream_t s) {
+    dim3 grid((g.nz + 255) / 256);
+    if (comp == 0) hipLaunchKernelGGL(arrival_tabs_kernel<0>, grid, dim3(256), 0, s, g, cell);
+    else if (comp == 1) hipLaunchKernelGGL(arrival_tabs_kernel<1>, grid, dim3(256), 0, s, g, cell);
+    else hipLaunchKernelGGL(arrival_tabs_kernel<2>, grid, dim3(256), 0, s, g, cell);
     return hipGetLastError();
 }
 
