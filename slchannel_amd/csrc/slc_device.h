@@ -443,62 +443,6 @@ __device__ inline double trilinear(const Grid& g, const TV& V, double xdx, doubl
     return out;
 }
 
-// trilinear with the z node interval m0 given (the reference's locate
-// result; k0 = m0 at order 2 -- no clamp is needed: m0 <= NZ - 2 for a
-// clamped z).
-// x/y part of the trilinear sample of component C: order-2 uniform weights
-// ((t - 1) * (-1), t * 1) and the wrapped column indices.
-template <int C>
-__device__ inline void trilinear_xy(const Grid& g, double xdx, double ydy, double* wx,
-                                    double* wy, int* ix, int* iy) {
-    double sx = xdx + Comp<C>::shift_x;
-    double ix0 = floor(sx);
-    double tx = sx - ix0;
-    double sy = ydy + Comp<C>::shift_y;
-    double iy0 = floor(sy);
-    double ty = sy - iy0;
-    const int fx = floor_int(ix0), fy = floor_int(iy0);
-    ix[0] = wrap_idx(fx, g.nx);
-    ix[1] = wrap_idx(fx + 1, g.nx);
-    iy[0] = wrap_idx(fy, g.ny);
-    iy[1] = wrap_idx(fy + 1, g.ny);
-    wx[0] = (tx - 1.0) * (-1.0);
-    wx[1] = tx * 1.0;
-    wy[0] = (ty - 1.0) * (-1.0);
-    wy[1] = ty * 1.0;
-}
-
-template <int C, typename TV = TrajVel>
-__device__ inline double trilinear_m(const Grid& g, const TV& V, double xdx, double ydy,
-                                     double zc, int m0) {
-    double wx[2], wy[2], wz[2];
-    int ix[2], iy[2];
-    trilinear_xy<C>(g, xdx, ydy, wx, wy, ix, iy);
-    const int k0 = m0;
-    const double* zn = znodes<C>(g);
-    const double* dinv = Comp<C>::centers ? g.dinv_c2 : g.dinv_f2;
-    double d0 = zc - zn[k0], d1 = zc - zn[k0 + 1];
-    wz[0] = d1 * dinv[k0 * 2 + 0];
-    wz[1] = d0 * dinv[k0 * 2 + 1];
-    double out = 0.0;
-    bool first = true;
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const int base = node_addr<C, TV::packed>(g, ix[i], iy[j], k0);
-            double wij = wx[i] * wy[j];
-#pragma unroll
-            for (int k = 0; k < 2; ++k) {
-                double term = (wij * wz[k]) * V.at(C, base + k);
-                out = first ? term : out + term;
-                first = false;
-            }
-        }
-    }
-    return out;
-}
-
 // Tricubic trajectory sample of component C (traj_interp_order = 4): the
 // order-4 stencil of semilag.py:471-500 (no clamp counting; zc already
 // clamped) and the sequential (i, j, k) sum of _gather_interp
