@@ -57,6 +57,9 @@ inline bool big_index(const Grid& g) {
     return pl * (g.nx + 2) >= 536870912.0 || pl >= 16777216.0 || g.nx + 2 >= (1 << 24);
 }
 
+// Compute units of the current device (cached per device).
+int device_cus();
+
 // LDS-tiled step kernels (slc_step.hip) of one component; mode: 0 advect,
 // 1 bdf1, 2 far, 3 near, 4 gather (feet given), 5 far + near in one pass (no
 // feet arrays)

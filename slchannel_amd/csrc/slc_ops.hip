@@ -191,15 +191,15 @@ __global__ __launch_bounds__(256, zwaves(CHU, EXPL)) void zsolve3_kernel(Grid g,
 
 // Arguments of `comps` components in one launch: a block per 4 columns, and
 // where those are more than the chip holds at once, as many as it holds.
-constexpr int kCUs = 256;
 static ZSolve3 zsolve3(const Grid& g, double beta, const double* dz_c, const double* dz_f,
                        int comps) {
     ZSolve3 a{};
     a.dz_c = dz_c;
     a.dz_f = dz_f;
     a.beta = beta;
-    const long ncols = (long)g.nx * g.ny, most =
-        kCUs * zwaves(zsolve_scan_ch(0, g.nz), beta != 0.0) / comps;
+    const long ncols = (long)g.nx * g.ny;
+    const long most = std::max<long>(
+        1, (long)device_cus() * zwaves(zsolve_scan_ch(0, g.nz), beta != 0.0) / comps);
     for (int c = 0; c < 3; ++c)
         a.nb[c] = (unsigned)std::min<long>((ncols + kZScanCols - 1) / kZScanCols, most);
     return a;

@@ -117,8 +117,7 @@ __global__ __launch_bounds__(kSB) __attribute__((amdgpu_waves_per_eu(kWideWaves)
     }
 }
 
-// Compute units of the current device (cached per device).
-static int device_cus() {
+int device_cus() {
     static std::atomic<int> cache[64];
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
