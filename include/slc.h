@@ -213,8 +213,8 @@ int slc_ab2_update(slc_plan* plan, double* u, double* v, double* w, const double
                    const double* rv_prev, const double* rw_prev, double dt, void* stream);
 
 /* slc_imex_rhs and slc_ab2_update in one pass over the fields: on the
- * interior, r = rhs(u, v, w) and un, vn, wn = the updated fields, in arrays
- * of their own; no other entry of either is written (the new fields leave
+ * interior, r = rhs(u, v, w) and un, vn, wn = the updated fields, all six in
+ * arrays of their own; no other entry of either is written (the new fields leave
  * without ghosts).  Replaces solver.py:1062-1081. */
 int slc_imex_advance(slc_plan* plan, const double* u, const double* v, const double* w,
                      double* un, double* vn, double* wn, double* ru, double* rv, double* rw,

@@ -254,8 +254,13 @@ extern "C" int slc_imex_advance(slc_plan* p, const double* u, const double* v, c
     if (!p) return fail(SLC_EINVAL, "null plan");
     if (!u || !v || !w || !un || !vn || !wn || !ru || !rv || !rw)
         return fail(SLC_EINVAL, "null array");
-    if (u == un || v == vn || w == wn)
-        return fail(SLC_EINVAL, "the new fields need arrays of their own");
+    // neighbours read the old fields while others are written
+    const double* const in[3] = {u, v, w};
+    const double* const out[6] = {un, vn, wn, ru, rv, rw};
+    for (int i = 0; i < 6; ++i) {
+        if (std::find(in, in + 3, out[i]) != in + 3 || std::find(out, out + i, out[i]) != out + i)
+            return fail(SLC_EINVAL, "the new fields and the rhs need arrays of their own");
+    }
     const bool prev = ru_prev || rv_prev || rw_prev;
     if (prev && !(ru_prev && rv_prev && rw_prev))
         return fail(SLC_EINVAL, "previous rhs: all three components or none");
