@@ -22,9 +22,16 @@
 //
 // One read of the fields in place of two (a pass of means, then one of
 // fluctuations about them; 86 + 82 us at 256^3, each at the rate of memory).
-// The shift keeps the precision: the shifted values are of the size of the
-// fluctuations, and what the last subtraction loses is the square of the
-// provisional mean's error, a fraction of the variance.
+// What the shift costs in precision: with m the provisional mean's error and s2
+// the variance, the last subtraction takes m^2 from s2 + m^2, so rounding of
+// the sums weighs up to 1 + 2 m^2 / s2 times as much as in sums about the mean
+// itself.  For fields whose columns are samples of one distribution m^2 is
+// s2 / 64 and less.  The columns are a regular 8 x 8 lattice: a pattern whose
+// wavenumbers are multiples of 8 in x and y may be met at one phase only
+// (m^2 = 4 s2 for a product of two cosines), and values that stand out on those
+// very columns have m^2 up to N / 64 s2, N the plane's columns, the most that
+// any field can have.  A variance below zero, which the final kernel sets to
+// zero, is at most such rounding.
 //
 // Layout of the pass: a workgroup is 64 z lanes x 4 column groups.  The z
 // lanes make every load a coalesced 512-byte row segment; each thread walks
