@@ -116,11 +116,15 @@ __device__ inline int wrap_idx(int i, int n) {
 // x / d, correctly rounded, for a d whose reciprocal is held as a pair:
 // h = RN(1/d) and h + l = 1/d to twice the precision (recip_pair).  The first
 // two operations give x (h + l) to just over half an ulp; with its exact
-// residual the last fused operation rounds to RN(x / d) (the correction step
-// of a division whose reciprocal is correctly rounded).  Four FP64
-// instructions where the general division's scaling, quarter-rate
-// reciprocal, refinement and fix-up take eleven; a tile lane divides eight
-// times.
+// residual the last fused operation rounds to RN(x / d) (Markstein's correction
+// step of a division whose reciprocal is correctly rounded, "Computation of
+// elementary functions on the IBM RISC System/6000 processor", 1990).  It has
+// no scaling: below about 2^-960 the residual is not exact and the last place
+// may differ, and an infinite x, or a quotient past the range, gives NaN (the
+// fractions and level differences formed from such a quotient are NaN either
+// way).  Four FP64 instructions where the general division's scaling,
+// quarter-rate reciprocal, refinement and fix-up take eleven; a tile lane
+// divides eight times.
 __device__ inline double quotient(double x, double d, double h, double l) {
     const double q = fma(x, h, x * l);
     return fma(fma(-d, q, x), h, q);

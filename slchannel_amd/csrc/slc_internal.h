@@ -79,8 +79,12 @@ hipError_t run_tile_step3(const Grid& g, int mode, const ArrivalTabs A[3], const
                           double* const out[3], unsigned long long* ncl, hipStream_t s);
 // Tiles of the step kernels for component comp (the defer flags' count).
 long step_tiles(const Grid& g, int comp);
-// Tiles of a component up to which the three components share a launch: where
-// two launches and tails (15-20 us) outweigh the merged kernel's 2-3%.
+// Tiles of a component up to which the three components share a launch, which
+// saves two launches and drained tails (10-25 us).  BDF2 predictor, one launch
+// against three, order 6: 1024 tiles 106 and 121 us, 8192 562 and 587, 12288
+// 833 and 858, 27648 1.89 and 1.91 ms, 65536 the same 4.46 ms; order 4: 62 and
+// 71 us, 386 and 400, 580 and 598, 1.40 and 1.41 ms, 3.32 ms.  Past the line the
+// saving is 3% and falling.
 constexpr long kMergeTiles = 8192;
 hipError_t run_arrival_tabs(const Grid& g, int comp, int* cell, hipStream_t s);
 hipError_t run_ustar(const Grid& g, double* const o[3], const double* const a[3],

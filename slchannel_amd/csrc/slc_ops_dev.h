@@ -1102,8 +1102,11 @@ __device__ inline double bulk_mean(const double* partials, int np, double total_
 // values.  The last block to finish forms the mean after the shift, fills
 // scal -- [0] correction, [1] forcing, [2] mean after the shift, [3] before
 // it -- and returns true (on every thread).  The sums cross blocks as
-// agent-scope accesses, each ahead of its block's ticket: a release fence
-// would write back the shifted values of the whole L2 with every block.
+// agent-scope accesses, each ahead of its block's ticket.  The order rests on
+// gfx950, not on the language's memory model: there an agent-scope store has
+// reached the device's point of coherence once vmcnt has counted it, so the
+// wait before the ticket publishes the sum.  A release at agent scope would
+// also write back the shifted values of the whole L2 with every block.
 // Two launches in place of five (sums, mean, shift and sums, mean, ghosts):
 // 24 -> 14 us at 64^3, 120 -> 117 us at 256^3 (bound by memory there).
 __device__ inline bool bulk_shift_body(const Grid& g, double* __restrict__ u,

@@ -7,9 +7,9 @@ namespace slc {
 // The three components' tiles of a step kernel in one launch: a small grid's
 // tiles fill the GPU together (32x24x32 has 96 tiles per component for 256
 // CUs), and two drained tails and launches go.  For grids up to kMergeTiles
-// tiles; on a larger one the single-component kernels, whose scalars fit their
-// registers better, are the faster (256^3, order 6: 4.28 ms for the three
-// against 4.39 ms).  Such a grid never needs 64-bit addressing.
+// tiles; on a larger one the launches saved are a few percent of the passes, at
+// 256^3 nothing (kMergeTiles).  A grid of so few tiles never needs 64-bit
+// addressing.
 struct Tile3 {
     Grid g;
     TrajVel V;
