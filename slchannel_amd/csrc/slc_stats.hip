@@ -26,7 +26,7 @@
 // the variance, the last subtraction takes m^2 from s2 + m^2, so rounding of
 // the sums weighs up to 1 + 2 m^2 / s2 times as much as in sums about the mean
 // itself.  For fields whose columns are samples of one distribution m^2 is
-// s2 / 64 and less.  The columns are a regular 8 x 8 lattice: a pattern whose
+// about s2 / 64.  The columns are a regular 8 x 8 lattice: a pattern whose
 // wavenumbers are multiples of 8 in x and y may be met at one phase only
 // (m^2 = 4 s2 for a product of two cosines), and values that stand out on those
 // very columns have m^2 up to N / 64 s2, N the plane's columns, the most that

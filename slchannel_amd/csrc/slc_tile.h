@@ -29,9 +29,9 @@
 // same order as the direct gather).
 //
 // What bounds it (fused BDF2 pass of u, 256^3, order 6; counters per
-// wavefront): 2200 VALU instructions (64% of the launch; half of them FP64),
-// 216 stencil values per foot from LDS (68%), the trajectory corners and z
-// tables through the vector cache (70%): no unit is full, four waves per SIMD
+// wavefront): 2272 VALU instructions (74% of the launch; half of them FP64),
+// 216 stencil values per foot from LDS (62%), the trajectory corners and z
+// tables through the vector cache (78%): no unit is full, four waves per SIMD
 // (128 VGPRs) do not hide the rest.  Measured with the index arithmetic in 32
 // bits and scalar registers, the row stride on the LDS banks and the boxes in
 // direct-to-LDS pieces: 1.61 -> 1.40 ms (w, whose odd rows went through
